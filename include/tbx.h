@@ -444,15 +444,17 @@ int tbx_balance21(int64_t *num_leaves, int64_t capacity, uint32_t *anchor,
                   uint8_t *depth, int bc);
 
 /* ---- tuning knobs (process-wide) ---------------------------------------
- * TBX_OPT_STEP_SHAPE: launch shape of the fused step kernel, used by later
- * step calls.  0: 256 threads; 1-3: 256 / 1024 / 512 threads with a
+ * TBX_OPT_STEP_SHAPE: launch shape of the fused step kernel in TBX_EXACT,
+ * used by later step calls; the other modes order a workgroup's points by
+ * leaf in one kernel (256 threads in TBX_FP64, 512 in the FP32 modes)
+ * whatever it says.  0: 256 threads; 1-3: 256 / 1024 / 512 threads with a
  * register budget of 4 waves per SIMD; 4-7: the workgroup's points
  * regrouped by leaf before each evaluation, 256 / 512 threads (budget 2
  * waves per SIMD) and 1024 / 512 threads (budget 4); 8-10: regrouped,
  * 1024 threads with a budget of 8 waves per SIMD (64 registers), 512 and
- * 768 threads with a budget of 6.  -1 (the default) picks per arithmetic
- * mode and degree the shape measured fastest (q = 14: 8 for TBX_FP32, 10
- * for TBX_FP32_HEAD64; 6 otherwise); shapes other than 0 and 6 exist for
+ * 768 threads with a budget of 6.  -1 (the default) is 6
+ * (tbx_step_shape names 8 and 10 for the FP32 modes at q = 14, which they
+ * ignore); shapes other than 0 and 6 exist for
  * q = 8 and 14 only (others run 6).
  * Every shape gives the same results.
  * TBX_OPT_TRACER_MFMA (default 1): a concentration with a multiple of 16
@@ -490,7 +492,7 @@ int tbx_get_option(int option, int *value);
 
 /* The step launch shape (TBX_OPT_STEP_SHAPE) that a step with these mode
  * flags at degree q runs with under the current option.  No counterpart in
- * the reference: it reports the launch configuration for profiling. */
+ * the reference: it reports the option's resolution; TBX_EXACT runs it. */
 int tbx_step_shape(uint32_t flags, int q, int *shape);
 
 const char *tbx_last_error(void);

@@ -61,9 +61,13 @@ __device__ __forceinline__ double wrap1(double c) {
 // non-periodic bc (tree_functor.h:464-479), extended to a clamp outside the
 // domain; negative and NaN coordinates take cell 0.
 __device__ __forceinline__ uint32_t cell21(double c) {
-  if (!(c >= 0.0)) return 0u;
-  const double f = floor(c * kKeyScale);
-  return f > kKeyScale - 1.0 ? (uint32_t)(kKeyScale - 1.0) : (uint32_t)f;
+  // clamped first (a NaN to 0), so the conversion's truncation is the floor
+  return (uint32_t)__builtin_fmin(__builtin_fmax(c * kKeyScale, 0.0), kKeyScale - 1.0);
+}
+
+// 2^-depth, by its exponent bits (depth <= 21).
+__device__ __forceinline__ double leaf_edge(uint32_t depth) {
+  return __hiloint2double((int)((1023u - depth) << 20), 0);
 }
 
 // Spread the low 21 bits of v to every third bit.
@@ -114,8 +118,22 @@ __device__ __forceinline__ int locate_key(const TreeView &t, uint64_t k) {
   return dir_search(t, k, dir_first(t, k), dir_last(t, k));
 }
 
+// Spread the low 6 bits of v to every third bit.
+__device__ __forceinline__ uint32_t spread3_6(uint32_t v) {
+  uint32_t x = (v | (v << 8)) & 0x0300fu;
+  x = (x | (x << 4)) & 0x030c3u;
+  return (x | (x << 2)) & 0x09249u;
+}
+
+// With an exact directory (level g <= 6) only the top g bits per axis
+// matter: the cell's index is formed in 32 bits instead of the 63-bit key.
 __device__ __forceinline__ int locate(const TreeView &t, double x, double y,
                                       double z) {
+  if (t.dir_exact) {
+    const uint32_t sh = (uint32_t)t.dir_shift / 3u;
+    return t.dir[spread3_6(cell21(x) >> sh) | (spread3_6(cell21(y) >> sh) << 1) |
+                 (spread3_6(cell21(z) >> sh) << 2)];
+  }
   return locate_key(t, point_key(x, y, z));
 }
 
@@ -126,7 +144,7 @@ __device__ __forceinline__ void leaf_xi(const TreeView &t, int leaf, double x,
                                         double &ey, double &ez) {
   const uint4 inf = t.info[leaf];
   const double s = (double)(1u << inf.w);
-  const double len = 1.0 / s;
+  const double len = leaf_edge(inf.w);
   const double cx = (double)inf.x * len;
   const double cy = (double)inf.y * len;
   const double cz = (double)inf.z * len;
@@ -348,6 +366,12 @@ __host__ __device__ constexpr int tri_index(int D, int i, int j, int k) {
   for (int a = 0; a < i; ++a) idx += (D - a) * (D - a + 1) / 2;
   for (int b = 0; b < j; ++b) idx += D - i - b;
   return idx + k;
+}
+
+// The same for (i, j, 0), in closed form.
+__host__ __device__ constexpr int tri_start(int D, int i, int j) {
+  const int n = D - i;
+  return (D * (D + 1) * (D + 2) - n * (n + 1) * (n + 2)) / 6 + j * n - j * (j - 1) / 2;
 }
 
 template <typename T>

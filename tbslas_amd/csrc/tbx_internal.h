@@ -67,23 +67,18 @@ struct SubArgs {
   int bc;
 };
 
-// Launch shapes of the fused step kernel (workgroup sizes below).  0-3 run
-// the points in arrival order; 4-7 regroup each workgroup's points by leaf
-// before every evaluation.  Shapes 0 and 6 (the default) are built for
-// every degree, the others for the benchmark degrees 8 and 14 only; an
-// unbuilt shape falls back to 6.
+// Launch shapes of the fused step kernel in TBX_EXACT (workgroup sizes
+// below; the other modes run k_step_rows at rows_step_block threads whatever
+// the option says).  0-3 run the points in arrival order; 4-7 regroup each
+// workgroup's points by leaf before every evaluation.  Shapes 0 and 6 (the
+// default) are built for every degree, the others for degrees 8 and 14
+// only; an unbuilt shape falls back to 6.
 constexpr int kStepShapes = 11;
 constexpr int kStepShapeBlock[kStepShapes] = {256, 256, 1024, 512, 256, 512, 1024, 512, 1024, 512, 768};
 constexpr int kDefaultStepShape = 6;
-// The step shape option's default, -1: the shape measured fastest for the
-// step's arithmetic mode and degree.  At q = 14 (adaptive tree of 36,324
-// leaves, 122,593,500 points, MI355X) the FP32 step kernel runs in 33.6 ms
-// with shape 8 (1024 threads, 64 VGPRs: two workgroups per CU) against
-// 42.6 ms with shape 6, and FP32 + FP64 head in 38.6 ms with shape 10 (768
-// threads, 80 VGPRs, two per CU) against 41.0 ms with shape 9 (512
-// threads, whose smaller regrouping leaves 1.49 leaf passes per wavefront)
-// and 44.9 ms with shape 6; FP64 keeps shape 6 (73.3 ms against 92-102 ms,
-// where the smaller budgets spill).
+// The step shape option's default, -1.  TBX_EXACT takes shape 6; the shapes
+// that tbx_step_shape names for the FP32 modes at degree 14 are those of the
+// scalar-operand kernel, which they no longer run.
 constexpr int kAutoStepShape = -1;
 inline int auto_step_shape(int mode, int q) {
   if (q == 14 && mode == kFp32) return 8;
@@ -128,6 +123,12 @@ struct StepArgs {
 };
 
 constexpr int kBlock = 256;
+// Workgroup of the step kernel in the modes but TBX_EXACT (tbx_rows.h): a
+// larger group pads fewer runs of a leaf to 16 places, a smaller one waits
+// less at its barriers.  At degree 14, FP64 (three waves per SIMD) takes
+// 3.5 ms with 256 threads and 4.2 with 512 (16.7 M points), FP32 + FP64
+// head 19.1 and 18.4 ms (123 M points).
+constexpr int rows_step_block(int mode) { return mode == kFma64 ? 256 : 512; }
 constexpr int kAdjBlock = 256;  // workgroup of the adjoint concentration kernel
 
 // Launchers instantiated once per degree Q (tbx_kernels.hip, -DTBX_Q=Q).

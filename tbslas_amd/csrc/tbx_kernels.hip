@@ -7,6 +7,7 @@
 
 #include "tbx_device.h"
 #include "tbx_mfma.h"
+#include "tbx_rows.h"
 
 #ifndef TBX_Q
 #error "compile with -DTBX_Q=<degree>"
@@ -17,14 +18,18 @@ namespace {
 
 constexpr int D = TBX_Q + 1;
 
-// EvalTree at caller points (tree_functor.h:397-791): wrap, locate,
-// contract.  out[i][l] point-major.
-template <int MODE>
-__global__ __launch_bounds__(kBlock) void k_eval(TreeView t,
-                                                 double *__restrict__ pts,
-                                                 int64_t n, int bc,
-                                                 int write_back,
-                                                 double *__restrict__ out) {
+// Waves per SIMD asked of the row kernels: the basis in registers, 2 D
+// values, leaves FP64 four up to degree 9 and three above, FP32 five and
+// four, without spills.
+constexpr int rows_waves(int mode) {
+  return mode == kFma64 ? (TBX_Q <= 9 ? 4 : 3) : (TBX_Q <= 9 ? 5 : 4);
+}
+
+// EvalTree at caller points (tree_functor.h:397-791) in the reference's
+// arithmetic: wrap, locate, contract.  out[i][l] point-major.
+__global__ __launch_bounds__(kBlock) void k_eval_exact(TreeView t, double *__restrict__ pts,
+                                                       int64_t n, int bc, int write_back,
+                                                       double *__restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
@@ -40,19 +45,17 @@ __global__ __launch_bounds__(kBlock) void k_eval(TreeView t,
   }
   const int dof = t.dof;
   double *o = out + i * dof;
-  eval_dof<D, MODE>(t, x, y, z, [&](int l, double v) { o[l] = v; });
+  eval_dof<D, kExact64>(t, x, y, z, [&](int l, double v) { o[l] = v; });
 }
 
 // A velocity functor (FieldExtrapFunctor / FieldSetFunctor / a scaled tree)
-// at caller points at time t; the extrapolating kind evaluates its
-// extrapolation (the second-stage functor).
-template <int MODE, int KIND>
-__global__ __launch_bounds__(kBlock) void k_veval(VelSource vel,
-                                                  double *__restrict__ pts,
-                                                  int64_t n, int bc,
-                                                  int write_back, double t,
-                                                  int scaled, double g,
-                                                  double *__restrict__ out) {
+// at caller points at time t, as k_eval_exact; the extrapolating kind
+// evaluates its extrapolation (the second-stage functor).
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_veval_exact(VelSource vel, double *__restrict__ pts,
+                                                        int64_t n, int bc, int write_back,
+                                                        double t, int scaled, double g,
+                                                        double *__restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
@@ -62,7 +65,7 @@ __global__ __launch_bounds__(kBlock) void k_veval(VelSource vel,
     z = wrap1(z);
   }
   double v0, v1, v2;
-  eval_velocity<D, MODE, KIND>(vel, 2, t, scaled, g, bc, x, y, z, v0, v1, v2);
+  eval_velocity<D, kExact64, KIND>(vel, 2, t, scaled, g, bc, x, y, z, v0, v1, v2);
   if (bc == TBX_BC_PERIODIC && write_back) {  // wrapped once per tree
     pts[3 * i + 0] = x;
     pts[3 * i + 1] = y;
@@ -73,16 +76,91 @@ __global__ __launch_bounds__(kBlock) void k_veval(VelSource vel,
   out[3 * i + 2] = v2;
 }
 
-// One IntegrateRK2 substep for caller points, in place.
-template <int MODE, int KIND>
-__global__ __launch_bounds__(kBlock) void k_traj(VelSource vel,
-                                                 double *__restrict__ xs,
-                                                 int64_t n, SubArgs a) {
+// One IntegrateRK2 substep for caller points, in place, as k_eval_exact.
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_traj_exact(VelSource vel, double *__restrict__ xs,
+                                                       int64_t n, SubArgs a) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   double x = xs[3 * i + 0], y = xs[3 * i + 1], z = xs[3 * i + 2];
-  rk2_substep<D, MODE, KIND>(vel, a.bc, a.htau, a.tau, a.scaled, a.g1, a.g2, a.ts1,
-                       a.ts2, x, y, z);
+  rk2_substep<D, kExact64, KIND>(vel, a.bc, a.htau, a.tau, a.scaled, a.g1, a.g2, a.ts1, a.ts2, x,
+                                 y, z);
+  xs[3 * i + 0] = x;
+  xs[3 * i + 1] = y;
+  xs[3 * i + 2] = z;
+}
+
+// The same three in the other modes: a workgroup's points ordered by leaf
+// and contracted row by row (tbx_rows.h).  Threads past the last point hold
+// a copy of it and take no part.  BLOCK: 256 threads, or 64 where that
+// leaves compute units without a workgroup (rows_block).
+template <int MODE, int BLOCK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_eval(
+    TreeView t, double *__restrict__ pts, int64_t n, int bc, int write_back,
+    double *__restrict__ out) {
+  __shared__ RowsLds<BLOCK> sh;
+  const int64_t i0 = (int64_t)blockIdx.x * BLOCK;
+  const bool live = i0 + (int)threadIdx.x < n;
+  const int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
+  double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
+  if (bc == TBX_BC_PERIODIC) {
+    x = wrap1(x);
+    y = wrap1(y);
+    z = wrap1(z);
+    if (write_back && live) {
+      pts[3 * i + 0] = x;
+      pts[3 * i + 1] = y;
+      pts[3 * i + 2] = z;
+    }
+  }
+  const int lf = locate(t, x, y, z);
+  const int count = order_by_leaf(sh, live, lf);
+  double *o = out + i * t.dof;
+  rows_dof<D, MODE>(sh, t, count, lf, x, y, z, [&](int l, double v) {
+    if (live) o[l] = v;
+  });
+}
+
+template <int MODE, int KIND, int BLOCK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_veval(
+    VelSource vel, double *__restrict__ pts, int64_t n, int bc, int write_back, double t,
+    int scaled, double g, double *__restrict__ out) {
+  __shared__ RowsLds<BLOCK> sh;
+  const int64_t i0 = (int64_t)blockIdx.x * BLOCK;
+  const bool live = i0 + (int)threadIdx.x < n;
+  const int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
+  double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
+  if (bc == TBX_BC_PERIODIC) {
+    x = wrap1(x);
+    y = wrap1(y);
+    z = wrap1(z);
+  }
+  const int lf = locate(vel.t[0], x, y, z);
+  const int count = order_by_leaf(sh, live, lf);
+  double v[3];
+  rows_velocity<D, MODE, KIND>(sh, vel, 2, t, scaled, g, bc, count, lf, x, y, z, v);
+  if (!live) return;
+  if (bc == TBX_BC_PERIODIC && write_back) {  // wrapped once per tree
+    pts[3 * i + 0] = x;
+    pts[3 * i + 1] = y;
+    pts[3 * i + 2] = z;
+  }
+  out[3 * i + 0] = v[0];
+  out[3 * i + 1] = v[1];
+  out[3 * i + 2] = v[2];
+}
+
+template <int MODE, int KIND, int BLOCK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_traj(
+    VelSource vel, double *__restrict__ xs, int64_t n, SubArgs a) {
+  __shared__ RowsLds<BLOCK> sh;
+  const int64_t i0 = (int64_t)blockIdx.x * BLOCK;
+  const bool live = i0 + (int)threadIdx.x < n;
+  const int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
+  double x = xs[3 * i + 0], y = xs[3 * i + 1], z = xs[3 * i + 2];
+  rows_substep<D, MODE, KIND>(sh, vel, a.bc, a.htau, a.tau, a.scaled, a.g1, a.g2, a.ts1, a.ts2,
+                              live, x, y, z);
+  if (!live) return;
   xs[3 * i + 0] = x;
   xs[3 * i + 1] = y;
   xs[3 * i + 2] = z;
@@ -184,14 +262,12 @@ __device__ __forceinline__ void arrival_node(const StepArgs &a, int64_t i0, int 
 }
 
 // The same step with the workgroup's points regrouped by leaf before each
-// of the 2 num_rk_step + 1 evaluations (regroup_pos in tbx_device.h; the
-// concentration's only in some modes, see below).  The
+// of the 2 num_rk_step + 1 evaluations (regroup_pos in tbx_device.h).  The
 // thread that holds a point after a regroup carries it on: the RK2 state
 // (start point, wrapped midpoint) travels with the point through LDS, and
 // the leaf found for the regroup is the one the evaluation uses.  Lanes
-// past the last arrival point carry a copy of it and store nothing.  MF:
-// the concentration's components go through eval_dof_mfma.
-template <int MODE, int KIND, int BLOCK, bool MF>
+// past the last arrival point carry a copy of it and store nothing.
+template <int MODE, int KIND, int BLOCK>
 __device__ __forceinline__ void k_step_rg_body(const VelSource &vel, const TreeView &conc,
                                                const StepArgs &a, double *__restrict__ vals,
                                                double *__restrict__ dep) {
@@ -288,14 +364,7 @@ __device__ __forceinline__ void k_step_rg_body(const VelSource &vel, const TreeV
     }
     lf = locate(conc, st[0], st[1], st[2]);
     double p3[3] = {st[0], st[1], st[2]};
-    // A departure point lies mostly in its midpoint's leaf, by which the
-    // points were just regrouped.  Regrouping again before a one-component
-    // contraction costs the FP32 + FP64 head and FP64 kernels more than the
-    // leaf passes it saves (headline kernel 25.3 against 26.1 ms at q = 14);
-    // the FP32 kernel at its 64-register budget, and many components on the
-    // matrix cores, keep it.
-    constexpr bool kConcRegroup = MF || !(MODE == kFp32h || MODE == kFma64);
-    if constexpr (kConcRegroup) regroup(sh, orig, lf, p3);
+    regroup(sh, orig, lf, p3);
     const int64_t gi = i0 + orig;
     const bool live = gi < a.npts;
     if (live && dep) {
@@ -305,19 +374,13 @@ __device__ __forceinline__ void k_step_rg_body(const VelSource &vel, const TreeV
     }
     const int64_t al = gi / a.P;
     const int am = (int)(gi - al * a.P);
-    if constexpr (MF) {
-      using T = typename ModeType<MODE>::T;
-      eval_dof_mfma<D, T>(conc, lf, p3[0], p3[1], p3[2], vals, al * conc.dof * a.P + am, a.P,
-                          live);
-    } else {
-      double *o = vals + al * conc.dof * a.P + am;
-      eval_dof<D, MODE>(
-          conc, p3[0], p3[1], p3[2],
-          [&](int l, double v) {
-            if (live) o[(int64_t)l * a.P] = v;
-          },
-          lf);
-    }
+    double *o = vals + al * conc.dof * a.P + am;
+    eval_dof<D, MODE>(
+        conc, p3[0], p3[1], p3[2],
+        [&](int l, double v) {
+          if (live) o[(int64_t)l * a.P] = v;
+        },
+        lf);
   }
 }
 
@@ -325,20 +388,141 @@ template <int MODE, int KIND, int BLOCK, int WPE>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step_rg(
     VelSource vel, TreeView conc, StepArgs a, double *__restrict__ vals,
     double *__restrict__ dep) {
-  k_step_rg_body<MODE, KIND, BLOCK, false>(vel, conc, a, vals, dep);
+  k_step_rg_body<MODE, KIND, BLOCK>(vel, conc, a, vals, dep);
+}
+
+// The step in every mode but TBX_EXACT (tbx_rows.h).  A thread keeps its
+// arrival point; before each velocity evaluation the workgroup's points are
+// ordered by leaf and its wavefronts take 64 places at a time from that
+// order.  The first substep's first stage takes the nodal values, and only
+// points without one are ordered and contracted.  MF: many components (a
+// multiple of 16) through eval_dof_mfma.
+template <int MODE, int KIND, int BLOCK, bool MF>
+__device__ __forceinline__ void k_step_rows_body(const VelSource &vel, const TreeView &conc,
+                                                 const StepArgs &a, double *__restrict__ vals,
+                                                 double *__restrict__ dep) {
+  constexpr int P = D * D * D;
+  __shared__ RowsLds<BLOCK> sh;
+  const uint32_t b = blockIdx.x;
+  const int64_t lb = (int64_t)(b & 7u) * a.per_xcd + (int64_t)(b >> 3);
+  if (lb >= a.nblocks) return;  // uniform over the workgroup
+  // leaf l0 + r / P, node r % P of the workgroup's arrival point t: the
+  // 64-bit division is the workgroup's, lanes divide 32-bit by a constant
+  const int64_t i0 = lb * BLOCK, l0 = i0 / P;
+  const uint32_t r0 = (uint32_t)(i0 - l0 * P);
+  const int np = a.npts - i0 < BLOCK ? (int)(a.npts - i0) : BLOCK;
+  const bool live = (int)threadIdx.x < np;
+  const uint32_t r = r0 + (live ? threadIdx.x : (uint32_t)np - 1u);
+  const int64_t leaf = l0 + r / (uint32_t)P;
+  const int m = (int)(r % (uint32_t)P);
+  double x, y, z;
+  {
+    const uint4 inf = conc.info[leaf];
+    const double len = leaf_edge(inf.w);
+    x = (double)inf.x * len + len * a.node[m % D];
+    y = (double)inf.y * len + len * a.node[(m / D) % D];
+    z = (double)inf.z * len + len * a.node[m / (D * D)];
+  }
+  int count = 0;
+#pragma unroll 1
+  for (int s = 0; s < a.nsub; ++s) {
+    // stage 1 at the (wrapped in place) start point (traj.inc:33)
+    if (a.bc == TBX_BC_PERIODIC) {
+      x = wrap1(x);
+      y = wrap1(y);
+      z = wrap1(z);
+    }
+    int lf = locate(vel.t[0], x, y, z);
+    double v[3] = {0.0, 0.0, 0.0};
+    bool need = live;
+    if constexpr (KIND == kVelTree || KIND == kVelExtrap) {
+      if (s == 0 && a.vnode)
+        need = live && !nodal_velocity<D>((const NodalT<MODE> *)a.vnode, vel.t[0],
+                                          conc.info[leaf], m, lf, P, a.scaled, a.g[0], v[0],
+                                          v[1], v[2]);
+    }
+    if (__syncthreads_or(need)) {
+      double u[3];
+      count = order_by_leaf(sh, need, lf);
+      rows_velocity<D, MODE, KIND>(sh, vel, 1, a.ts[2 * s], a.scaled, a.g[2 * s], a.bc, count,
+                                   lf, x, y, z, u);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[c] = need ? u[c] : v[c];
+    }
+    count = rows_midpoint<D, MODE, KIND>(sh, vel, a.bc, a.htau, a.tau, a.scaled, a.g[2 * s + 1],
+                                         a.ts[2 * s + 1], live, v, x, y, z);
+  }
+  // con_evaluator(departure points) wraps them in place (semilag.inc:43)
+  if (a.bc == TBX_BC_PERIODIC) {
+    x = wrap1(x);
+    y = wrap1(y);
+    z = wrap1(z);
+  }
+  if (live && dep) {
+    dep[3 * (i0 + threadIdx.x) + 0] = x;
+    dep[3 * (i0 + threadIdx.x) + 1] = y;
+    dep[3 * (i0 + threadIdx.x) + 2] = z;
+  }
+  const int lf = locate(conc, x, y, z);
+  if constexpr (MF) {
+    // a wavefront takes 64 places of the order by leaf at a time (a padding
+    // place stores its point's values a second time)
+    using T = typename ModeType<MODE>::T;
+    sh.e[0][threadIdx.x] = x;
+    sh.e[1][threadIdx.x] = y;
+    sh.e[2][threadIdx.x] = z;
+    sh.leaf[threadIdx.x] = lf;
+    count = order_by_leaf(sh, live, lf);
+    __syncthreads();
+#pragma unroll 1
+    for (int p0 = (int)(threadIdx.x & ~63u); p0 < count; p0 += BLOCK) {
+      const int pos = p0 + (int)(threadIdx.x & 63u);
+      const int src = sh.order[pos < count ? pos : count - 1];
+      const uint32_t q = r0 + (uint32_t)src;
+      eval_dof_mfma<D, T>(conc, sh.leaf[src], sh.e[0][src], sh.e[1][src], sh.e[2][src], vals,
+                          (l0 + q / (uint32_t)P) * conc.dof * P + (int64_t)(q % (uint32_t)P), P,
+                          pos < count);
+    }
+  } else {
+    // a departure point lies mostly in its midpoint's leaf: the midpoints'
+    // order serves the concentration too
+    double *o = vals + leaf * conc.dof * P + m;
+    rows_dof<D, MODE>(sh, conc, count, lf, x, y, z, [&](int l, double v) {
+      if (live) o[(int64_t)l * P] = v;
+    });
+  }
+}
+
+template <int MODE, int KIND, int BLOCK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_step_rows(
+    VelSource vel, TreeView conc, StepArgs a, double *__restrict__ vals,
+    double *__restrict__ dep) {
+  k_step_rows_body<MODE, KIND, BLOCK, false>(vel, conc, a, vals, dep);
 }
 
 // The same step with the concentration's components contracted on the
 // matrix cores (conc.dof a multiple of 16; FP64 or FP32 arithmetic).
 template <int MODE, int KIND, int BLOCK, int WPE>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step_rg_mfma(
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step_rows_mfma(
     VelSource vel, TreeView conc, StepArgs a, double *__restrict__ vals,
     double *__restrict__ dep) {
-  k_step_rg_body<MODE, KIND, BLOCK, true>(vel, conc, a, vals, dep);
+  k_step_rows_body<MODE, KIND, BLOCK, true>(vel, conc, a, vals, dep);
 }
 
 inline unsigned grid_for(int64_t n) {
   return (unsigned)((n + kBlock - 1) / kBlock);
+}
+
+// Calls f with the workgroup size of the point kernels for n points and the
+// grid: 64 threads while 256 would leave some of the 256 compute units
+// without a workgroup, 256 above (the larger group finds fewer runs of a
+// leaf to pad).
+template <typename F>
+void with_rows_block(int64_t n, F f) {
+  if (n <= 256 * 256)
+    f(std::integral_constant<int, 64>{}, (unsigned)((n + 63) / 64));
+  else
+    f(std::integral_constant<int, 256>{}, (unsigned)((n + 255) / 256));
 }
 
 // Calls f with the arithmetic mode as a compile-time constant.
@@ -440,13 +624,22 @@ hipError_t launch_step_mode(const VelSource &vel, const TreeView &conc, const St
     if constexpr (MODE == kFma64 || MODE == kFp32) {
       if (vel.kind != kVelTree || a.shape != kMfmaStepShape) return hipErrorInvalidValue;
       constexpr int B = mfma_step_block(MODE), W = mfma_step_waves(MODE);
-      hipLaunchKernelGGL((k_step_rg_mfma<MODE, kVelTree, B, W>), dim3((unsigned)(8 * a.per_xcd)),
+      hipLaunchKernelGGL((k_step_rows_mfma<MODE, kVelTree, B, W>), dim3((unsigned)(8 * a.per_xcd)),
                          dim3(B), 0, s, vel, conc, a, vals, dep);
       return hipGetLastError();
     } else {
       return hipErrorInvalidValue;
     }
   }
+  if constexpr (MODE != kExact64) {
+    constexpr int kB = rows_step_block(MODE);
+    return with_kind(vel.kind, [&](auto k) {
+      hipLaunchKernelGGL((k_step_rows<MODE, decltype(k)::value, kB>),
+                         dim3((unsigned)(8 * a.per_xcd)), dim3(kB), 0, s, vel, conc, a,
+                         vals, dep);
+      return hipGetLastError();
+    });
+  } else {
   // the composite velocity kinds run the default shape only (the host
   // sizes the grid for the shape it asks for: kDefaultStepShape then)
   if (vel.kind == kVelExtrap)
@@ -482,6 +675,7 @@ hipError_t launch_step_mode(const VelSource &vel, const TreeView &conc, const St
     default:  // shape 6, and the shapes not built for this degree
       return launch_step_rg_shape<MODE, T, 1024, 4>(vel, conc, a, vals, dep, s);
   }
+  }
 }
 
 }  // namespace
@@ -495,8 +689,16 @@ hipError_t TBX_CAT(launch_eval_q, TBX_Q)(int mode, const TreeView &t,
                                          hipStream_t s) {
   if (n <= 0) return hipSuccess;
   return with_mode(mode, [&](auto m) {
-    hipLaunchKernelGGL(k_eval<decltype(m)::value>, dim3(grid_for(n)), dim3(kBlock), 0, s, t, pts,
-                       n, bc, write_back, out);
+    constexpr int M = decltype(m)::value;
+    if constexpr (M == kExact64) {
+      hipLaunchKernelGGL(k_eval_exact, dim3(grid_for(n)), dim3(kBlock), 0, s, t, pts, n, bc,
+                         write_back, out);
+    } else {
+      with_rows_block(n, [&](auto b, unsigned grid) {
+        hipLaunchKernelGGL((k_eval<M, decltype(b)::value>), dim3(grid), dim3(decltype(b)::value),
+                           0, s, t, pts, n, bc, write_back, out);
+      });
+    }
     return hipGetLastError();
   });
 }
@@ -520,8 +722,17 @@ hipError_t TBX_CAT(launch_veval_q, TBX_Q)(int mode, const VelSource &vel,
   if (n <= 0) return hipSuccess;
   return with_mode(mode, [&](auto m) {
     return with_kind(vel.kind, [&](auto k) {
-      hipLaunchKernelGGL((k_veval<decltype(m)::value, decltype(k)::value>), dim3(grid_for(n)),
-                         dim3(kBlock), 0, s, vel, pts, n, bc, write_back, t, scaled, g, out);
+      constexpr int M = decltype(m)::value, K = decltype(k)::value;
+      if constexpr (M == kExact64) {
+        hipLaunchKernelGGL(k_veval_exact<K>, dim3(grid_for(n)), dim3(kBlock), 0, s, vel, pts, n,
+                           bc, write_back, t, scaled, g, out);
+      } else {
+        with_rows_block(n, [&](auto b, unsigned grid) {
+          hipLaunchKernelGGL((k_veval<M, K, decltype(b)::value>), dim3(grid),
+                             dim3(decltype(b)::value), 0, s, vel, pts, n, bc, write_back, t,
+                             scaled, g, out);
+        });
+      }
       return hipGetLastError();
     });
   });
@@ -533,8 +744,15 @@ hipError_t TBX_CAT(launch_traj_q, TBX_Q)(int mode, const VelSource &vel,
   if (n <= 0) return hipSuccess;
   return with_mode(mode, [&](auto m) {
     return with_kind(vel.kind, [&](auto k) {
-      hipLaunchKernelGGL((k_traj<decltype(m)::value, decltype(k)::value>), dim3(grid_for(n)),
-                         dim3(kBlock), 0, s, vel, x, n, a);
+      constexpr int M = decltype(m)::value, K = decltype(k)::value;
+      if constexpr (M == kExact64) {
+        hipLaunchKernelGGL(k_traj_exact<K>, dim3(grid_for(n)), dim3(kBlock), 0, s, vel, x, n, a);
+      } else {
+        with_rows_block(n, [&](auto b, unsigned grid) {
+          hipLaunchKernelGGL((k_traj<M, K, decltype(b)::value>), dim3(grid),
+                             dim3(decltype(b)::value), 0, s, vel, x, n, a);
+        });
+      }
       return hipGetLastError();
     });
   });

@@ -1,0 +1,56 @@
+"""The row contraction (a workgroup's points ordered by leaf, 16 lanes to a
+leaf) at the sizes where its ordering and padding change: point counts about
+the row, the wavefront and the two workgroup sizes, more leaves in a
+workgroup than its table has slots, points outside the domain, component
+counts about its groups of three, every class of degree.
+
+Bars: TBX_FP64 within 1e-12 relative L-inf of the oracle (sums of at most
+969 terms below 1 in FP64 rounding, as the other FP64 parity bars);
+TBX_FP32 within 2e-6 (FP32 rounding of as many); a point's value does not
+depend on the points around it (bit-identical)."""
+import numpy as np
+import pytest
+
+from conftest import random_tree
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("q", [1, 2, 3, 4, 7, 8, 11, 14, 15, 16])
+def test_rows_match_oracle(tb, orc, q):
+    import torch
+
+    dof = 1 + q % 5
+    anchor, depth = random_tree(q, max_depth=4, p_split=0.5, min_depth=2)
+    rng = np.random.default_rng(q)
+    deg = np.array([i + j + k for i in range(q + 1) for j in range(q + 1 - i)
+                    for k in range(q + 1 - i - j)])
+    coeff = rng.standard_normal((len(depth), dof, tb.ncoef(q))) * 0.5 ** deg
+    g, o = tb.Tree(anchor, depth, q, dof, coeff), orc.Tree(anchor, depth, q, dof, coeff)
+    pts = rng.random((65536 + 257, 3)) * 1.2 - 0.1  # some outside [0, 1]^3
+    pts[:400] = pts[0]                              # one leaf for whole workgroups
+    ref, _ = orc.eval_tree(o, pts, 0)
+    ref = ref.reshape(len(pts), dof)
+    big = np.abs(ref).max()
+    x = torch.from_numpy(pts).cuda()
+    whole = g.eval(x, 0, "fp64")
+    assert np.abs(whole.cpu().numpy() - ref).max() <= 1e-12 * big
+    assert np.abs(g.eval(x, 0, "fp32").cpu().numpy() - ref).max() <= 2e-6 * big
+    for n in (1, 15, 16, 17, 63, 64, 65, 255, 257, 1000, 65536):
+        a = len(pts) - n  # other neighbours, the same values
+        assert torch.equal(g.eval(x[a:].contiguous(), 0, "fp64"), whole[a:]), n
+
+
+def test_rows_nonfinite_leaf_stays_alone(tb):
+    import torch
+
+    anchor, depth = tb.uniform_leaves(2)
+    coeff = np.random.default_rng(0).standard_normal((64, 1, tb.ncoef(6)))
+    x = torch.rand((5000, 3), dtype=torch.float64, device="cuda")
+    t = tb.Tree(anchor, depth, 6, 1, coeff)
+    want, leaf = t.eval(x), t.locate(x)
+    coeff[5] = np.nan
+    coeff[9] = np.inf
+    got = tb.Tree(anchor, depth, 6, 1, coeff).eval(x)
+    bad = (leaf == 5) | (leaf == 9)
+    assert bool((~torch.isfinite(got[bad])).all()) and torch.equal(got[~bad], want[~bad])
