@@ -92,6 +92,104 @@ __global__ __launch_bounds__(kBlock) void k_to_f32(const double *__restrict__ in
   if (i < n) out[i] = (float)in[i];
 }
 
+// Order of a call's points by leaf (counting sort; order_words(n, L) words of
+// scratch): leaf and rank of every point, hist, then perm.  Groups follow
+// each other in no particular order; a point's place in its group depends on
+// the run, its value does not.
+//
+// k_order_count: rank = the point's number in its leaf.  A wavefront adds
+// once per leaf that several of its lanes share, so that many points of one
+// leaf do not queue on its counter.  meta[1] counts the wavefronts whose
+// neighbouring lanes change leaf eight times or more.
+__global__ __launch_bounds__(kBlock) void k_order_count(TreeView t,
+                                                        const double *__restrict__ pts,
+                                                        int64_t n, int bc,
+                                                        int32_t *__restrict__ leaf,
+                                                        int32_t *__restrict__ rank,
+                                                        int32_t *__restrict__ hist,
+                                                        int32_t *__restrict__ meta) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const bool live = i < n;
+  const int lane = (int)(threadIdx.x & 63u);
+  int lf = 0;
+  if (live) {
+    double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
+    if (bc == TBX_BC_PERIODIC) {
+      x = wrap1(x);
+      y = wrap1(y);
+      z = wrap1(z);
+    }
+    lf = locate(t, x, y, z);
+  }
+  const int left = __shfl_up(lf, 1, 64);
+  const int changes =
+      __builtin_popcountll(__builtin_amdgcn_ballot_w64(live && lane > 0 && lf != left));
+  const int scattered = __syncthreads_count(lane == 0 && changes >= 8);
+  if (threadIdx.x == 0 && scattered) atomicAdd(&meta[1], scattered);
+  uint64_t pending = __builtin_amdgcn_ballot_w64(live);
+  bool todo = live;
+  int r = 0;
+  for (int it = 0; it < 3 && pending; ++it) {
+    const int src = __builtin_ctzll(pending);
+    const int k = __builtin_amdgcn_readlane(lf, src);
+    const bool mine = todo && lf == k;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
+    if (__builtin_popcountll(m) < 4) break;
+    int base = 0;
+    if (lane == src) base = atomicAdd(&hist[k], __builtin_popcountll(m));
+    base = __builtin_amdgcn_readlane(base, src);
+    if (mine) {
+      r = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+      todo = false;
+    }
+    pending &= ~m;
+  }
+  if (todo) r = atomicAdd(&hist[lf], 1);
+  if (live) {
+    leaf[i] = lf;
+    rank[i] = r;
+  }
+}
+
+// hist[l] = first place of leaf l's points: a wavefront's 64 leaves take
+// their places together.  meta[0]: places taken so far.
+__global__ __launch_bounds__(kBlock) void k_order_start(int32_t *__restrict__ hist, int64_t L,
+                                                        int32_t *__restrict__ meta) {
+  const int64_t l = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int lane = (int)(threadIdx.x & 63u);
+  const int c = l < L ? hist[l] : 0;
+  int incl = c;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += o;
+  }
+  int base = 0;
+  if (lane == 63 && incl) base = atomicAdd(&meta[0], incl);
+  base = __builtin_amdgcn_readlane(base, 63);
+  if (l < L) hist[l] = base + incl - c;
+}
+
+// perm[place] = point; the identity where the points came in runs of a leaf
+// already (under a quarter of the wavefronts scattered), which keeps their
+// accesses coalesced.
+__global__ __launch_bounds__(kBlock) void k_order_place(const int32_t *__restrict__ leaf,
+                                                        const int32_t *__restrict__ rank,
+                                                        const int32_t *__restrict__ hist,
+                                                        const int32_t *__restrict__ meta,
+                                                        int64_t n, int32_t *__restrict__ perm) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const bool scattered = 4 * (int64_t)meta[1] > (n + 63) / 64;
+  perm[scattered ? hist[leaf[i]] + rank[i] : i] = (int32_t)i;
+}
+
+__global__ __launch_bounds__(kBlock) void k_zero_words(int32_t *__restrict__ p, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
 inline unsigned grid_for(int64_t n) {
   return (unsigned)((n + kBlock - 1) / kBlock);
 }
@@ -104,6 +202,21 @@ hipError_t launch_locate(const TreeView &t, const double *pts, int64_t n,
   const int64_t per = (int64_t)kBlock * kLocatePts;
   hipLaunchKernelGGL(k_locate, dim3((unsigned)((n + per - 1) / per)), dim3(kBlock), 0, s, t,
                      pts, n, bc, leaf);
+  return hipGetLastError();
+}
+
+int64_t order_words(int64_t n, int64_t L) { return 3 * n + L + 2; }
+
+hipError_t launch_order_points(const TreeView &t, const double *pts, int64_t n, int bc,
+                               int32_t *words, int32_t **perm, hipStream_t s) {
+  int32_t *leaf = words, *rank = leaf + n, *meta = rank + n, *hist = meta + 2;
+  *perm = hist + t.L;
+  hipLaunchKernelGGL(k_zero_words, dim3(grid_for(t.L + 2)), dim3(kBlock), 0, s, meta, t.L + 2);
+  hipLaunchKernelGGL(k_order_count, dim3(grid_for(n)), dim3(kBlock), 0, s, t, pts, n, bc, leaf,
+                     rank, hist, meta);
+  hipLaunchKernelGGL(k_order_start, dim3(grid_for(t.L)), dim3(kBlock), 0, s, hist, t.L, meta);
+  hipLaunchKernelGGL(k_order_place, dim3(grid_for(n)), dim3(kBlock), 0, s, leaf, rank, hist,
+                     meta, n, *perm);
   return hipGetLastError();
 }
 

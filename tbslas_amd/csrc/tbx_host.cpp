@@ -482,11 +482,12 @@ int prepare_view(tbx_tree *t, int mode, hipStream_t s, ScratchArena *arena, Tree
   X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16)
 
 hipError_t dispatch_eval(int q, int mode, const TreeView &t, double *pts,
-                         int64_t n, int bc, int wb, double *out, hipStream_t s) {
+                         int64_t n, int bc, int wb, double *out, const int32_t *perm,
+                         hipStream_t s) {
   switch (q) {
 #define X(Q) \
   case Q:    \
-    return launch_eval_q##Q(mode, t, pts, n, bc, wb, out, s);
+    return launch_eval_q##Q(mode, t, pts, n, bc, wb, out, perm, s);
     TBX_Q_CASES(X)
 #undef X
   }
@@ -518,12 +519,12 @@ hipError_t dispatch_veval(int q, int mode, const VelSource &vel, double *pts, in
   return hipErrorInvalidValue;
 }
 
-hipError_t dispatch_traj(int q, int mode, const VelSource &vel, double *x,
-                         int64_t n, const SubArgs &a, hipStream_t s) {
+hipError_t dispatch_traj(int q, int mode, const VelSource &vel, const double *x0, double *x,
+                         int64_t n, const SubArgs &a, const int32_t *perm, hipStream_t s) {
   switch (q) {
 #define X(Q) \
   case Q:    \
-    return launch_traj_q##Q(mode, vel, x, n, a, s);
+    return launch_traj_q##Q(mode, vel, x0, x, n, a, perm, s);
     TBX_Q_CASES(X)
 #undef X
   }
@@ -581,17 +582,108 @@ int check_bc(int bc) {
   return TBX_OK;
 }
 
-// Stage factors of one substep at current time tcur (traj.inc:33-40).
-SubArgs sub_args(double tcur, double tau, tbx_tfac_fn g, void *gctx, int bc) {
+// Scratch of one call, stream-ordered: from a pool per device that keeps up
+// to kPoolKeep bytes between calls (a plain hipMallocAsync returns its memory
+// to the system at the next synchronisation) and gives them back when the
+// device's last tree is destroyed.  Safe from several threads and streams.
+constexpr uint64_t kPoolKeep = (uint64_t)256 << 20;
+std::mutex g_pool_mu;
+struct DevicePool {
+  hipMemPool_t pool = nullptr;
+  int64_t trees = 0;
+};
+std::map<int, DevicePool> g_pools;
+
+void pool_tree_count(int device, int change) {
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  DevicePool &p = g_pools[device];
+  p.trees += change;
+  if (p.trees == 0 && p.pool) (void)hipMemPoolTrimTo(p.pool, 0);
+}
+
+// null without an error message where the memory is not to be had.
+void *pool_alloc(size_t bytes, hipStream_t s) {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return nullptr;
+  hipMemPool_t pool;
+  {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    DevicePool &p = g_pools[device];
+    if (!p.pool) {
+      hipMemPoolProps props{};
+      props.allocType = hipMemAllocationTypePinned;
+      props.location.type = hipMemLocationTypeDevice;
+      props.location.id = device;
+      uint64_t keep = kPoolKeep;
+      if (hipMemPoolCreate(&p.pool, &props) != hipSuccess ||
+          hipMemPoolSetAttribute(p.pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+        (void)hipGetLastError();
+        p.pool = nullptr;
+        return nullptr;
+      }
+    }
+    pool = p.pool;
+  }
+  void *m = nullptr;
+  if (hipMallocFromPoolAsync(&m, bytes, pool, s) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return m;
+}
+
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+// The order by leaf of n points that `evals` components are evaluated at,
+// where it pays: perm stays null, and the points are taken as they come,
+//  - in TBX_EXACT (its kernels take points as they come);
+//  - under kOrderWork multiply-adds in all (ordering costs some 15 us of
+//    launches and 40 us per million points), or fewer than two points a
+//    leaf (nothing to bring together);
+//  - on a stream that is being captured (nothing is allocated there), and
+//    without memory for it.
+constexpr double kOrderWork = 3e7;
+struct PointOrder {
+  void *words = nullptr;
+  int32_t *perm = nullptr;
+  hipStream_t s = nullptr;
+  hipError_t make(const tbx_tree *t, const double *pts, int64_t n, int bc, int mode, double evals,
+                  hipStream_t st) {
+    if (mode == kExact64 || n < 2 * t->L || n > INT32_MAX ||
+        (double)n * evals * t->nc < kOrderWork || capturing(st))
+      return hipSuccess;
+    words = pool_alloc(sizeof(int32_t) * (size_t)order_words(n, t->L), st);
+    if (!words) return hipSuccess;
+    s = st;
+    return launch_order_points(t->view(), pts, n, bc, (int32_t *)words, &perm, st);
+  }
+  ~PointOrder() {
+    if (words) (void)hipFreeAsync(words, s);
+  }
+};
+
+// Stage factors of n substeps from time tcur (traj.inc:33-40); tcur advances.
+SubArgs sub_args(double &tcur, double tau, int n, tbx_tfac_fn g, void *gctx, int bc) {
   SubArgs a{};
   a.tau = tau;
   a.htau = 0.5 * tau;
   a.scaled = g ? 1 : 0;
-  a.ts1 = tcur;
-  a.ts2 = tcur + 0.5 * tau;
-  a.g1 = g ? g(a.ts1, gctx) : 1.0;
-  a.g2 = g ? g(a.ts2, gctx) : 1.0;
   a.bc = bc;
+  a.nsub = n;
+  for (int k = 0; k < n; ++k) {
+    a.ts[2 * k] = tcur;
+    a.ts[2 * k + 1] = tcur + 0.5 * tau;
+    a.g[2 * k] = g ? g(a.ts[2 * k], gctx) : 1.0;
+    a.g[2 * k + 1] = g ? g(a.ts[2 * k + 1], gctx) : 1.0;
+    tcur = tcur + tau;  // traj.inc:65
+  }
   return a;
 }
 
@@ -815,6 +907,7 @@ int tbx_tree_create(const tbx_tree_desc *desc, tbx_tree **out) {
     free_tree(t);
     return rc;
   }
+  pool_tree_count(t->device, 1);
   *out = t;
   return TBX_OK;
 }
@@ -822,6 +915,7 @@ int tbx_tree_create(const tbx_tree_desc *desc, tbx_tree **out) {
 int tbx_tree_destroy(tbx_tree *t) {
   if (!t) return fail(TBX_EINVAL, "tbx_tree_destroy: null tree");
   hipDeviceSynchronize();
+  pool_tree_count(t->device, -1);
   free_tree(t);
   return TBX_OK;
 }
@@ -877,8 +971,10 @@ int tbx_eval(const tbx_tree *tc, double *pts, int64_t n, int bc, uint32_t flags,
   int mode;
   if ((rc = mode_of(flags, &mode))) return rc;
   if ((rc = prepare_mode(t, mode, (hipStream_t)s))) return rc;
+  PointOrder order;
+  HIP_TRY(order.make(t, pts, n, bc, mode, t->dof, (hipStream_t)s));
   HIP_TRY(dispatch_eval(t->q, mode, t->view(), pts, n, bc,
-                        (flags & TBX_WRITE_BACK_WRAP) ? 1 : 0, out, (hipStream_t)s));
+                        (flags & TBX_WRITE_BACK_WRAP) ? 1 : 0, out, order.perm, (hipStream_t)s));
   return TBX_OK;
 }
 
@@ -930,15 +1026,15 @@ int tbx_traj_rk2_v(const tbx_velocity *vel, const double *xinit, int64_t n, doub
   VelSource vs;
   if ((rc = prepare_velocity(vel, mode, (hipStream_t)s, &vs, &q, "tbx_traj_rk2"))) return rc;
   if (n == 0) return TBX_OK;
-  if (xsol != xinit)
-    HIP_TRY(hipMemcpyAsync(xsol, xinit, sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToDevice,
-                           (hipStream_t)s));
+  PointOrder order;  // by the start points' leaves, for all substeps
+  HIP_TRY(order.make(vel->trees[0], xinit, n, bc, mode, 6.0 * num_rk_step, (hipStream_t)s));
   const double tau = (tfinal - tinit) / num_rk_step;  // traj.inc:55
   double tcur = tinit;
-  for (int k = 0; k < num_rk_step; ++k) {
-    const SubArgs a = sub_args(tcur, tau, vel->g, vel->gctx, bc);
-    HIP_TRY(dispatch_traj(q, mode, vs, xsol, n, a, (hipStream_t)s));
-    tcur = tcur + tau;  // traj.inc:65
+  for (int k = 0; k < num_rk_step; k += kMaxSub) {
+    const SubArgs a =
+        sub_args(tcur, tau, std::min(kMaxSub, num_rk_step - k), vel->g, vel->gctx, bc);
+    HIP_TRY(dispatch_traj(q, mode, vs, k == 0 ? xinit : xsol, xsol, n, a, order.perm,
+                          (hipStream_t)s));
   }
   return TBX_OK;
 }
@@ -1395,7 +1491,7 @@ int tbx_adjoint_run(const tbx_tree *vel, tbx_tfac_fn g, void *gctx, tbx_tree *co
     auto forward = [&](int n, double *dep) -> int {
       if (stationary && keep_dep && have_dep && conc->dof == 1) {
         HIP_TRY(dispatch_eval(conc->q, c.mode, conc->view(), deps[0], (int64_t)conc->L * conc->P(),
-                              bc, 0, conc->d_vals, st));
+                              bc, 0, conc->d_vals, nullptr, st));
         return refit(conc, conc->d_vals, st);
       }
       const int r = step_insitu(&v, conc, n, dt, 1, bc, flags, dep, st, "tbx_adjoint_run");
@@ -2219,7 +2315,8 @@ int tbx_check_cheb_output(const tbx_tree *tc, const double *ref, uint32_t flags,
     double x[TBX_MAX_Q + 1];
     first_kind_nodes_host(n, x);
     HIP_TRY(launch_grid_points(t->view(), x, n, pts, st));
-    HIP_TRY(dispatch_eval(t->q, mode, t->view(), pts, npts, TBX_BC_FREESPACE, 0, val, st));
+    HIP_TRY(dispatch_eval(t->q, mode, t->view(), pts, npts, TBX_BC_FREESPACE, 0, val, nullptr,
+                          st));
     std::vector<double> h((size_t)nb * std::max(dof, 4));
     // pass 0: the volume-weighted mean error per component (utils.txx:158-187)
     HIP_TRY(launch_metric(t->d_info, n, val, ref, npts, dof, nullptr, 0, part, st));
@@ -2753,7 +2850,8 @@ int tbx_tree_write_vtu(const tbx_tree *tc, const char *prefix, int order, tbx_st
     HIP_TRY(hipMallocAsync((void **)&pts, sizeof(double) * 3 * (size_t)npts, st));
     HIP_TRY(hipMallocAsync((void **)&val, sizeof(double) * t->dof * (size_t)npts, st));
     HIP_TRY(launch_grid_points(t->view(), node, n, pts, st));
-    HIP_TRY(dispatch_eval(t->q, kFma64, t->view(), pts, npts, TBX_BC_FREESPACE, 0, val, st));
+    HIP_TRY(dispatch_eval(t->q, kFma64, t->view(), pts, npts, TBX_BC_FREESPACE, 0, val, nullptr,
+                          st));
     HIP_TRY(hipMemcpyAsync(hval.data(), val, sizeof(double) * hval.size(), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     return TBX_OK;

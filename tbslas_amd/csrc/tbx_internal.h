@@ -55,15 +55,14 @@ struct VelSource {
 
 constexpr int kMaxSub = 16;  // RK substeps fused into one step launch
 
-// One IntegrateRK2 substep: stage factors of the time modulation.
+// Consecutive IntegrateRK2 substeps: stage factors of the time modulation.
 struct SubArgs {
   double tau;   // (tfinal - tinit) / num_rk_step   (traj.inc:55)
   double htau;  // 0.5 * tau                         (traj.inc:36)
-  double g1;    // g(t)            (1 when steady)
-  double g2;    // g(t + 0.5 tau)
-  double ts1;   // stage times t and t + 0.5 tau (traj.inc:33, 40)
-  double ts2;
-  int scaled;   // multiply by g1/g2
+  double g[2 * kMaxSub];   // g(t), g(t + 0.5 tau) per substep (1 when steady)
+  double ts[2 * kMaxSub];  // stage times t and t + 0.5 tau (traj.inc:33, 40)
+  int nsub;
+  int scaled;   // multiply by g
   int bc;
 };
 
@@ -135,9 +134,11 @@ constexpr int kAdjBlock = 256;  // workgroup of the adjoint concentration kernel
 #define TBX_DECLARE_Q(Q)                                                      \
   hipError_t launch_eval_q##Q(int mode, const TreeView &t, double *pts,       \
                               int64_t n, int bc, int write_back, double *out, \
+                              const int32_t *perm, hipStream_t s);            \
+  hipError_t launch_traj_q##Q(int mode, const VelSource &vel,                 \
+                              const double *x0, double *x, int64_t n,         \
+                              const SubArgs &a, const int32_t *perm,          \
                               hipStream_t s);                                 \
-  hipError_t launch_traj_q##Q(int mode, const VelSource &vel, double *x,      \
-                              int64_t n, const SubArgs &a, hipStream_t s);    \
   hipError_t launch_step_q##Q(int mode, const VelSource &vel,                 \
                               const TreeView &conc, const StepArgs &a,        \
                               double *vals, double *dep, hipStream_t s);      \
@@ -280,6 +281,11 @@ hipError_t launch_gather_rows(const double *src, const int64_t *map, int64_t nro
                               double *dst, hipStream_t s);
 
 // Degree-independent launchers (tbx_common.hip).
+// Order of n points by leaf: *perm (inside words, order_words(n, L) 32-bit
+// words) lists the points, those of a leaf together.  n < 2^31.
+int64_t order_words(int64_t n, int64_t L);
+hipError_t launch_order_points(const TreeView &t, const double *pts, int64_t n, int bc,
+                               int32_t *words, int32_t **perm, hipStream_t s);
 hipError_t launch_locate(const TreeView &t, const double *pts, int64_t n,
                          int bc, int32_t *leaf, hipStream_t s);
 hipError_t launch_grid_points(const TreeView &t, const double *node, int d,

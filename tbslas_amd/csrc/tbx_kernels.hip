@@ -76,15 +76,17 @@ __global__ __launch_bounds__(kBlock) void k_veval_exact(VelSource vel, double *_
   out[3 * i + 2] = v2;
 }
 
-// One IntegrateRK2 substep for caller points, in place, as k_eval_exact.
+// IntegrateRK2 substeps for caller points (x0 may be xs), as k_eval_exact.
 template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_traj_exact(VelSource vel, double *__restrict__ xs,
-                                                       int64_t n, SubArgs a) {
+__global__ __launch_bounds__(kBlock) void k_traj_exact(VelSource vel, const double *x0,
+                                                       double *xs, int64_t n, SubArgs a) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  double x = xs[3 * i + 0], y = xs[3 * i + 1], z = xs[3 * i + 2];
-  rk2_substep<D, kExact64, KIND>(vel, a.bc, a.htau, a.tau, a.scaled, a.g1, a.g2, a.ts1, a.ts2, x,
-                                 y, z);
+  double x = x0[3 * i + 0], y = x0[3 * i + 1], z = x0[3 * i + 2];
+#pragma unroll 1
+  for (int s = 0; s < a.nsub; ++s)
+    rk2_substep<D, kExact64, KIND>(vel, a.bc, a.htau, a.tau, a.scaled, a.g[2 * s],
+                                   a.g[2 * s + 1], a.ts[2 * s], a.ts[2 * s + 1], x, y, z);
   xs[3 * i + 0] = x;
   xs[3 * i + 1] = y;
   xs[3 * i + 2] = z;
@@ -92,16 +94,17 @@ __global__ __launch_bounds__(kBlock) void k_traj_exact(VelSource vel, double *__
 
 // The same three in the other modes: a workgroup's points ordered by leaf
 // and contracted row by row (tbx_rows.h).  Threads past the last point hold
-// a copy of it and take no part.  BLOCK: 256 threads, or 64 where that
-// leaves compute units without a workgroup (rows_block).
+// a copy of it and take no part.  BLOCK: with_rows_block.  perm (may be
+// null): the order of the points, those of a leaf together.
 template <int MODE, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_eval(
     TreeView t, double *__restrict__ pts, int64_t n, int bc, int write_back,
-    double *__restrict__ out) {
+    double *__restrict__ out, const int32_t *__restrict__ perm) {
   __shared__ RowsLds<BLOCK> sh;
   const int64_t i0 = (int64_t)blockIdx.x * BLOCK;
   const bool live = i0 + (int)threadIdx.x < n;
-  const int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
+  int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
+  if (perm) i = perm[i];
   double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
   if (bc == TBX_BC_PERIODIC) {
     x = wrap1(x);
@@ -152,14 +155,18 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
 
 template <int MODE, int KIND, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_traj(
-    VelSource vel, double *__restrict__ xs, int64_t n, SubArgs a) {
+    VelSource vel, const double *x0, double *xs, int64_t n, SubArgs a,
+    const int32_t *__restrict__ perm) {
   __shared__ RowsLds<BLOCK> sh;
   const int64_t i0 = (int64_t)blockIdx.x * BLOCK;
   const bool live = i0 + (int)threadIdx.x < n;
-  const int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
-  double x = xs[3 * i + 0], y = xs[3 * i + 1], z = xs[3 * i + 2];
-  rows_substep<D, MODE, KIND>(sh, vel, a.bc, a.htau, a.tau, a.scaled, a.g1, a.g2, a.ts1, a.ts2,
-                              live, x, y, z);
+  int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
+  if (perm) i = perm[i];
+  double x = x0[3 * i + 0], y = x0[3 * i + 1], z = x0[3 * i + 2];
+#pragma unroll 1
+  for (int s = 0; s < a.nsub; ++s)
+    rows_substep<D, MODE, KIND>(sh, vel, a.bc, a.htau, a.tau, a.scaled, a.g[2 * s],
+                                a.g[2 * s + 1], a.ts[2 * s], a.ts[2 * s + 1], live, x, y, z);
   if (!live) return;
   xs[3 * i + 0] = x;
   xs[3 * i + 1] = y;
@@ -477,7 +484,7 @@ __device__ __forceinline__ void k_step_rows_body(const VelSource &vel, const Tre
 #pragma unroll 1
     for (int p0 = (int)(threadIdx.x & ~63u); p0 < count; p0 += BLOCK) {
       const int pos = p0 + (int)(threadIdx.x & 63u);
-      const int src = sh.order[pos < count ? pos : count - 1];
+      const int src = sh.order[pos < count ? pos : count - 1] & kPlaceMask;
       const uint32_t q = r0 + (uint32_t)src;
       eval_dof_mfma<D, T>(conc, sh.leaf[src], sh.e[0][src], sh.e[1][src], sh.e[2][src], vals,
                           (l0 + q / (uint32_t)P) * conc.dof * P + (int64_t)(q % (uint32_t)P), P,
@@ -686,7 +693,7 @@ hipError_t launch_step_mode(const VelSource &vel, const TreeView &conc, const St
 hipError_t TBX_CAT(launch_eval_q, TBX_Q)(int mode, const TreeView &t,
                                          double *pts, int64_t n, int bc,
                                          int write_back, double *out,
-                                         hipStream_t s) {
+                                         const int32_t *perm, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   return with_mode(mode, [&](auto m) {
     constexpr int M = decltype(m)::value;
@@ -696,7 +703,7 @@ hipError_t TBX_CAT(launch_eval_q, TBX_Q)(int mode, const TreeView &t,
     } else {
       with_rows_block(n, [&](auto b, unsigned grid) {
         hipLaunchKernelGGL((k_eval<M, decltype(b)::value>), dim3(grid), dim3(decltype(b)::value),
-                           0, s, t, pts, n, bc, write_back, out);
+                           0, s, t, pts, n, bc, write_back, out, perm);
       });
     }
     return hipGetLastError();
@@ -739,18 +746,20 @@ hipError_t TBX_CAT(launch_veval_q, TBX_Q)(int mode, const VelSource &vel,
 }
 
 hipError_t TBX_CAT(launch_traj_q, TBX_Q)(int mode, const VelSource &vel,
-                                         double *x, int64_t n,
-                                         const SubArgs &a, hipStream_t s) {
+                                         const double *x0, double *x,
+                                         int64_t n, const SubArgs &a,
+                                         const int32_t *perm, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   return with_mode(mode, [&](auto m) {
     return with_kind(vel.kind, [&](auto k) {
       constexpr int M = decltype(m)::value, K = decltype(k)::value;
       if constexpr (M == kExact64) {
-        hipLaunchKernelGGL(k_traj_exact<K>, dim3(grid_for(n)), dim3(kBlock), 0, s, vel, x, n, a);
+        hipLaunchKernelGGL(k_traj_exact<K>, dim3(grid_for(n)), dim3(kBlock), 0, s, vel, x0, x, n,
+                           a);
       } else {
         with_rows_block(n, [&](auto b, unsigned grid) {
           hipLaunchKernelGGL((k_traj<M, K, decltype(b)::value>), dim3(grid),
-                             dim3(decltype(b)::value), 0, s, vel, x, n, a);
+                             dim3(decltype(b)::value), 0, s, vel, x0, x, n, a, perm);
         });
       }
       return hipGetLastError();

@@ -300,6 +300,24 @@ __device__ __forceinline__ T row_contract(const T *__restrict__ c, const T (&px)
 // ---------------------------------------------------------------------------
 // A workgroup's points.
 // ---------------------------------------------------------------------------
+// order's entries: a thread, with the bits above kPlaceMask set where the
+// place is a copy that pads a run.
+constexpr int kPlaceMask = 0x7fff;
+
+// The leaf of the first pending lane of the lane's DPP row (of its first
+// lane, if none is).
+__device__ __forceinline__ int row_leaf(uint64_t pending, int leaf) {
+  const int row = (int)(threadIdx.x & 48u);
+  const uint32_t rest = (uint32_t)(pending >> row) & 0xffffu;
+  return __builtin_amdgcn_ds_bpermute((row + (rest ? __builtin_ctz(rest) : 0)) << 2, leaf);
+}
+
+// Orders a wavefront's LDS writes before its other lanes' reads.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <int BLOCK>
 struct RowsLds {
   double e[3][BLOCK];  // leaf coordinates in, values out (per thread's point)
@@ -314,8 +332,10 @@ struct RowsLds {
 // Orders the active threads' points by leaf: afterwards order[0, count) are
 // their threads, points of one leaf together and padded to a multiple of 16
 // with copies of the last one; returns count, a multiple of 16.  Leaves
-// beyond kRgSlots share the last run.  A wavefront enters each of its
-// distinct leaves once (one hash probe and one add per leaf, not per lane).
+// that find no slot in eight probes share the last run.  A wavefront enters
+// leaves that several of its lanes share once for them all, until it meets
+// one of under three lanes (scattered points enter lane by lane, in
+// parallel: one after another 64 leaves would take some 20,000 clocks).
 // Every thread of the workgroup must call it; the caller synchronises
 // before order is read.
 template <int BLOCK>
@@ -326,26 +346,30 @@ __device__ __forceinline__ int order_by_leaf(RowsLds<BLOCK> &s, bool active, int
     s.cnt[i] = 0;
   }
   __syncthreads();
-  int slot = 0, rank = 0;
+  int slot = kRgSlots, rank = 0;
+  bool todo = active;
+  auto insert = [&]() {  // the thread's leaf into the table: its slot
+    uint32_t h = ((uint32_t)leaf * 0x9E3779B1u) >> 26;  // 6 bits: kRgSlots == 64
+#pragma unroll 1
+    for (int probe = 0; probe < 8; ++probe) {
+      const int prev = atomicCAS(&s.key[h], -1, leaf);
+      if (prev == -1 || prev == leaf) return (int)h;
+      h = (h + 1) & (kRgSlots - 1);
+    }
+    return kRgSlots;
+  };
   uint64_t pending = __builtin_amdgcn_ballot_w64(active);
-  while (pending) {
+#pragma unroll 1
+  for (int it = 0; it < 6 && pending; ++it) {
     const int src = __builtin_ctzll(pending);
     const int k = __builtin_amdgcn_readlane(leaf, src);
-    const bool mine = active && leaf == k;
+    const bool mine = todo && leaf == k;
     const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
+    if (__builtin_popcountll(m) < 3) break;
     pending &= ~m;
     int sl = kRgSlots, base = 0;
     if (lane == src) {
-      uint32_t h = ((uint32_t)k * 0x9E3779B1u) >> 26;  // 6 bits: kRgSlots == 64
-#pragma unroll 1
-      for (int probe = 0; probe < kRgSlots; ++probe) {
-        const int prev = atomicCAS(&s.key[h], -1, k);
-        if (prev == -1 || prev == k) {
-          sl = (int)h;
-          break;
-        }
-        h = (h + 1) & (kRgSlots - 1);
-      }
+      sl = insert();
       base = atomicAdd(&s.cnt[sl], __builtin_popcountll(m));
     }
     sl = __builtin_amdgcn_readlane(sl, src);
@@ -354,7 +378,12 @@ __device__ __forceinline__ int order_by_leaf(RowsLds<BLOCK> &s, bool active, int
       slot = sl;
       rank = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                               __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+      todo = false;
     }
+  }
+  if (todo) {
+    slot = insert();
+    rank = atomicAdd(&s.cnt[slot], 1);
   }
   __syncthreads();
   const int mine = s.cnt[slot];  // points of the thread's run
@@ -375,7 +404,7 @@ __device__ __forceinline__ int order_by_leaf(RowsLds<BLOCK> &s, bool active, int
   if (active) {
     s.order[first + rank] = (uint16_t)tid;
     if (rank == mine - 1)
-      for (int i = rank + 1; i & 15; ++i) s.order[first + i] = (uint16_t)tid;
+      for (int i = rank + 1; i & 15; ++i) s.order[first + i] = (uint16_t)(tid | ~kPlaceMask);
   }
   return count;
 }
@@ -395,7 +424,7 @@ __device__ __forceinline__ void rows(RowsLds<BLOCK> &s, const TreeView &t, int c
   const int lane = (int)(threadIdx.x & 63u);
 #pragma unroll 1
   for (int p0 = (int)(threadIdx.x & ~63u); p0 < count; p0 += BLOCK) {
-    const int src = s.order[p0 + lane < count ? p0 + lane : count - 1];
+    const int src = s.order[p0 + lane < count ? p0 + lane : count - 1] & kPlaceMask;
     const int leaf = s.leaf[src];
     const double ex = s.e[0][src], ey = s.e[1][src], ez = s.e[2][src];
     // zero outside [-1, 1] (cheb_poly); evaluated at 0 there and dropped
@@ -407,10 +436,7 @@ __device__ __forceinline__ void rows(RowsLds<BLOCK> &s, const TreeView &t, int c
     uint64_t pending = __builtin_amdgcn_ballot_w64(true);
 #pragma unroll 1
     while (pending) {
-      // the leaf of the row's first pending lane (of any, if none is)
-      const uint32_t rest = (uint32_t)(pending >> (lane & 48)) & 0xffffu;
-      const int from = (lane & 48) + (rest ? __builtin_ctz(rest) : 0);
-      const int lf = __builtin_amdgcn_ds_bpermute(from << 2, leaf);
+      const int lf = row_leaf(pending, leaf);
       const bool mine = leaf == lf;
       pending &= ~__builtin_amdgcn_ballot_w64(mine);
       const T *cb = coeff_base<MODE>(t) + ((size_t)lf * t.dof + c0) * NC + (lane & 15);

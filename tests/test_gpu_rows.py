@@ -54,3 +54,73 @@ def test_rows_nonfinite_leaf_stays_alone(tb):
     got = tb.Tree(anchor, depth, 6, 1, coeff).eval(x)
     bad = (leaf == 5) | (leaf == 9)
     assert bool((~torch.isfinite(got[bad])).all()) and torch.equal(got[~bad], want[~bad])
+
+
+def _tree(tb, q, dof, seed):
+    anchor, depth = random_tree(seed, max_depth=4, p_split=0.4, min_depth=2)
+    deg = np.array([i + j + k for i in range(q + 1) for j in range(q + 1 - i)
+                    for k in range(q + 1 - i - j)])
+    rng = np.random.default_rng(seed)
+    return tb.Tree(anchor, depth, q, dof,
+                   rng.standard_normal((len(depth), dof, tb.ncoef(q))) * 0.3 ** deg)
+
+
+@pytest.mark.parametrize("mode", ["fp64", "fp32", "fp32h"])
+@pytest.mark.parametrize("kind", ["uniform", "one leaf", "sorted", "outside"])
+def test_points_ordered_by_leaf_keep_their_values(tb, mode, kind):
+    # 300,001 points of degree 8 and three components are ordered by leaf
+    # first, 3,000 at a time they are not: the same bits
+    import torch
+
+    t = _tree(tb, 8, 3, 2)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.rand((300001, 3), dtype=torch.float64, device="cuda", generator=g)
+    if kind == "one leaf":
+        x[1000:] = x[1000:] * 0.01 + 0.5
+    elif kind == "sorted":
+        x = x[t.locate(x).argsort()].contiguous()
+    elif kind == "outside":
+        x = x * 1.5 - 0.25
+    bc = int(kind == "outside")
+    y = x.clone()
+    whole = t.eval(y, bc, mode, write_back=True)
+    parts = torch.cat([t.eval(x[a:a + 3000].contiguous(), bc, mode) for a in range(0, len(x), 3000)])
+    assert torch.equal(whole, parts)
+    want = torch.where(x < 0, x + 1, torch.where(x >= 1, x - 1, x)) if bc else x
+    assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("nrk", [1, 3, 16, 17, 33])
+def test_ordered_trajectories_keep_their_values(tb, nrk):
+    import torch
+
+    v = _tree(tb, 6, 3, 5)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.rand((200003, 3), dtype=torch.float64, device="cuda", generator=g)
+    whole = tb.traj_rk2(v, x, 0.1, 0.0, nrk, 1, g=lambda t: 1.0 + t)
+    parts = torch.cat([tb.traj_rk2(v, x[a:a + 1000].contiguous(), 0.1, 0.0, nrk, 1,
+                                   g=lambda t: 1.0 + t) for a in range(0, len(x), 1000)])
+    assert torch.equal(whole, parts)
+    y = x.clone()
+    tb.traj_rk2(v, y, 0.1, 0.0, nrk, 1, g=lambda t: 1.0 + t, out=y)
+    assert torch.equal(y, whole)
+
+
+def test_evaluation_under_capture(tb):
+    # a captured call allocates nothing and takes the points as they come
+    import torch
+
+    t = _tree(tb, 8, 3, 3)
+    x = torch.rand((200001, 3), dtype=torch.float64, device="cuda")
+    want = t.eval(x)
+    s = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        out = t.eval(x)
+    for _ in range(3):
+        out.zero_()
+        x.copy_(torch.rand_like(x))
+        want = t.eval(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
