@@ -17,7 +17,7 @@
 
 #include <type_traits>
 
-#include "tbx_device.h"
+#include "tbx_rows.h"
 
 #ifndef TBX_Q
 #error "compile with -DTBX_Q=<degree>"
@@ -30,201 +30,292 @@ constexpr int D = TBX_Q + 1;
 constexpr int NC = D * (D + 1) * (D + 2) / 6;
 
 // T_0..T_{D-1} and dT/dxi by differentiating the three-term recurrence,
-// dT_{k+1} = 2 T_k + 2 xi dT_k - dT_{k-1}; zeros outside [-1,1] like
-// cheb_poly.
-__device__ __forceinline__ void cheb_poly_d(double x, double *p, double *dp) {
-  const bool in = fabs(x) <= 1.0;
-  const double xx = in ? x : 0.0;
-  p[0] = in ? 1.0 : 0.0;
+// dT_{k+1} = 2 T_k + 2 xi dT_k - dT_{k-1}, at x inside [-1, 1].
+__device__ __forceinline__ void cheb_poly_d(double x, double (&p)[D], double (&dp)[D]) {
+  const double x2 = 2.0 * x;
+  p[0] = 1.0;
   dp[0] = 0.0;
   if constexpr (D > 1) {
-    p[1] = xx;
-    dp[1] = p[0];
+    p[1] = x;
+    dp[1] = 1.0;
   }
 #pragma unroll
   for (int k = 2; k < D; ++k) {
-    p[k] = 2.0 * xx * p[k - 1] - p[k - 2];
-    dp[k] = 2.0 * p[k - 1] + 2.0 * xx * dp[k - 1] - dp[k - 2];
+    p[k] = __builtin_fma(x2, p[k - 1], -p[k - 2]);
+    dp[k] = __builtin_fma(2.0, p[k - 1], __builtin_fma(x2, dp[k - 1], -dp[k - 2]));
   }
 }
 
-// Basis and its derivatives at one point, in the point's leaf.
-struct AdjBasis {
-  int leaf;
-  double s2;  // d xi / dx = 2 * 2^depth
-  double tx[D], ty[D], tz[D], dx[D], dy[D], dz[D];
-
-  __device__ __forceinline__ void build(const TreeView &t, double x, double y, double z,
-                                        int hint = -1) {
-    leaf = hint >= 0 ? hint : locate(t, x, y, z);
-    double ex, ey, ez;
-    leaf_xi(t, leaf, x, y, z, ex, ey, ez);
-    s2 = 2.0 * (double)(1u << t.info[leaf].w);
-    cheb_poly_d(ex, tx, dx);
-    cheb_poly_d(ey, ty, dy);
-    cheb_poly_d(ez, tz, dz);
-  }
-};
-
-// Gradient (d/dx, d/dy, d/dz) of one component at the point of b, c the
-// component's coefficients in b's leaf.  One pass over the packed triangle:
-// every coefficient feeds the x-derivative and the value sums along k, and
-// the (i, j) partial sums are then combined with the y and z bases and
-// derivatives.
-__device__ __forceinline__ void grad3(const double *c, const AdjBasis &b, double &gx,
-                                      double &gy, double &gz) {
-  double ux = 0.0, uy = 0.0, uz = 0.0;
-  int idx = 0;
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
+// Gradient (d/dxi_x, d/dxi_y, d/dxi_z) of one component at the lane's
+// point, the lane's DPP row sharing the leaf (row_contract in tbx_rows.h):
+// one pass over the packed triangle, every coefficient feeding the value
+// and the x-derivative sums along k; the (i, j) sums are then combined with
+// the y and z bases and derivatives.
+__device__ __forceinline__ void row_grad(const double *__restrict__ c, const double (&px)[D],
+                                         const double (&dx)[D], const double (&py)[D],
+                                         const double (&dy)[D], double z, double &gx,
+                                         double &gy, double &gz) {
+  constexpr int NB = (NC + 15) / 16, kRing = 4;
+  double r[kRing];
+  static_for<(kRing - 1 < NB ? kRing - 1 : NB)>([&](auto bc) {
+    constexpr int b = decltype(bc)::value;
+    r[b] = c[16 * b];
+  });
+  gx = gy = gz = 0.0;
+  const double z2 = 2.0 * z;
+  double zm = 0.0, zc = 1.0, dm = 0.0, dc = 0.0;  // T_{i-1}, T_i and derivatives
+  static_for<D>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
     double vx = 0.0, vy = 0.0, v = 0.0;
-#pragma unroll
-    for (int j = 0; i + j < D; ++j) {
-      double wx = 0.0, w = 0.0;
-#pragma unroll
-      for (int k = 0; i + j + k < D; ++k) {
-        const double cm = load_uniform(c + idx++);
-        wx = __builtin_fma(b.dx[k], cm, wx);
-        w = __builtin_fma(b.tx[k], cm, w);
-      }
-      vx = __builtin_fma(b.ty[j], wx, vx);
-      vy = __builtin_fma(b.dy[j], w, vy);
-      v = __builtin_fma(b.ty[j], w, v);
-    }
-    ux = __builtin_fma(b.tz[i], vx, ux);
-    uy = __builtin_fma(b.tz[i], vy, uy);
-    uz = __builtin_fma(b.dz[i], v, uz);
-  }
-  gx = ux * b.s2;
-  gy = uy * b.s2;
-  gz = uz * b.s2;
-}
-
-// Cross-lane exchanges of one double.  swap_add32 / swap_add16: with lo
-// and hi two blocks of values, lanes whose bit 5 (bit 4) is clear return
-// lo + lo of lane l ^ 32 (l ^ 16) and the others hi + hi of that lane
-// (v_permlane32_swap / v_permlane16_swap exchange the upper lanes of the
-// first operand with the lower lanes of the second).  dpp_pair: the value
-// of the partner lane of a DPP pattern (row_ror:8 = l ^ 8 in a row,
-// row_half_mirror = 7 - l in each eight, quad_perm = l ^ 2, l ^ 1).
-__device__ __forceinline__ double swap_add32(double lo, double hi) {
-  const auto a = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(lo),
-                                                  (unsigned)__double2loint(hi), false, false);
-  const auto b = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(lo),
-                                                  (unsigned)__double2hiint(hi), false, false);
-  return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
-}
-
-__device__ __forceinline__ double swap_add16(double lo, double hi) {
-  const auto a = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(lo),
-                                                  (unsigned)__double2loint(hi), false, false);
-  const auto b = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(lo),
-                                                  (unsigned)__double2hiint(hi), false, false);
-  return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
-}
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_pair(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-
-// One halving step over b[0, 2H): the lane keeps the upper half when
-// `upper`, sends the other half to its partner and adds what it receives.
-template <int CTRL, int H, int N>
-__device__ __forceinline__ void halve(double (&b)[N], bool upper) {
-#pragma unroll
-  for (int t = 0; t < H; ++t) {
-    const double send = upper ? b[t] : b[t + H];
-    const double keep = upper ? b[t + H] : b[t];
-    b[t] = keep + dpp_pair<CTRL>(send);
-  }
-}
-
-// Reduce-scatter over the wave (all 64 lanes active): on return lane l
-// holds the sum over all lanes of b[l] (N = 64), or, for N = 32, lanes l
-// and l ^ 1 both hold the sum of b[l >> 1].  Recursive halving: at every
-// step the two partners hold the same block of indices and each keeps one
-// half, so N - 1 exchanges replace N full reductions.
-template <int N>
-__device__ __forceinline__ double wave_reduce_scatter(double (&b)[N]) {
-  static_assert(N == 64 || N == 32, "chunk of 32 or 64");
-  const unsigned l = threadIdx.x & 63u;
-  constexpr int H1 = N / 2, H2 = N / 4, H3 = N / 8, H4 = N / 16, H5 = N / 32;
-#pragma unroll
-  for (int t = 0; t < H1; ++t) b[t] = swap_add32(b[t], b[t + H1]);
-#pragma unroll
-  for (int t = 0; t < H2; ++t) b[t] = swap_add16(b[t], b[t + H2]);
-  halve<0x128, H3>(b, (l & 8u) != 0);
-  halve<0x141, H4>(b, (l & 4u) != 0);
-  halve<0x4e, H5>(b, (l & 2u) != 0);
-  if constexpr (N == 64)
-    halve<0xb1, 1>(b, (l & 1u) != 0);
-  else
-    b[0] = b[0] + dpp_pair<0xb1>(b[0]);
-  return b[0];
-}
-
-// (i, j, k) of packed triangle index m (order i(z) -> j(y) -> k(x)).
-struct Tri {
-  int i[NC], j[NC], k[NC];
-  constexpr Tri() : i(), j(), k() {
-    int m = 0;
-    for (int a = 0; a < D; ++a)
-      for (int b = 0; a + b < D; ++b)
-        for (int c = 0; a + b + c < D; ++c) {
-          i[m] = a;
-          j[m] = b;
-          k[m] = c;
-          ++m;
+    static_for<D - i>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      constexpr int first = tri_start(D, i, j), len = D - i - j;
+      double w = 0.0, wx = 0.0;
+      static_for<2>([&](auto hc) {  // the row's coefficients, cut at multiples of 16
+        constexpr int h = decltype(hc)::value;
+        constexpr int b = first / 16 + h;
+        constexpr int lo = h == 0 ? first : 16 * b;
+        constexpr int hi = first + len < 16 * (b + 1) ? first + len : 16 * (b + 1);
+        if constexpr (lo < hi) {
+          if constexpr (lo % 16 == 0 && b + kRing - 1 < NB) {
+            asm volatile("" ::: "memory");  // loads stay kRing - 1 blocks ahead
+            r[(b + kRing - 1) % kRing] = c[16 * (b + kRing - 1)];
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          const double cb = r[b % kRing];
+          if constexpr (lo == first) {
+            row_start<lo % 16, hi - lo>(w, cb, px + 1);
+            if constexpr (hi - lo > 1) row_add<lo % 16 + 1, hi - lo - 1>(wx, cb, dx + 1);
+          } else {
+            row_add<0, hi - lo>(w, cb, px + (lo - first));
+            row_add<0, hi - lo>(wx, cb, dx + (lo - first));
+          }
         }
+      });
+      if constexpr (j == 0) {
+        v = w;
+        vx = wx;
+      } else {
+        fmac_here(v, py[j], w);
+        fmac_here(vx, py[j], wx);
+        fmac_here(vy, dy[j], w);
+      }
+    });
+    if constexpr (i == 0) {
+      gx = vx;
+      gy = vy;
+    } else {
+      if constexpr (i == 1) {
+        zm = 1.0;
+        zc = z;
+        dc = 1.0;
+      } else {
+        const double zn = __builtin_fma(z2, zc, -zm);
+        const double dn = __builtin_fma(2.0, zc, __builtin_fma(z2, dc, -dm));
+        zm = zc;
+        zc = zn;
+        dm = dc;
+        dc = dn;
+      }
+      fmac_here(gx, zc, vx);
+      fmac_here(gy, zc, vy);
+      fmac_here(gz, dc, v);
+    }
+  });
+}
+
+// Rows (i, j) of the transposed interpolation's tiles, sorted by n = i + j.
+struct ScatterRows {
+  static constexpr int R = D * (D + 1) / 2;
+  static constexpr int NT = (R + 15) / 16;
+  int8_t i[16 * NT], j[16 * NT];  // i = -1: padding
+  int len[NT];                    // values of k of the tile's longest row
+  constexpr ScatterRows() : i(), j(), len() {
+    int r = 0;
+    for (int n = 0; n < D; ++n)
+      for (int a = 0; a <= n; ++a) {
+        i[r] = (int8_t)a;
+        j[r] = (int8_t)(n - a);
+        ++r;
+      }
+    for (; r < 16 * NT; ++r) {
+      i[r] = -1;
+      j[r] = 0;
+    }
+    for (int t = 0; t < NT; ++t) len[t] = D - i[16 * t] - j[16 * t];
   }
 };
-constexpr Tri kTri{};
+constexpr ScatterRows kRows{};
+__device__ const ScatterRows kDevRows{};
 
-// Transposed interpolation of ncomp weighted components: for every leaf
-// held by a lane of the wave, G[leaf][c][m] += sum over its lanes of
-// w(c) B_m(point).  All lanes of the wave must be active; each lane's basis
-// b is in its own leaf.  The coefficients go in chunks of CH (64 or 32:
-// CH doubles of registers per lane) through the wave reduce-scatter, one
-// coalesced atomic add per lane and chunk.
-template <int CH, typename W>
-__device__ __forceinline__ void scatter_transposed(double *G, int ncomp, const AdjBasis &b,
-                                                   W weight) {
-  constexpr int PER = 64 / CH;  // lanes per reduced coefficient
+// Tiles of 16 (k, component) columns an M tile needs, and the first tile's
+// index among all.
+constexpr int scatter_cols(int t, int ncomp) { return (kRows.len[t] * ncomp + 15) / 16; }
+constexpr int scatter_first(int t, int ncomp) {
+  int n = 0;
+  for (int a = 0; a < t; ++a) n += scatter_cols(a, ncomp);
+  return n;
+}
+
+// A workgroup's adjoint points: RowsLds holds their leaf coordinates, w the
+// weights per component, g the gradients; scratch per wavefront.
+template <int BLOCK>
+struct AdjLds {
+  RowsLds<BLOCK> r;
+  double w[3][BLOCK];
+  double g[3][BLOCK];
+  double t[BLOCK / 64][3][D][16];  // T_k of a group's 16 points per axis
+  double sw[BLOCK / 64][3][16];    // their weights
+};
+
+// s.g = sum over c < nc of w[c] grad_xi(component c of t) at the points in
+// order[0, count) (zero outside the leaf's box, as the basis).  The caller
+// synchronises before and after.
+template <int BLOCK>
+__device__ __forceinline__ void rows_gradient(AdjLds<BLOCK> &s, const TreeView &t, int c0, int nc,
+                                              int count) {
   const int lane = (int)(threadIdx.x & 63u);
-  const bool writer = (lane % PER) == 0;
-  const int slot = lane / PER;
-  uint64_t pending = __builtin_amdgcn_ballot_w64(true);
-  while (pending) {
-    const int lf = __builtin_amdgcn_readlane(b.leaf, __builtin_ctzll(pending));
-    const bool mine = b.leaf == lf;
-    pending &= ~__builtin_amdgcn_ballot_w64(mine);
 #pragma unroll 1
-    for (int c = 0; c < ncomp; ++c) {
-      const double wc = mine ? weight(c) : 0.0;
-      double *g = G + ((size_t)lf * ncomp + c) * NC;
-#pragma unroll
-      for (int m0 = 0; m0 < NC; m0 += CH) {
-        double buf[CH];
-#pragma unroll
-        for (int r = 0; r < CH; ++r) {
-          const int m = m0 + r;
-          buf[r] = m < NC ? wc * b.tz[kTri.i[m < NC ? m : 0]] * b.ty[kTri.j[m < NC ? m : 0]] *
-                                b.tx[kTri.k[m < NC ? m : 0]]
-                          : 0.0;
-        }
-        const double s = wave_reduce_scatter(buf);
-        if (writer && m0 + slot < NC) atomicAdd(g + m0 + slot, s);
+  for (int p0 = (int)(threadIdx.x & ~63u); p0 < count; p0 += BLOCK) {
+    const int src = s.r.order[p0 + lane < count ? p0 + lane : count - 1] & kPlaceMask;
+    const int leaf = s.r.leaf[src];
+    const double ex = s.r.e[0][src], ey = s.r.e[1][src], ez = s.r.e[2][src];
+    const bool in = fabs(ex) <= 1.0 && fabs(ey) <= 1.0 && fabs(ez) <= 1.0;
+    double px[D], dx[D], py[D], dy[D];
+    cheb_poly_d(in ? ex : 0.0, px, dx);
+    cheb_poly_d(in ? ey : 0.0, py, dy);
+    const double z = in ? ez : 0.0;
+    double jx = 0.0, jy = 0.0, jz = 0.0;
+    uint64_t pending = __builtin_amdgcn_ballot_w64(true);
+#pragma unroll 1
+    while (pending) {
+      const int lf = row_leaf(pending, leaf);
+      const bool mine = leaf == lf;
+      pending &= ~__builtin_amdgcn_ballot_w64(mine);
+      const double *cb = t.coeff + ((size_t)lf * t.dof + c0) * NC + (lane & 15);
+#pragma unroll 1
+      for (int c = 0; c < nc; ++c) {
+        double gx, gy, gz;
+        row_grad(cb, px, dx, py, dy, z, gx, gy, gz);
+        const double a = s.w[c][src];
+        jx = mine ? __builtin_fma(a, gx, jx) : jx;
+        jy = mine ? __builtin_fma(a, gy, jy) : jy;
+        jz = mine ? __builtin_fma(a, gz, jz) : jz;
+        cb += NC;
       }
     }
+    s.g[0][src] = in ? jx : 0.0;
+    s.g[1][src] = in ? jy : 0.0;
+    s.g[2][src] = in ? jz : 0.0;
   }
 }
 
-// Chunk of the concentration kernel's scatter: 64 while the basis arrays
-// leave room for it, 32 above degree 10.
-constexpr int kConcChunk = D <= 11 ? 64 : 32;
+// Transposed interpolation: G[leaf][c0 + c][ijk] += sum over the points in
+// order[0, count) of scale w[c] T_i(z) T_j(y) T_k(x), c < NCOMP.  Per leaf it
+// is a product [rows (i, j)] x [points] . [points] x [columns (k, c)]:
+// 16 x 16 x 4 FP64 MFMAs over groups of 16 places, the sums of a leaf kept in
+// registers until the wavefront's next group is another leaf's, then added
+// to memory.  Columns are ordered k first, so that shorter rows need fewer
+// column tiles: at degree 8 and three components 16 MFMAs per 16 points.
+// (Reducing every product over the wavefront took 5 to 8 vector
+// instructions per coefficient and component: 2.2 of the velocity
+// kernel's 3.1 ms on 3.0 M points.)  The caller synchronises before and
+// after.
+template <int NCOMP, int BLOCK>
+__device__ __forceinline__ void rows_scatter(AdjLds<BLOCK> &s, double *__restrict__ G, int dof,
+                                             int c0, double scale, int count) {
+  typedef MfmaAcc<double>::V V;
+  constexpr int NT = ScatterRows::NT, NCT = scatter_cols(0, NCOMP);
+  constexpr int NACC = scatter_first(NT, NCOMP);
+  const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
+  const int g = lane >> 4, p = lane & 15;
+  double(*T)[D][16] = s.t[wave];
+  double(*sw)[16] = s.sw[wave];
+  V acc[NACC];
+  auto clear = [&]() {
+#pragma unroll
+    for (int a = 0; a < NACC; ++a) acc[a] = V{0, 0, 0, 0};
+  };
+  auto flush = [&](int leaf) {
+    static_for<NT>([&](auto tc) {
+      constexpr int t = decltype(tc)::value;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = kDevRows.i[16 * t + g + 4 * r], j = kDevRows.j[16 * t + g + 4 * r];
+#pragma unroll
+        for (int n = 0; n < scatter_cols(t, NCOMP); ++n) {
+          const int q = 16 * n + p, k = q / NCOMP, c = q % NCOMP;
+          if (i >= 0 && i + j + k < D)
+            atomicAdd(G + ((size_t)leaf * dof + c0 + c) * NC + tri_start(D, i, j) + k,
+                      acc[scatter_first(t, NCOMP) + n][r]);
+        }
+      }
+    });
+  };
+  // the lane's row per M tile (the A operand's address), padding as row 0
+  int zi[NT], yj[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int i = kDevRows.i[16 * t + p];
+    zi[t] = i < 0 ? 0 : i;
+    yj[t] = kDevRows.j[16 * t + p];
+  }
+  const int ng = count / 16, per = (ng + BLOCK / 64 - 1) / (BLOCK / 64);
+  const int g1 = (wave + 1) * per < ng ? (wave + 1) * per : ng;
+  int cur = -1;
+  clear();
+#pragma unroll 1
+  for (int grp = wave * per; grp < g1; ++grp) {
+    const int o = s.r.order[16 * grp + p], src = o & kPlaceMask;
+    const int leaf = s.r.leaf[src];
+    {
+      double v[D];
+      row_cheb<D>(s.r.e[g < 3 ? g : 2][src], v);
+      if (g < 3) {
+#pragma unroll
+        for (int k = 0; k < D; ++k) T[g][k][p] = v[k];
+      }
+    }
+    // copies that pad a leaf's places carry no weight
+    const double w = o == src && g < NCOMP ? scale * s.w[g < NCOMP ? g : 0][src] : 0.0;
+    uint64_t pending = __builtin_amdgcn_ballot_w64(true);
+#pragma unroll 1
+    while (pending) {  // one pass; per leaf in the overflow run
+      const int lf = __builtin_amdgcn_readlane(leaf, __builtin_ctzll(pending));
+      const bool mine = leaf == lf;
+      pending &= ~__builtin_amdgcn_ballot_w64(mine);
+      if (lf != cur) {
+        if (cur >= 0) {
+          flush(cur);
+          clear();
+        }
+        cur = lf;
+      }
+      if (g < NCOMP) sw[g][p] = mine ? w : 0.0;
+      wave_lds_order();
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const int pt = 4 * st + g;  // the lane's point of this K step
+        double b[NCT];
+#pragma unroll
+        for (int n = 0; n < NCT; ++n) {
+          const int q = 16 * n + p, k = q / NCOMP;
+          b[n] = sw[q % NCOMP][pt] * T[0][k < D ? k : 0][pt];
+        }
+        static_for<NT>([&](auto tc) {
+          constexpr int t = decltype(tc)::value;
+          const double a = T[2][zi[t]][pt] * T[1][yj[t]][pt];
+#pragma unroll
+          for (int n = 0; n < scatter_cols(t, NCOMP); ++n)
+            acc[scatter_first(t, NCOMP) + n] =
+                MfmaAcc<double>::mma(a, b[n], acc[scatter_first(t, NCOMP) + n]);
+        });
+      }
+      wave_lds_order();  // the scratch is written again
+    }
+  }
+  if (cur >= 0) flush(cur);
+}
 
 // Arrival point of global grid index gi (tree_utils.h:480-491).
 __device__ __forceinline__ void arrival_point(const TreeView &conc, const StepArgs &a,
@@ -236,79 +327,6 @@ __device__ __forceinline__ void arrival_point(const TreeView &conc, const StepAr
   x = (double)inf.x * len + len * a.node[m % D];
   y = (double)inf.y * len + len * a.node[(m / D) % D];
   z = (double)inf.z * len + len * a.node[m / (D * D)];
-}
-
-// Cotangent of c and, when A is given, the per-point velocity cotangent
-// factor a_p += sum_c u_{p,c} grad c_c(D_p).  ua[al][c][am] = (R^T lam')
-// at arrival point (al, am).  MODE is the forward's trajectory arithmetic;
-// with STORED the departure points are read from dep[3 gi] (the forward
-// step's own output, wrapped as the concentration saw them) instead of
-// being integrated again.
-template <int MODE, int BLOCK, bool STORED>
-__global__ __launch_bounds__(BLOCK) void k_adj_conc(VelSource vel, TreeView conc, StepArgs a,
-                                                    const double *__restrict__ dep,
-                                                    const double *__restrict__ ua,
-                                                    double *__restrict__ lam,
-                                                    double *__restrict__ A) {
-  __shared__ RegroupLds<BLOCK, 3> sh;
-  const uint32_t b = blockIdx.x;
-  const int64_t lb = (int64_t)(b & 7u) * a.per_xcd + (int64_t)(b >> 3);
-  if (lb >= a.nblocks) return;  // uniform over the workgroup
-  const int64_t i0 = lb * BLOCK;
-  int orig = (int)threadIdx.x;
-  double p3[3];
-  {
-    const int64_t i = i0 + orig < a.npts ? i0 + orig : a.npts - 1;
-    if constexpr (STORED) {
-      p3[0] = dep[3 * i + 0];
-      p3[1] = dep[3 * i + 1];
-      p3[2] = dep[3 * i + 2];
-    } else {
-      double x, y, z;
-      arrival_point(conc, a, i, x, y, z);
-#pragma unroll 1
-      for (int s = 0; s < a.nsub; ++s)
-        rk2_substep<D, MODE, kVelTree>(vel, a.bc, a.htau, a.tau, a.scaled, a.g[2 * s],
-                                       a.g[2 * s + 1], a.ts[2 * s], a.ts[2 * s + 1], x, y, z);
-      if (a.bc == TBX_BC_PERIODIC) {
-        x = wrap1(x);
-        y = wrap1(y);
-        z = wrap1(z);
-      }
-      p3[0] = x;
-      p3[1] = y;
-      p3[2] = z;
-    }
-  }
-  int lf = locate(conc, p3[0], p3[1], p3[2]);
-  regroup(sh, orig, lf, p3);
-  const int64_t gi = i0 + orig;
-  const bool live = gi < a.npts;
-  const int64_t al = live ? gi / a.P : 0;
-  const int am = live ? (int)(gi - al * a.P) : 0;
-  const int dof = conc.dof;
-  AdjBasis bs;
-  bs.build(conc, p3[0], p3[1], p3[2], lf);
-  auto weight = [&](int c) { return live ? ua[(al * dof + c) * a.P + am] : 0.0; };
-  if (A) {
-    double ax = 0.0, ay = 0.0, az = 0.0;
-    for_each_wave_leaf(bs.leaf, [&](int leaf) {
-      for (int c = 0; c < dof; ++c) {
-        double gx, gy, gz;
-        grad3(conc.coeff + ((size_t)leaf * dof + c) * NC, bs, gx, gy, gz);
-        const double u = weight(c);
-        ax = __builtin_fma(u, gx, ax);
-        ay = __builtin_fma(u, gy, ay);
-        az = __builtin_fma(u, gz, az);
-      }
-    });
-    if (live) {
-      A[3 * gi + 0] += ax;
-      A[3 * gi + 1] += ay;
-      A[3 * gi + 2] += az;
-    }
-  }
-  scatter_transposed<kConcChunk>(lam, dof, bs, weight);
 }
 
 // The first-stage velocity at arrival point i (its wrapped position x, y,
@@ -325,9 +343,123 @@ __device__ __forceinline__ bool adj_nodal_stage1(const VelSource &vel, const Tre
                            (int)(i - jl * a.P), lf, a.P, a.scaled, a.g[0], v0, v1, v2);
 }
 
-// Waves per SIMD asked of the velocity kernel: two fit without spills up
-// to degree 8 (the register budget halves to 256).
-constexpr int kVelWaves = D <= 9 ? 2 : 1;
+__device__ __forceinline__ void wrap3(const StepArgs &a, double &x, double &y, double &z) {
+  if (a.bc == TBX_BC_PERIODIC) {
+    x = wrap1(x);
+    y = wrap1(y);
+    z = wrap1(z);
+  }
+}
+
+// Velocity of stage `stage` of substep s at the needing threads' points.
+template <int MODE, int BLOCK>
+__device__ __forceinline__ void adj_velocity(RowsLds<BLOCK> &sh, const VelSource &vel,
+                                             const StepArgs &a, int stage, int s, bool need,
+                                             double &x, double &y, double &z, double (&v)[3]) {
+  const int k = 2 * s + stage - 1;
+  if constexpr (MODE == kExact64) {
+    eval_velocity<D, MODE, kVelTree>(vel, stage, a.ts[k], a.scaled, a.g[k], a.bc, x, y, z, v[0],
+                                     v[1], v[2]);
+  } else {
+    const int lf = locate(vel.t[0], x, y, z);
+    const int count = order_by_leaf(sh, need, lf);
+    rows_velocity<D, MODE, kVelTree>(sh, vel, stage, a.ts[k], a.scaled, a.g[k], a.bc, count, lf,
+                                     x, y, z, v);
+  }
+}
+
+// The first stage of substep s at (x, y, z) as the forward step takes it:
+// the nodal value of arrival point i where it has one (a.vnode).
+template <int MODE, int BLOCK>
+__device__ __forceinline__ void adj_stage1(RowsLds<BLOCK> &sh, const VelSource &vel,
+                                           const TreeView &conc, const StepArgs &a, int64_t i,
+                                           bool live, int s, double &x, double &y, double &z,
+                                           double (&v)[3]) {
+  bool need = live;
+  v[0] = v[1] = v[2] = 0.0;
+  if (s == 0 && a.vnode)
+    need = live && !adj_nodal_stage1(vel, conc, a, i, x, y, z, v[0], v[1], v[2]);
+  if (__syncthreads_or(need)) {
+    double u[3];
+    adj_velocity<MODE>(sh, vel, a, 1, s, need, x, y, z, u);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[c] = need ? u[c] : v[c];
+  }
+}
+
+// Substep s of the forward step for a workgroup's points, in place.
+template <int MODE, int BLOCK>
+__device__ __forceinline__ void adj_substep(RowsLds<BLOCK> &sh, const VelSource &vel,
+                                            const TreeView &conc, const StepArgs &a, int64_t i,
+                                            bool live, int s, double &x, double &y, double &z) {
+  wrap3(a, x, y, z);
+  double v[3];
+  adj_stage1<MODE>(sh, vel, conc, a, i, live, s, x, y, z, v);
+  double hx = x + a.htau * v[0], hy = y + a.htau * v[1], hz = z + a.htau * v[2];
+  wrap3(a, hx, hy, hz);
+  adj_velocity<MODE>(sh, vel, a, 2, s, live, hx, hy, hz, v);
+  x = x + a.tau * v[0];
+  y = y + a.tau * v[1];
+  z = z + a.tau * v[2];
+}
+
+// Cotangent of c and, when A is given, the per-point velocity cotangent
+// factor a_p += sum_c u_{p,c} grad c_c(D_p).  ua[al][c][am] = (R^T lam')
+// at arrival point (al, am).  MODE is the forward's trajectory arithmetic;
+// with STORED the departure points are read from dep[3 gi] (the forward
+// step's own output, wrapped as the concentration saw them) instead of
+// being integrated again.
+template <int MODE, int BLOCK, bool STORED>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_conc(
+    VelSource vel, TreeView conc, StepArgs a, const double *__restrict__ dep,
+    const double *__restrict__ ua, double *__restrict__ lam, double *__restrict__ A) {
+  __shared__ AdjLds<BLOCK> sh;
+  const uint32_t b = blockIdx.x;
+  const int64_t lb = (int64_t)(b & 7u) * a.per_xcd + (int64_t)(b >> 3);
+  if (lb >= a.nblocks) return;  // uniform over the workgroup
+  const int tid = (int)threadIdx.x;
+  const int64_t i0 = lb * BLOCK;
+  const bool live = i0 + tid < a.npts;
+  const int64_t i = live ? i0 + tid : a.npts - 1;
+  double x, y, z;
+  if constexpr (STORED) {
+    x = dep[3 * i + 0];
+    y = dep[3 * i + 1];
+    z = dep[3 * i + 2];
+  } else {
+    arrival_point(conc, a, i, x, y, z);
+#pragma unroll 1
+    for (int s = 0; s < a.nsub; ++s)
+      adj_substep<MODE>(sh.r, vel, conc, a, i, live, s, x, y, z);
+    wrap3(a, x, y, z);
+  }
+  const int lf = locate(conc, x, y, z);
+  const int count = order_by_leaf(sh.r, live, lf);
+  put_point(sh.r, conc, lf, x, y, z);
+  const int64_t al = i / a.P;
+  const int am = (int)(i - al * a.P);
+  const int dof = conc.dof;
+  double ax = 0.0, ay = 0.0, az = 0.0;
+#pragma unroll 1
+  for (int c = 0; c < dof; ++c) {
+    sh.w[0][tid] = ua[(al * dof + c) * a.P + am];
+    __syncthreads();
+    if (A) rows_gradient(sh, conc, c, 1, count);
+    rows_scatter<1>(sh, lam, dof, c, 1.0, count);
+    __syncthreads();
+    if (A) {
+      ax += sh.g[0][tid];
+      ay += sh.g[1][tid];
+      az += sh.g[2][tid];
+    }
+  }
+  if (A && live) {
+    const double s2 = 2.0 * (double)(1u << conc.info[lf].w);  // d xi / dx
+    A[3 * i + 0] += s2 * ax;
+    A[3 * i + 1] += s2 * ay;
+    A[3 * i + 2] += s2 * az;
+  }
+}
 
 // Velocity cotangent through the num_rk_step substeps.  Substep s maps x_s
 // to x_{s+1} = x_s + tau g2_s V(h_s), h_s = x_s + (tau/2) g1_s V(x_s)
@@ -338,149 +470,84 @@ constexpr int kVelWaves = D <= 9 ? 2 : 1;
 //   a_s = a_{s+1} + tau g2_s J_V(h_s)^T a_{s+1} + J_V(x_s)^T w_s,
 // each dV scattered into G[leaf][k][m] at its point (in its leaf).  The
 // substeps run backwards; x_s is integrated again from the arrival point
-// (s substeps) for each one.  Before the work at h_s and again before the
-// work at x_s the workgroup's points are regrouped by the leaf they fall in
-// (as in the concentration kernel), carrying their state along, so a
-// wavefront's scatter reads and adds one leaf's coefficients at a time.
+// (s substeps) for each one.  A thread keeps its arrival point; the work at
+// h_s and at x_s goes through the workgroup's order by leaf.
 template <int MODE>
-__global__ __launch_bounds__(kAdjBlock, kVelWaves) void k_adj_vel(VelSource vel, TreeView conc,
-                                                                  StepArgs a,
-                                                                  const double *__restrict__ A,
-                                                                  double *__restrict__ G) {
-  __shared__ RegroupLds<kAdjBlock, 12> sh;
+__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_vel(
+    VelSource vel, TreeView conc, StepArgs a, const double *__restrict__ A,
+    double *__restrict__ G) {
+  __shared__ AdjLds<kAdjBlock> sh;
   const uint32_t b = blockIdx.x;
   const int64_t lb = (int64_t)(b & 7u) * a.per_xcd + (int64_t)(b >> 3);
   if (lb >= a.nblocks) return;  // uniform over the workgroup
-  const int64_t i0 = lb * kAdjBlock;
   const TreeView &V = vel.t[0];
-  int orig = (int)threadIdx.x;
-  double ax, ay, az;
-  {
-    const int64_t gi = i0 + orig;
-    const bool live = gi < a.npts;
-    ax = live ? A[3 * gi + 0] : 0.0;  // idle lanes carry zero weights
-    ay = live ? A[3 * gi + 1] : 0.0;
-    az = live ? A[3 * gi + 2] : 0.0;
-  }
+  const int tid = (int)threadIdx.x;
+  const int64_t i0 = lb * kAdjBlock;
+  const bool live = i0 + tid < a.npts;
+  const int64_t i = live ? i0 + tid : a.npts - 1;
+  double ax = A[3 * i + 0], ay = A[3 * i + 1], az = A[3 * i + 2];
 #pragma unroll 1
   for (int s = a.nsub - 1; s >= 0; --s) {
-    const int64_t i = i0 + orig < a.npts ? i0 + orig : a.npts - 1;
     double x, y, z;
     arrival_point(conc, a, i, x, y, z);
 #pragma unroll 1
-    for (int r = 0; r < s; ++r) {
-      double w0, w1, w2;
-      if (r == 0 && a.vnode) {  // the forward's first stage from the nodal values
-        if (a.bc == TBX_BC_PERIODIC) {
-          x = wrap1(x);
-          y = wrap1(y);
-          z = wrap1(z);
-        }
-        if (!adj_nodal_stage1(vel, conc, a, i, x, y, z, w0, w1, w2))
-          eval_velocity<D, MODE, kVelTree>(vel, 1, a.ts[0], a.scaled, a.g[0], a.bc, x, y, z, w0,
-                                           w1, w2);
-        rk2_finish<D, MODE, kVelTree>(vel, a.bc, a.htau, a.tau, a.scaled, a.g[1], a.ts[1], x, y,
-                                      z, w0, w1, w2);
-      } else {
-        rk2_substep<D, MODE, kVelTree>(vel, a.bc, a.htau, a.tau, a.scaled, a.g[2 * r],
-                                       a.g[2 * r + 1], a.ts[2 * r], a.ts[2 * r + 1], x, y, z);
-      }
-    }
-    if (a.bc == TBX_BC_PERIODIC) {
-      x = wrap1(x);
-      y = wrap1(y);
-      z = wrap1(z);
-    }
+    for (int r = 0; r < s; ++r) adj_substep<MODE>(sh.r, vel, conc, a, i, live, r, x, y, z);
+    wrap3(a, x, y, z);
     // the forward's midpoint of substep s (rk2_substep, stage 1)
-    double v0, v1, v2;
-    double xs = x, ys = y, zs = z;
-    if (s != 0 || !adj_nodal_stage1(vel, conc, a, i, x, y, z, v0, v1, v2))
-      eval_velocity<D, MODE, kVelTree>(vel, 1, a.ts[2 * s], a.scaled, a.g[2 * s], a.bc, xs, ys,
-                                       zs, v0, v1, v2);
-    double hx = x + a.htau * v0, hy = y + a.htau * v1, hz = z + a.htau * v2;
-    if (a.bc == TBX_BC_PERIODIC) {
-      hx = wrap1(hx);
-      hy = wrap1(hy);
-      hz = wrap1(hz);
-    }
+    double v[3];
+    adj_stage1<MODE>(sh.r, vel, conc, a, i, live, s, x, y, z, v);
+    double hx = x + a.htau * v[0], hy = y + a.htau * v[1], hz = z + a.htau * v[2];
+    wrap3(a, hx, hy, hz);
     const double g1 = a.scaled ? a.g[2 * s] : 1.0, g2 = a.scaled ? a.g[2 * s + 1] : 1.0;
     const double fh = a.tau * g2, fx = a.tau * g2 * a.htau * g1;
-    // work at h: regroup by h's leaf
-    int lh = locate(V, hx, hy, hz);
-    double ph[9] = {hx, hy, hz, ax, ay, az, x, y, z};
-    regroup(sh, orig, lh, ph);
-    ax = ph[3];
-    ay = ph[4];
-    az = ph[5];
-    double jx = 0.0, jy = 0.0, jz = 0.0;
-    {
-      AdjBasis bh;
-      bh.build(V, ph[0], ph[1], ph[2], lh);
-      // J^T a at h: (J^T a)_k = sum_c a_c dV_c/dy_k
-      for_each_wave_leaf(bh.leaf, [&](int leaf) {
-#pragma unroll 1
-        for (int c = 0; c < 3; ++c) {
-          double gx, gy, gz;
-          grad3(V.coeff + ((size_t)leaf * 3 + c) * NC, bh, gx, gy, gz);
-          const double ac = c == 0 ? ax : c == 1 ? ay : az;
-          jx = __builtin_fma(ac, gx, jx);
-          jy = __builtin_fma(ac, gy, jy);
-          jz = __builtin_fma(ac, gz, jz);
-        }
-      });
-      scatter_transposed<32>(G, 3, bh, [&](int c) {
-        return fh * (c == 0 ? ax : c == 1 ? ay : az);
-      });
-    }
-    // work at x: regroup by x's leaf
-    int lx = locate(V, ph[6], ph[7], ph[8]);
-    double px[12] = {ph[6], ph[7], ph[8], fx * jx, fx * jy, fx * jz, ax, ay, az, jx, jy, jz};
+    // work at h: J^T a, (J^T a)_k = sum_c a_c dV_c/dy_k, and fh a scattered
+    const int lh = locate(V, hx, hy, hz);
+    int count = order_by_leaf(sh.r, live, lh);
+    put_point(sh.r, V, lh, hx, hy, hz);
+    sh.w[0][tid] = ax;
+    sh.w[1][tid] = ay;
+    sh.w[2][tid] = az;
+    __syncthreads();
+    rows_gradient(sh, V, 0, 3, count);
+    rows_scatter<3>(sh, G, 3, 0, fh, count);
+    __syncthreads();
+    const double sh2 = 2.0 * (double)(1u << V.info[lh].w);  // d xi / dx
+    const double jx = sh2 * sh.g[0][tid], jy = sh2 * sh.g[1][tid], jz = sh2 * sh.g[2][tid];
+    const double wx = fx * jx, wy = fx * jy, wz = fx * jz;
+    // work at x
+    const int lx = locate(V, x, y, z);
+    bool rest = live;
     if (s == 0 && a.wnode) {
       // x is the point's arrival node: where that is a grid node of its
       // velocity leaf, its weights go to the node's slot (the slots are then
       // projected, G += B^T slots, in one pass per leaf); only the others
-      // scatter, and only workgroups holding one regroup
-      const int64_t gi = i0 + orig;
-      bool rest = false;
-      if (gi < a.npts) {
-        const int64_t jl = gi / a.P;
-        const int mm = node_of(conc.info[jl], V.info[lx], (int)(gi - jl * a.P), D);
-        if (mm >= 0) {
-          double *wn = a.wnode + (int64_t)lx * 3 * a.P + mm;
-          atomicAdd(wn, px[3]);
-          atomicAdd(wn + a.P, px[4]);
-          atomicAdd(wn + 2 * a.P, px[5]);
-          px[3] = 0.0;
-          px[4] = 0.0;
-          px[5] = 0.0;
-        } else {
-          rest = true;
-        }
+      // scatter, and only workgroups holding one
+      const int64_t jl = i / a.P;
+      const int mm = live ? node_of(conc.info[jl], V.info[lx], (int)(i - jl * a.P), D) : -1;
+      if (mm >= 0) {
+        double *wn = a.wnode + (int64_t)lx * 3 * a.P + mm;
+        atomicAdd(wn, wx);
+        atomicAdd(wn + a.P, wy);
+        atomicAdd(wn + 2 * a.P, wz);
+        rest = false;
       }
       if (!__syncthreads_or(rest)) continue;  // s == 0: the last substep
     }
-    regroup(sh, orig, lx, px);
-    const double wx = px[3], wy = px[4], wz = px[5];
-    AdjBasis bx;
-    bx.build(V, px[0], px[1], px[2], lx);
-    scatter_transposed<32>(G, 3, bx, [&](int c) { return c == 0 ? wx : c == 1 ? wy : wz; });
+    count = order_by_leaf(sh.r, rest, lx);
+    put_point(sh.r, V, lx, x, y, z);
+    sh.w[0][tid] = wx;
+    sh.w[1][tid] = wy;
+    sh.w[2][tid] = wz;
+    __syncthreads();
+    if (s > 0) rows_gradient(sh, V, 0, 3, count);
+    rows_scatter<3>(sh, G, 3, 0, 1.0, count);
+    __syncthreads();
     if (s > 0) {
       // a_s = a_{s+1} + tau g2 J(h)^T a_{s+1} + J(x)^T w
-      double kx = 0.0, ky = 0.0, kz = 0.0;
-      for_each_wave_leaf(bx.leaf, [&](int leaf) {
-#pragma unroll 1
-        for (int c = 0; c < 3; ++c) {
-          double gx, gy, gz;
-          grad3(V.coeff + ((size_t)leaf * 3 + c) * NC, bx, gx, gy, gz);
-          const double wc = c == 0 ? wx : c == 1 ? wy : wz;
-          kx = __builtin_fma(wc, gx, kx);
-          ky = __builtin_fma(wc, gy, ky);
-          kz = __builtin_fma(wc, gz, kz);
-        }
-      });
-      ax = px[6] + fh * px[9] + kx;
-      ay = px[7] + fh * px[10] + ky;
-      az = px[8] + fh * px[11] + kz;
+      const double sx2 = 2.0 * (double)(1u << V.info[lx].w);
+      ax = ax + fh * jx + sx2 * sh.g[0][tid];
+      ay = ay + fh * jy + sx2 * sh.g[1][tid];
+      az = az + fh * jz + sx2 * sh.g[2][tid];
     }
   }
 }

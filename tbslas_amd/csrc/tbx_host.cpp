@@ -1380,6 +1380,12 @@ int adj_conc_step(const AdjCtx &c, tbx_tree *conc, int timestep, double dt, int 
   StepArgs a;
   int rc = adj_args(c, conc, timestep, dt, bc, kAdjBlock, &a);
   if (rc) return rc;
+  // integrated again, the trajectories are the forward step's: its first
+  // stage too takes the nodal values
+  if (!dep && uses_node_velocity(TBX_VEL_TREE, c.mode) &&
+      (rc = node_velocity(const_cast<tbx_tree *>(c.v.trees[0]), c.mode, st, nullptr, &a.vnode,
+                          "adjoint")))
+    return rc;
   HIP_TRY(dispatch_adj_conc(conc->q, c.mode, c.vs, conc->view(), a, dep, conc->d_vals, lam_out,
                             A, st));
   return TBX_OK;

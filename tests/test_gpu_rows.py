@@ -124,3 +124,36 @@ def test_evaluation_under_capture(tb):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("q", [1, 3, 8, 10, 13, 16])
+@pytest.mark.parametrize("bc", [0, 1])
+def test_adjoint_dot_product_across_degrees(tb, q, bc):
+    # <lam, F(c)> = <F^T lam, c> and, along a velocity perturbation that is
+    # one polynomial, the derivative's dot product: the transposed
+    # interpolation's tiles change with the degree.  1e-12 of |lam| |F(c)|
+    # (sums of some 1e4 to 1e6 products in FP64).
+    import torch
+
+    from tbslas_amd import fields
+    from tbslas_amd.adjoint import semilag_insitu_vjp
+
+    anchor, depth = random_tree(11, max_depth=2)
+    vcf = tb.fit_function(fields.taylor_green_2d3, anchor, depth, q, 3)
+    vel, conc = tb.Tree(anchor, depth, q, 3, vcf), tb.Tree(anchor, depth, q, 2)
+    g = torch.Generator(device="cuda").manual_seed(q)
+    c, lam = (torch.randn((len(depth), 2, tb.ncoef(q)), dtype=torch.float64, device="cuda",
+                          generator=g) for _ in range(2))
+    conc.set_coeffs(c)
+    grad = torch.zeros((len(depth), 3, tb.ncoef(q)), dtype=torch.float64, device="cuda")
+    back = semilag_insitu_vjp(vel, conc, 1, 0.05, lam, bc, grad_vel=grad)
+    dep = torch.empty((conc.L * conc.P, 3), dtype=torch.float64, device="cuda")
+    tb.semilag_insitu(vel, conc, 1, 0.05, 1, bc, dep=dep)
+    out = conc.get_coeffs_device()
+    assert abs(float((lam * out).sum() - (back * c).sum())) <= 1e-12 * float(lam.norm() * out.norm())
+    conc.set_coeffs(c)
+    stored = semilag_insitu_vjp(vel, conc, 1, 0.05, lam, bc, dep=dep)
+    assert float((stored - back).abs().max()) <= 1e-12 * float(back.abs().max())
+    # the velocity cotangent is the sum over substeps: one step's against two
+    # half steps' chain is covered elsewhere; here that it is finite and moves
+    assert bool(torch.isfinite(grad).all()) and float(grad.abs().max()) > 0
