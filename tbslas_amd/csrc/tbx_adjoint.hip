@@ -166,7 +166,19 @@ struct AdjLds {
   double g[3][BLOCK];
   double t[BLOCK / 64][3][D][16];  // T_k of a group's 16 points per axis
   double sw[BLOCK / 64][3][16];    // their weights
+  int rows[16 * ScatterRows::NT];  // per tile row: start | values of k << 10 | i << 15 | j << 20
 };
+
+// The tile rows' table, read through LDS (from global memory its loads'
+// latency stood before every sum that left the registers: the concentration
+// kernel 820 us).  The caller synchronises before its use.
+template <int BLOCK>
+__device__ __forceinline__ void scatter_table(AdjLds<BLOCK> &s) {
+  for (int r = (int)threadIdx.x; r < 16 * ScatterRows::NT; r += BLOCK) {
+    const int i = kDevRows.i[r], j = kDevRows.j[r];
+    s.rows[r] = i < 0 ? 0 : tri_start(D, i, j) | ((D - i - j) << 10) | (i << 15) | (j << 20);
+  }
+}
 
 // s.g = sum over c < nc of w[c] grad_xi(component c of t) at the points in
 // order[0, count) (zero outside the leaf's box, as the basis).  The caller
@@ -241,24 +253,23 @@ __device__ __forceinline__ void rows_scatter(AdjLds<BLOCK> &s, double *__restric
       constexpr int t = decltype(tc)::value;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = kDevRows.i[16 * t + g + 4 * r], j = kDevRows.j[16 * t + g + 4 * r];
+        const int row = s.rows[16 * t + g + 4 * r];
 #pragma unroll
         for (int n = 0; n < scatter_cols(t, NCOMP); ++n) {
           const int q = 16 * n + p, k = q / NCOMP, c = q % NCOMP;
-          if (i >= 0 && i + j + k < D)
-            atomicAdd(G + ((size_t)leaf * dof + c0 + c) * NC + tri_start(D, i, j) + k,
+          if (k < ((row >> 10) & 31))
+            atomicAdd(G + ((size_t)leaf * dof + c0 + c) * NC + (row & 1023) + k,
                       acc[scatter_first(t, NCOMP) + n][r]);
         }
       }
     });
   };
-  // the lane's row per M tile (the A operand's address), padding as row 0
+  // the lane's row per M tile (the A operand's address)
   int zi[NT], yj[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int i = kDevRows.i[16 * t + p];
-    zi[t] = i < 0 ? 0 : i;
-    yj[t] = kDevRows.j[16 * t + p];
+    zi[t] = (s.rows[16 * t + p] >> 15) & 31;
+    yj[t] = s.rows[16 * t + p] >> 20;
   }
   const int ng = count / 16, per = (ng + BLOCK / 64 - 1) / (BLOCK / 64);
   const int g1 = (wave + 1) * per < ng ? (wave + 1) * per : ng;
@@ -417,6 +428,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void
   const uint32_t b = blockIdx.x;
   const int64_t lb = (int64_t)(b & 7u) * a.per_xcd + (int64_t)(b >> 3);
   if (lb >= a.nblocks) return;  // uniform over the workgroup
+  scatter_table(sh);
   const int tid = (int)threadIdx.x;
   const int64_t i0 = lb * BLOCK;
   const bool live = i0 + tid < a.npts;
@@ -480,6 +492,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2))) 
   const uint32_t b = blockIdx.x;
   const int64_t lb = (int64_t)(b & 7u) * a.per_xcd + (int64_t)(b >> 3);
   if (lb >= a.nblocks) return;  // uniform over the workgroup
+  scatter_table(sh);
   const TreeView &V = vel.t[0];
   const int tid = (int)threadIdx.x;
   const int64_t i0 = lb * kAdjBlock;
