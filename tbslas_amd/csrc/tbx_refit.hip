@@ -23,7 +23,7 @@
 // B[k][j] in lane j + 16 k, D[i][j] in lane j + 16 (i % 4), register i / 4.
 #include <hip/hip_runtime.h>
 
-#include "tbx_internal.h"
+#include "tbx_rows.h"
 
 namespace tbx {
 namespace {
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_refit_gemm(
 
 // Packed index of term (i, j, k) of the triangle i -> j -> k, i+j+k < D.
 template <int D>
-__device__ __forceinline__ int tri_index(int i, int j, int k) {
+__device__ __forceinline__ int packed_index(int i, int j, int k) {
   // terms before block i: sum_{a<i} (D-a)(D-a+1)/2; before row j of block
   // i: sum_{b<j} (D-i-b)
   const int n = D - i;
@@ -268,9 +268,9 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_project(const double *_
 #pragma unroll
           for (int c = 0; c < D; ++c) s = __builtin_fma(tab.T[i][c], x[c], s);
           if constexpr (ACC)
-            w[tri_index<D>(i, j, k)] += s;
+            w[packed_index<D>(i, j, k)] += s;
           else
-            w[tri_index<D>(i, j, k)] = s;
+            w[packed_index<D>(i, j, k)] = s;
         }
       }
       if constexpr (!ACC)
@@ -283,10 +283,17 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_project(const double *_
 // The transpose: v = B u per row (u rows of stride KP in packed order), the
 // row's polynomial at the D^3 grid nodes, v[c][b][a] (x fastest), by the
 // three one-axis contractions z, y, x through LDS.  TO: the output precision
-// (FP32 for the FP32 modes' nodal velocities).  (A variant contracting x
-// first over the triangle, with y and z in registers, does a third fewer
-// multiply-adds but ran 1.3x slower: its scalar-operand and register loads
-// cost more than the LDS reads they replace.)
+// (FP32 for the FP32 modes' nodal velocities).
+//
+// A line's D outputs are sums over its D inputs with the one-axis table's
+// entries as the other factor.  The table sits in registers, row i across
+// the 16 lanes of each DPP row, and v_fmac broadcasts the entry it needs
+// (row_outer) in place of one LDS read per multiply-add: 108,972 rows of
+// degree 14 1.42 -> 1.00 ms, 4,096 x 3 rows of degree 10 143 -> 73 us, of
+// degree 8 62 -> 42 us.  At degree 16 the 17 entries do not fit a row's
+// lanes; its table stays in LDS.  (A variant
+// contracting x first over the triangle, with y and z in registers, does a
+// third fewer multiply-adds but ran 1.3x slower than the LDS form.)
 template <int D, typename TO>
 __global__ __launch_bounds__(kRefitThreads) void k_refit_expand(const double *__restrict__ U,
                                                                 int64_t rows, RefitTable tab,
@@ -294,6 +301,7 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_expand(const double *__
   constexpr int P = D * D * D;
   constexpr int R = refit_rows<D>();
   constexpr int TS = R > 1 ? D * D : kRefitThreads;  // threads of a row's team
+  constexpr bool kDpp = D <= 16;
   __shared__ double sa[R * P];
   __shared__ double sb[R * P];
   __shared__ double sT[D * D];
@@ -303,82 +311,92 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_expand(const double *__
   const bool team = tid < R * TS;
   double *ra = sa + rl * P, *rb = sb + rl * P;
   for (int t = tid; t < D * D; t += kRefitThreads) sT[t] = tab.T[t / D][t % D];
+  __syncthreads();
+  double tr[kDpp ? D : 1];  // row i of the table, entry lane % 16
+  if constexpr (kDpp) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) tr[i] = sT[i * D + ((tid & 15) < D ? (tid & 15) : 0)];
+  }
+  // out[c] = sum_i T[i][c] x[i]; every lane takes part (its table entries
+  // are read by its neighbours)
+  auto line = [&](const double (&x)[D], double (&out)[D]) {
+#pragma unroll
+    for (int c = 0; c < D; ++c) out[c] = 0.0;
+    if constexpr (kDpp) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) row_outer<0, D>(out, tr[i], x[i]);
+    } else {
+#pragma unroll 1
+      for (int c = 0; c < D; ++c) {
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < D; ++i) s = __builtin_fma(sT[i * D + c], x[i], s);
+#pragma unroll
+        for (int e = 0; e < D; ++e) out[e] = e == c ? s : out[e];
+      }
+    }
+  };
   // the first (j, k) line of the thread's next row loaded during the
   // current row's LDS stages, as in k_refit_project
   const int64_t stride = (int64_t)gridDim.x * R;
-  double xn[D];
-  auto fetch = [&](int64_t r) {
-    const int j = tl / D, k = tl % D;
-    if (refit_prefetch<D>() && team && tl < D * D && j + k < D && r < rows) {
-      const double *u = U + r * KP;
-      const int ni = D - j - k;
+  auto inputs = [&](int64_t r, int t, double (&x)[D]) {
+    const int j = t / D, k = t % D;
+    const bool in = team && t < D * D && j + k < D && r < rows;
+    const double *u = U + (in ? r : 0) * KP;
+    const int ni = in ? D - j - k : 0;
 #pragma unroll
-      for (int i = 0; i < D; ++i) xn[i] = i < ni ? u[tri_index<D>(i, j, k)] : 0.0;
-    }
+    for (int i = 0; i < D; ++i) x[i] = i < ni ? u[tri_start(D, i, j) + k] : 0.0;
   };
-  fetch((int64_t)blockIdx.x * R + rl);
-  __syncthreads();
+  double xn[D];
+  if constexpr (refit_prefetch<D>()) inputs((int64_t)blockIdx.x * R + rl, tl, xn);
   for (int64_t r0 = (int64_t)blockIdx.x * R; r0 < rows; r0 += stride) {
     const int64_t r = r0 + rl;
     const bool act = team && r < rows;
-    if (act) {
-      const double *u = U + r * KP;
-      for (int t = tl; t < D * D; t += TS) {  // t = j * D + k
-        const int j = t / D, k = t % D;
-        if (j + k >= D) continue;
-        double x[D];
-        const int ni = D - j - k;
-        if (refit_prefetch<D>() && t == tl) {
-#pragma unroll
-          for (int i = 0; i < D; ++i) x[i] = xn[i];
-        } else {
-#pragma unroll
-          for (int i = 0; i < D; ++i) x[i] = i < ni ? u[tri_index<D>(i, j, k)] : 0.0;
-        }
-        for (int c = 0; c < D; ++c) {
-          double s = 0.0;
-#pragma unroll
-          for (int i = 0; i < D; ++i) s = __builtin_fma(sT[i * D + c], x[i], s);
-          rb[(c * D + j) * D + k] = s;
-        }
-      }
-    }
-    fetch(r + stride);
-    __syncthreads();
-    if (act) {
-      for (int t = tl; t < D * D; t += TS) {  // t = c * D + k
-        const int c = t / D, k = t % D;
-        double x[D];
-#pragma unroll
-        for (int j = 0; j < D; ++j) x[j] = j + k < D ? rb[(c * D + j) * D + k] : 0.0;
-        for (int b = 0; b < D; ++b) {
-          double s = 0.0;
-#pragma unroll
-          for (int j = 0; j < D; ++j) s = __builtin_fma(sT[j * D + b], x[j], s);
-          ra[(c * D + b) * D + k] = s;
-        }
-      }
-    }
-    __syncthreads();
-    if (act) {
-      TO *v = V + r * P;
-      for (int t = tl; t < D * D; t += TS) {  // t = c * D + b
-        double x[D];
-#pragma unroll
-        for (int k = 0; k < D; ++k) x[k] = ra[t * D + k];
-        auto out = [&](int a) {
-          double s = 0.0;
-#pragma unroll
-          for (int k = 0; k < D; ++k) s = __builtin_fma(sT[k * D + a], x[k], s);
-          v[t * D + a] = (TO)s;
-        };
-        if constexpr (R > 1) {  // as in k_refit_project
+    // lines past the last are computed and dropped
+    constexpr int kLines = (D * D + TS - 1) / TS;
 #pragma unroll 1
-          for (int a = 0; a < D; ++a) out(a);
-        } else {
+    for (int n = 0; n < kLines; ++n) {
+      const int t = tl + n * TS, j = t / D, k = t % D;  // t = j * D + k
+      double x[D], o[D];
+      if (refit_prefetch<D>()) {
 #pragma unroll
-          for (int a = 0; a < D; ++a) out(a);
-        }
+        for (int i = 0; i < D; ++i) x[i] = xn[i];
+      } else {
+        inputs(r, t, x);
+      }
+      line(x, o);
+      if (act && t < D * D && j + k < D) {
+#pragma unroll
+        for (int c = 0; c < D; ++c) rb[(c * D + j) * D + k] = o[c];
+      }
+    }
+    if constexpr (refit_prefetch<D>()) inputs(r + stride, tl, xn);
+    __syncthreads();
+#pragma unroll 1
+    for (int n = 0; n < kLines; ++n) {
+      const int t = tl + n * TS < D * D ? tl + n * TS : D * D - 1;
+      const int c = t / D, k = t % D;  // t = c * D + k
+      double x[D], o[D];
+#pragma unroll
+      for (int j = 0; j < D; ++j) x[j] = j + k < D ? rb[(c * D + j) * D + k] : 0.0;
+      line(x, o);
+      if (act && tl + n * TS < D * D) {
+#pragma unroll
+        for (int b = 0; b < D; ++b) ra[(c * D + b) * D + k] = o[b];
+      }
+    }
+    __syncthreads();
+    TO *v = V + (act ? r : 0) * P;
+#pragma unroll 1
+    for (int n = 0; n < kLines; ++n) {
+      const int t = tl + n * TS < D * D ? tl + n * TS : D * D - 1;  // t = c * D + b
+      double x[D], o[D];
+#pragma unroll
+      for (int k = 0; k < D; ++k) x[k] = ra[t * D + k];
+      line(x, o);
+      if (act && tl + n * TS < D * D) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) v[t * D + a] = (TO)o[a];
       }
     }
     __syncthreads();  // the next rows reuse sa and sb

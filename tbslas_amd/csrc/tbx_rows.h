@@ -220,6 +220,48 @@ __device__ __forceinline__ void row_start(float &w, float c, const float *p) {
 #undef TBX_F
 #undef TBX_M
 
+// acc[n] += c[K + n] x, n < N: lanes K .. K + N - 1 of the DPP row's register
+// c, one accumulator each (the s_nop as above).
+template <int K, int N>
+__device__ __forceinline__ void row_outer(double *acc, double c, double x) {
+  static_assert(N >= 1 && N <= 16 && K + N <= 16, "within a row");
+  if constexpr (N >= 8) {
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, %8, %9 row_newbcast:%10+0 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, %8, %9 row_newbcast:%10+1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, %8, %9 row_newbcast:%10+2 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, %8, %9 row_newbcast:%10+3 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %4, %8, %9 row_newbcast:%10+4 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %5, %8, %9 row_newbcast:%10+5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %6, %8, %9 row_newbcast:%10+6 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %7, %8, %9 row_newbcast:%10+7 row_mask:0xf bank_mask:0xf\n\t"
+                 : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7])
+                 : "v"(c), "v"(x), "n"(K));
+    if constexpr (N > 8) row_outer<K + 8, N - 8>(acc + 8, c, x);
+  } else if constexpr (N >= 4) {
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, %4, %5 row_newbcast:%6+0 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, %4, %5 row_newbcast:%6+1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, %4, %5 row_newbcast:%6+2 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, %4, %5 row_newbcast:%6+3 row_mask:0xf bank_mask:0xf\n\t"
+                 : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])
+                 : "v"(c), "v"(x), "n"(K));
+    if constexpr (N > 4) row_outer<K + 4, N - 4>(acc + 4, c, x);
+  } else if constexpr (N >= 2) {
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, %2, %3 row_newbcast:%4+0 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, %2, %3 row_newbcast:%4+1 row_mask:0xf bank_mask:0xf\n\t"
+                 : "+v"(acc[0]), "+v"(acc[1])
+                 : "v"(c), "v"(x), "n"(K));
+    if constexpr (N > 2) row_outer<K + 2, N - 2>(acc + 2, c, x);
+  } else {
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3+0 row_mask:0xf bank_mask:0xf\n\t"
+                 : "+v"(acc[0])
+                 : "v"(c), "v"(x), "n"(K));
+  }
+}
+
 // w += a b in its place among the row operations: left to the scheduler, the
 // outer sums gather at the end and every row's partial sum stays live.
 __device__ __forceinline__ void fmac_here(double &w, double a, double b) {
