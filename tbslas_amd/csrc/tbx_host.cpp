@@ -1773,7 +1773,7 @@ struct tbx_batch_s {
   std::vector<BatchProblem> host;  // table for the current configuration
   float *d_vel32 = nullptr, *d_conc32[2] = {nullptr, nullptr};
   float *d_vnode = nullptr;        // the velocities at their grid nodes, or null
-  std::map<int, double *> d_M;     // refit operator per degree
+  std::map<int, double *> d_H;     // per degree: the refit's operator, then its table
   BatchProblem *d_table = nullptr;
   unsigned long long *d_counter = nullptr;
   int64_t total_items = 0;
@@ -1812,7 +1812,7 @@ void free_batch(tbx_batch *b) {
   hipFree(b->d_vnode);
   hipFree(b->d_conc32[0]);
   hipFree(b->d_conc32[1]);
-  for (auto &kv : b->d_M) hipFree(kv.second);
+  for (auto &kv : b->d_H) hipFree(kv.second);
   hipFree(b->d_table);
   hipFree(b->d_counter);
   delete b;
@@ -1920,11 +1920,13 @@ int tbx_batch_create(int nprob, const tbx_tree *const *vel, const tbx_tree *cons
     HIP_TRY(hipMalloc(&b->d_counter, sizeof(unsigned long long)));
     HIP_TRY(hipStreamCreate(&b->cap));
     for (int q : {6, 8, 10}) {
-      const std::vector<double> &M = pt2coeff_cached(q);
+      const RefitOperator &op = refit_operator_cached(q);
+      std::vector<double> h(op.H);
+      for (int k = 0; k <= q; ++k) h.insert(h.end(), op.tab.T[k], op.tab.T[k] + q + 1);
       double *d = nullptr;
-      HIP_TRY(hipMalloc(&d, sizeof(double) * M.size()));
-      b->d_M[q] = d;
-      HIP_TRY(hipMemcpy(d, M.data(), sizeof(double) * M.size(), hipMemcpyHostToDevice));
+      HIP_TRY(hipMalloc(&d, sizeof(double) * h.size()));
+      b->d_H[q] = d;
+      HIP_TRY(hipMemcpy(d, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
     }
     b->host.resize(nprob);
     // the stationary velocities at their grid nodes for the first RK2
@@ -1953,7 +1955,10 @@ int tbx_batch_create(int nprob, const tbx_tree *const *vel, const tbx_tree *cons
       }
       pb.out32[0] = b->d_conc32[1] + b->conc_off[p];
       pb.out32[1] = b->d_conc32[0] + b->conc_off[p];
-      pb.M = b->d_M[tc->q];
+      const RefitOperator &op = refit_operator_cached(tc->q);
+      pb.H = b->d_H[tc->q];
+      pb.T = pb.H + op.H.size();
+      pb.np = op.NP;
       if (b->d_vnode) {
         float *vn = b->d_vnode + onode;
         const int erc = expand_grid_values(const_cast<tbx_tree *>(tv), nullptr, vn, nullptr,

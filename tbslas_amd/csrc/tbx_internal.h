@@ -194,12 +194,14 @@ struct BatchProblem {
   TreeView vel;         // coeff32: the batch's FP32 velocity coefficients
   TreeView conc[2];     // coeff32: the FP32 state read by a step of parity k
   float *out32[2];      // written by a step of parity k (= conc[1 - k].coeff32)
-  const double *M;      // [P][Nc] refit operator
+  const double *T;      // [d][d] one-axis table, T_k at node a
+  const double *H;      // [Nc][np] refit operator after the projection
   const float *vnode;   // the velocity at its grid nodes [Lv][3][P] (FP32), or null
   int64_t item0;        // first work item
   int64_t L;            // concentration leaves
   int32_t q;
   int32_t bc;
+  int32_t np;           // row stride of H
   double tau, htau;
   double node[17];
 };
