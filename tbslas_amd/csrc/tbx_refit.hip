@@ -133,16 +133,6 @@ __global__ __launch_bounds__(kGemmThreads) void k_refit_gemm(
     }
 }
 
-// Packed index of term (i, j, k) of the triangle i -> j -> k, i+j+k < D.
-template <int D>
-__device__ __forceinline__ int packed_index(int i, int j, int k) {
-  // terms before block i: sum_{a<i} (D-a)(D-a+1)/2; before row j of block
-  // i: sum_{b<j} (D-i-b)
-  const int n = D - i;
-  const int before_i = (D * (D + 1) * (D + 2) - n * (n + 1) * (n + 2)) / 6;
-  return before_i + j * n - j * (j - 1) / 2 + k;
-}
-
 constexpr int kRefitThreads = 256;
 
 // Rows a workgroup works on at once: as many teams of D^2 threads (one per
@@ -160,6 +150,46 @@ constexpr bool refit_prefetch() {
   return D * D <= kRefitThreads;
 }
 
+// A line of a one-axis contraction: out[n] = sum_a M(n, a) x[a] in the order
+// of a, M(n, a) = T[n][a] (rows_out) or T[a][n].  The table sits in
+// registers, the entries of input a across the 16 lanes of each DPP row, and
+// v_fmac broadcasts the one it needs (row_outer).  The 17th output of degree
+// 16 has its entries across the lanes of one register of its own, but for
+// the last, which is in all lanes of another.
+template <int D>
+struct RefitLine {
+  static constexpr int N = D < 16 ? D : 16;
+  double tr[D], last, corner;
+  __device__ __forceinline__ RefitLine(const double (&T)[TBX_MAX_Q + 1][TBX_MAX_Q + 1],
+                                       bool rows_out) {
+    const int l = (int)(threadIdx.x & 15u), n = l < D ? l : 0;
+#pragma unroll
+    for (int a = 0; a < D; ++a) tr[a] = rows_out ? T[n][a] : T[a][n];
+    if constexpr (D > 16) {
+      last = rows_out ? T[16][n] : T[n][16];
+      corner = T[16][16];
+    }
+  }
+  __device__ __forceinline__ void operator()(const double (&x)[D], double (&o)[D]) const {
+#pragma unroll
+    for (int n = 0; n < D; ++n) o[n] = 0.0;
+#pragma unroll
+    for (int a = 0; a < D; ++a) row_outer<0, N>(o, tr[a], x[a]);
+    if constexpr (D > 16) {
+      static_for<16>([&](auto a) {
+        row_outer<decltype(a)::value, 1>(o + 16, last, x[decltype(a)::value]);
+      });
+      o[16] = __builtin_fma(corner, x[16], o[16]);
+    }
+  }
+};
+
+// Waves per SIMD asked of the projection and the expansion: without spills.
+template <int D>
+constexpr int refit_waves() {
+  return D <= 11 ? 4 : D == 16 ? 2 : 3;
+}
+
 // w = S v per row with S = S_z (x) S_y (x) S_x restricted to the triangle:
 // one team of threads per row (refit_rows rows per workgroup at a time).
 //   a[c][b][k] = sum_a S[k][a] v[c][b][a]
@@ -171,8 +201,18 @@ constexpr bool refit_prefetch() {
 // (cs = P, ps = 1 for [L][dof][P] values; cs = 1, ps = dof for point-major
 // [L][P][dof]); W rows have stride ldw, entries Nc .. ldw-1 written as 0.
 // ACC: w is added to W instead (entries past Nc untouched).
+//
+// The intermediate lives in one LDS buffer: the second contraction's lines
+// are read and written back by one thread each.  Every lane of a workgroup
+// takes part in each line (its table entries are read by its neighbours);
+// lines past the last, and rows of idle threads, are computed and dropped.
+// With scalar table operands and two buffers, before: 36,324 rows of degree
+// 14 644 us, now 331; 4,096 x 3 rows of degree 10 56 -> 44 us, 4,096 rows of
+// degree 8 14 -> 11 us.  Bound by its LDS stages; the values' read alone
+// would take 0.19 ms, 25 us and 4.6 us.
 template <int D, bool ACC>
-__global__ __launch_bounds__(kRefitThreads) void k_refit_project(const double *__restrict__ V,
+__global__ __launch_bounds__(kRefitThreads) __attribute__((
+    amdgpu_waves_per_eu(refit_waves<D>()))) void k_refit_project(const double *__restrict__ V,
                                                                  int64_t rows, int dof,
                                                                  int64_t cs, int64_t ps,
                                                                  RefitTable tab,
@@ -181,102 +221,89 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_project(const double *_
   constexpr int P = D * D * D, NC = D * (D + 1) * (D + 2) / 6;
   constexpr int R = refit_rows<D>();
   constexpr int TS = R > 1 ? D * D : kRefitThreads;  // threads of a row's team
+  constexpr int kLines = (D * D + TS - 1) / TS;
   __shared__ double sa[R * P];
-  __shared__ double sb[R * P];
   const int tid = threadIdx.x;
   const int rl = tid / TS < R ? tid / TS : R - 1;  // this thread's row of the group
   const int tl = tid - (tid / TS) * TS;
   const bool team = tid < R * TS;
-  double *ra = sa + rl * P, *rb = sb + rl * P;
-  // The one-axis table S is read from the kernel arguments: every index
-  // into it is wave-uniform, so its entries arrive as scalar operands
-  // instead of LDS broadcasts (k_refit_expand keeps its copy in LDS; read
-  // this way there it ran slower).
-  // The first (c, b) line of the thread's next row is loaded while the
-  // current row goes through its LDS stages, so that each row does not
-  // wait for its own loads (two workgroups per CU at q = 14).
+  double *ra = sa + rl * P;
+  const RefitLine<D> line(tab.T, true);
+  // Up to degree 8 the first (c, b) line of the thread's next row is loaded
+  // while the current row goes through its LDS stages, so that each row does
+  // not wait for its own loads; above, the registers are better spent on a
+  // further wave per SIMD (degree 10 48.8 -> 44.0 us, degree 14 58 -> 51 us).
+  constexpr bool ahead = D <= 9;
   const int64_t stride = (int64_t)gridDim.x * R;
-  double xn[D];
-  auto fetch = [&](int64_t r) {
-    if (refit_prefetch<D>() && team && tl < D * D && r < rows) {
-      const double *v = V + (r / dof) * (int64_t)P * dof + (r % dof) * cs;
+  auto inputs = [&](int64_t r, int t, double (&x)[D]) {
+    const bool in = team && t < D * D && r < rows;
+    const double *v = V + ((in ? r : 0) / dof) * (int64_t)P * dof + ((in ? r : 0) % dof) * cs;
 #pragma unroll
-      for (int a = 0; a < D; ++a) xn[a] = v[(tl * D + a) * ps];
-    }
+    for (int a = 0; a < D; ++a) x[a] = in ? v[(t * D + a) * ps] : 0.0;
   };
-  fetch((int64_t)blockIdx.x * R + rl);
-  __syncthreads();
+  double xn[D];
+  if constexpr (ahead) inputs((int64_t)blockIdx.x * R + rl, tl, xn);
   for (int64_t r0 = (int64_t)blockIdx.x * R; r0 < rows; r0 += stride) {
     const int64_t r = r0 + rl;
     const bool act = team && r < rows;
-    if (act) {
-      const double *v = V + (r / dof) * (int64_t)P * dof + (r % dof) * cs;
-      for (int t = tl; t < D * D; t += TS) {  // t = c * D + b
-        double x[D];
-        if (refit_prefetch<D>() && t == tl) {
-#pragma unroll
-          for (int a = 0; a < D; ++a) x[a] = xn[a];
-        } else {
-#pragma unroll
-          for (int a = 0; a < D; ++a) x[a] = v[(t * D + a) * ps];
-        }
-        auto out = [&](int k) {
-          double s = 0.0;
-#pragma unroll
-          for (int a = 0; a < D; ++a) s = __builtin_fma(tab.T[k][a], x[a], s);
-          ra[t * D + k] = s;
-        };
-        // several rows at once: one output at a time keeps the registers
-        // (and the waves per SIMD) that the rows' latency needs; one row:
-        // all outputs unrolled for their independent chains
-        if constexpr (R > 1) {
 #pragma unroll 1
-          for (int k = 0; k < D; ++k) out(k);
-        } else {
+    for (int n = 0; n < kLines; ++n) {
+      const int t = tl + n * TS;  // t = c * D + b
+      double x[D], o[D];
+      if constexpr (ahead) {
 #pragma unroll
-          for (int k = 0; k < D; ++k) out(k);
+        for (int a = 0; a < D; ++a) x[a] = xn[a];
+      } else {
+        inputs(r, t, x);
+      }
+      line(x, o);
+      if (act && t < D * D) {
+#pragma unroll
+        for (int k = 0; k < D; ++k) ra[t * D + k] = o[k];
+      }
+    }
+    if constexpr (ahead) inputs(r + stride, tl, xn);
+    __syncthreads();
+#pragma unroll 1
+    for (int n = 0; n < kLines; ++n) {
+      const int t = tl + n * TS < D * D ? tl + n * TS : D * D - 1;
+      double *p = ra + t / D * (D * D) + t % D;  // t = c * D + k
+      double x[D], o[D];
+#pragma unroll
+      for (int b = 0; b < D; ++b) x[b] = p[b * D];
+      line(x, o);
+      if (act && tl + n * TS < D * D) {
+#pragma unroll
+        for (int j = 0; j < D; ++j) p[j * D] = o[j];
+      }
+    }
+    __syncthreads();
+    double *w = W + (act ? r : 0) * ldw;
+#pragma unroll 1
+    for (int n = 0; n < kLines; ++n) {
+      const int t = tl + n * TS < D * D ? tl + n * TS : D * D - 1;
+      const int j = t / D, k = t % D;  // t = j * D + k
+      double x[D], o[D];
+#pragma unroll
+      for (int c = 0; c < D; ++c) x[c] = ra[c * (D * D) + t];
+      line(x, o);
+      if (act && tl + n * TS < D * D) {
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+          if (i + j + k < D) {
+            if constexpr (ACC)
+              w[tri_start(D, i, j) + k] += o[i];
+            else
+              w[tri_start(D, i, j) + k] = o[i];
+          }
         }
       }
     }
-    fetch(r + stride);
-    __syncthreads();
-    if (act) {
-      for (int t = tl; t < D * D; t += TS) {  // t = c * D + k
-        const int c = t / D, k = t % D;
-        double x[D];
-#pragma unroll
-        for (int b = 0; b < D; ++b) x[b] = ra[(c * D + b) * D + k];
-        for (int j = 0; j + k < D; ++j) {
-          double s = 0.0;
-#pragma unroll
-          for (int b = 0; b < D; ++b) s = __builtin_fma(tab.T[j][b], x[b], s);
-          rb[(c * D + j) * D + k] = s;
-        }
-      }
-    }
-    __syncthreads();
-    if (act) {
-      double *w = W + r * ldw;
-      for (int t = tl; t < D * D; t += TS) {  // t = j * D + k
-        const int j = t / D, k = t % D;
-        if (j + k >= D) continue;
-        double x[D];
-#pragma unroll
-        for (int c = 0; c < D; ++c) x[c] = rb[(c * D + j) * D + k];
-        for (int i = 0; i + j + k < D; ++i) {
-          double s = 0.0;
-#pragma unroll
-          for (int c = 0; c < D; ++c) s = __builtin_fma(tab.T[i][c], x[c], s);
-          if constexpr (ACC)
-            w[packed_index<D>(i, j, k)] += s;
-          else
-            w[packed_index<D>(i, j, k)] = s;
-        }
-      }
-      if constexpr (!ACC)
+    if constexpr (!ACC) {
+      if (act)
         for (int m = NC + tl; m < ldw; m += TS) w[m] = 0.0;
     }
-    __syncthreads();  // the next rows reuse sa and sb
+    __syncthreads();  // the next rows reuse sa
   }
 }
 
@@ -285,57 +312,29 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_project(const double *_
 // three one-axis contractions z, y, x through LDS.  TO: the output precision
 // (FP32 for the FP32 modes' nodal velocities).
 //
-// A line's D outputs are sums over its D inputs with the one-axis table's
-// entries as the other factor.  The table sits in registers, row i across
-// the 16 lanes of each DPP row, and v_fmac broadcasts the entry it needs
-// (row_outer) in place of one LDS read per multiply-add: 108,972 rows of
-// degree 14 1.42 -> 1.00 ms, 4,096 x 3 rows of degree 10 143 -> 73 us, of
-// degree 8 62 -> 42 us.  At degree 16 the 17 entries do not fit a row's
-// lanes; its table stays in LDS.  (A variant
+// With the table read from LDS and two buffers: 108,972 rows of degree 14
+// 1.42 ms; the table in registers 1.00; one buffer (each line of the second
+// contraction is read and written back by one thread), so that five
+// workgroups in place of two fit a compute unit's LDS, 0.87 ms.  Of degree
+// 10, 4,096 x 3 rows: 143, 73, 67 us; of degree 8: 62, 42, 39 us.  Reading
+// and writing alone would take 0.4 ms, 31 us and 17 us.  (A variant
 // contracting x first over the triangle, with y and z in registers, does a
 // third fewer multiply-adds but ran 1.3x slower than the LDS form.)
 template <int D, typename TO>
-__global__ __launch_bounds__(kRefitThreads) void k_refit_expand(const double *__restrict__ U,
+__global__ __launch_bounds__(kRefitThreads) __attribute__((
+    amdgpu_waves_per_eu(refit_waves<D>()))) void k_refit_expand(const double *__restrict__ U,
                                                                 int64_t rows, RefitTable tab,
                                                                 int KP, TO *__restrict__ V) {
   constexpr int P = D * D * D;
   constexpr int R = refit_rows<D>();
   constexpr int TS = R > 1 ? D * D : kRefitThreads;  // threads of a row's team
-  constexpr bool kDpp = D <= 16;
   __shared__ double sa[R * P];
-  __shared__ double sb[R * P];
-  __shared__ double sT[D * D];
   const int tid = threadIdx.x;
   const int rl = tid / TS < R ? tid / TS : R - 1;  // this thread's row of the group
   const int tl = tid - (tid / TS) * TS;
   const bool team = tid < R * TS;
-  double *ra = sa + rl * P, *rb = sb + rl * P;
-  for (int t = tid; t < D * D; t += kRefitThreads) sT[t] = tab.T[t / D][t % D];
-  __syncthreads();
-  double tr[kDpp ? D : 1];  // row i of the table, entry lane % 16
-  if constexpr (kDpp) {
-#pragma unroll
-    for (int i = 0; i < D; ++i) tr[i] = sT[i * D + ((tid & 15) < D ? (tid & 15) : 0)];
-  }
-  // out[c] = sum_i T[i][c] x[i]; every lane takes part (its table entries
-  // are read by its neighbours)
-  auto line = [&](const double (&x)[D], double (&out)[D]) {
-#pragma unroll
-    for (int c = 0; c < D; ++c) out[c] = 0.0;
-    if constexpr (kDpp) {
-#pragma unroll
-      for (int i = 0; i < D; ++i) row_outer<0, D>(out, tr[i], x[i]);
-    } else {
-#pragma unroll 1
-      for (int c = 0; c < D; ++c) {
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < D; ++i) s = __builtin_fma(sT[i * D + c], x[i], s);
-#pragma unroll
-        for (int e = 0; e < D; ++e) out[e] = e == c ? s : out[e];
-      }
-    }
-  };
+  double *ra = sa + rl * P;
+  const RefitLine<D> line(tab.T, false);
   // the first (j, k) line of the thread's next row loaded during the
   // current row's LDS stages, as in k_refit_project
   const int64_t stride = (int64_t)gridDim.x * R;
@@ -358,7 +357,7 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_expand(const double *__
     for (int n = 0; n < kLines; ++n) {
       const int t = tl + n * TS, j = t / D, k = t % D;  // t = j * D + k
       double x[D], o[D];
-      if (refit_prefetch<D>()) {
+      if constexpr (refit_prefetch<D>()) {
 #pragma unroll
         for (int i = 0; i < D; ++i) x[i] = xn[i];
       } else {
@@ -367,7 +366,7 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_expand(const double *__
       line(x, o);
       if (act && t < D * D && j + k < D) {
 #pragma unroll
-        for (int c = 0; c < D; ++c) rb[(c * D + j) * D + k] = o[c];
+        for (int c = 0; c < D; ++c) ra[(c * D + j) * D + k] = o[c];
       }
     }
     if constexpr (refit_prefetch<D>()) inputs(r + stride, tl, xn);
@@ -375,14 +374,15 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_expand(const double *__
 #pragma unroll 1
     for (int n = 0; n < kLines; ++n) {
       const int t = tl + n * TS < D * D ? tl + n * TS : D * D - 1;
-      const int c = t / D, k = t % D;  // t = c * D + k
+      const int k = t % D;  // t = c * D + k
+      double *p = ra + t / D * (D * D) + k;
       double x[D], o[D];
 #pragma unroll
-      for (int j = 0; j < D; ++j) x[j] = j + k < D ? rb[(c * D + j) * D + k] : 0.0;
+      for (int j = 0; j < D; ++j) x[j] = j + k < D ? p[j * D] : 0.0;
       line(x, o);
       if (act && tl + n * TS < D * D) {
 #pragma unroll
-        for (int b = 0; b < D; ++b) ra[(c * D + b) * D + k] = o[b];
+        for (int b = 0; b < D; ++b) p[b * D] = o[b];
       }
     }
     __syncthreads();
@@ -399,7 +399,7 @@ __global__ __launch_bounds__(kRefitThreads) void k_refit_expand(const double *__
         for (int a = 0; a < D; ++a) v[t * D + a] = (TO)o[a];
       }
     }
-    __syncthreads();  // the next rows reuse sa and sb
+    __syncthreads();  // the next rows reuse sa
   }
 }
 
