@@ -9,11 +9,12 @@
 //
 //   M = 16 components, N = 16 points, K = 4 basis terms per instruction.
 //
-// K walks the packed triangle four terms at a time, the four lane groups
-// g = lane / 16 taking terms 4q + g (165 terms in 42 chunks at q = 8).  A
-// lane's A operand is coeff[c0 + lane % 16][4q + g], its B operand
-// T_i(z) T_j(y) T_k(x) of term 4q + g at its tile point: the chunk's four
-// products are formed and the lane picks its own.
+// K walks the packed triangle in chunks of 4 S terms (S = 4 in FP32, 2 in
+// FP64), the four lane groups g = lane / 16 taking S consecutive ones each
+// (165 terms in 11 FP32 chunks at q = 8).  A lane's A operands are those
+// terms of coeff[c0 + lane % 16], one 16-byte load; its B operands
+// T_i(z) T_j(y) T_k(x) at its tile point: the chunk's products are formed
+// and the lane picks its own.
 //
 // Operand layouts of v_mfma_{f64,f32}_16x16x4 (both measured on gfx950):
 // A[i][k] in lane i + 16 k, B[k][j] in lane j + 16 k; the result D[i][j]
@@ -91,14 +92,14 @@ __device__ __forceinline__ int64_t lane_read_i64(int64_t v, int src) {
   return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 
-// The packed triangle in chunks of four consecutive terms: chunk q holds
-// packed indices 4q .. 4q + 3 (lane group g takes 4q + g), with their
-// (i, j, k); indices past Nc are padding.
-template <int D>
+// The packed triangle in chunks of 4 S consecutive terms: lane group g takes
+// the S terms from 4 S q + S g of chunk q, with their (i, j, k); indices past
+// Nc are padding.  S terms are one 16-byte load.
+template <int D, int S>
 struct MfmaChunks {
   static constexpr int NC = D * (D + 1) * (D + 2) / 6;
-  static constexpr int N = (NC + 3) / 4;
-  int i[4 * N], j[4 * N], k[4 * N];
+  static constexpr int N = (NC + 4 * S - 1) / (4 * S);
+  int i[4 * S * N], j[4 * S * N], k[4 * S * N];
   constexpr MfmaChunks() : i(), j(), k() {
     int m = 0;
     for (int a = 0; a < D; ++a)
@@ -109,7 +110,7 @@ struct MfmaChunks {
           k[m] = c;
           ++m;
         }
-    for (; m < 4 * N; ++m) i[m] = j[m] = k[m] = 0;
+    for (; m < 4 * S * N; ++m) i[m] = j[m] = k[m] = 0;
   }
 };
 
@@ -118,82 +119,87 @@ struct MfmaChunks {
 // offset a 32-bit register and the chunk's a scalar.  Reads past the extent
 // return 0.  Descriptor word 3 of the gfx9 family (raw, 32-bit data).
 constexpr int kBufferWord3 = 0x00020000;
+constexpr int kChunkBytes = 64;  // of one component in a chunk of terms
 
-template <typename T>
-__device__ __forceinline__ T buffer_coeff(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  if constexpr (sizeof(T) == 8) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-    return __hiloint2double((int)v[1], (int)v[0]);
-  } else {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+template <typename T, int S>
+__device__ __forceinline__ void buffer_coeffs(__amdgpu_buffer_rsrc_t r, int voff, int soff,
+                                              T (&a)[S]) {
+  static_assert(sizeof(T) * S == 16, "one 16-byte load");
+  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    if constexpr (sizeof(T) == 8)
+      a[s] = __hiloint2double((int)v[2 * s + 1], (int)v[2 * s]);
+    else
+      a[s] = __uint_as_float(v[s]);
   }
 }
 
-// One leaf's terms for NT M tiles (16 NT components) and the two N tiles:
-// acc[mt][n] += coeff tile mt x basis tile n.  rsrc covers the leaf's
-// components from the first of the tiles; voff = the lane's byte offset
-// (component lane % 16, term slot g); in[n]: the lane's tile point n lies
-// in the leaf (its B operand is zero otherwise).  K runs over the packed
-// triangle four terms at a time; the lane's B operand is the product of
-// its term's three basis values, picked among the chunk's four by 0/1
-// weights (no divergent selection).  The
-// chunks are unrolled; the A operands are loaded two chunks ahead and a
-// scheduling barrier closes every chunk, which keeps the loads in flight
-// under the MFMAs without hoisting them all to the top.
-template <int D, typename T, int NT>
+// One leaf's terms for NT M tiles (16 NT components) and N tiles N0 .. N1 - 1
+// of the two: acc[mt][n] += coeff tile mt x basis tile n.  rsrc covers the
+// leaf's components from the first of the tiles; voff = the lane's byte
+// offset (component lane % 16, terms S g ..); in[n]: the lane's tile point n
+// lies in the leaf (its B operand is zero otherwise).
+//
+// The order of the terms over K is free: a lane group takes S consecutive
+// ones (16 bytes), so that a component's cache line is visited twice and not
+// once per four terms.  Visited eight times, by some ten wavefronts with 64
+// components each, the lines did not stay in the 32 KB L1 and the matrix
+// cores waited (see eval_dof_mfma for the times).  The chunk's products are
+// formed once per tile point and each lane picks its S by its group's bits.
+// The chunks are unrolled; an M tile's next operands are loaded when its
+// products of the chunk are done, under the other tiles' MFMAs, and
+// scheduling barriers keep that order.
+template <int D, typename T, int NT, int N0, int N1>
 __device__ __forceinline__ void mfma_leaf_terms(__amdgpu_buffer_rsrc_t rsrc, int voff, int g,
                                                 const bool (&in)[2], const T (&tz)[2][D],
                                                 const T (&ty)[2][D], const T (&tx)[2][D],
                                                 typename MfmaAcc<T>::V (&acc)[4][2]) {
   using Acc = MfmaAcc<T>;
-  constexpr int NC = MfmaChunks<D>::NC;
-  constexpr int NQ = MfmaChunks<D>::N;
-  const bool last_valid = 4 * (NQ - 1) + g < NC;  // the final chunk's padding
-  // the lane's pick among a chunk's four products as 0/1 weights: a
-  // branch-free, exact selection (finite products times 0 and 1)
-  T w[4];
+  constexpr int S = 16 / (int)sizeof(T);
+  constexpr int NC = MfmaChunks<D, S>::NC;
+  constexpr int NQ = MfmaChunks<D, S>::N;
+  const bool odd = g & 1, high = g & 2;
+  T a[NT][S];
+  auto load = [&](int q, int mt) {
+    buffer_coeffs<T, S>(rsrc, voff, (int)sizeof(T) * (mt * 16 * NC + 4 * S * q), a[mt]);
+    if (q == NQ - 1) {  // the final chunk's padding
 #pragma unroll
-  for (int s = 0; s < 4; ++s) w[s] = g == s ? (T)1 : (T)0;
-  auto load = [&](int q, T (&a)[NT]) {
-#pragma unroll
-    for (int mt = 0; mt < NT; ++mt) {
-      const int soff = (int)sizeof(T) * (mt * 16 * NC + 4 * q);
-      const T v = buffer_coeff<T>(rsrc, voff, soff);
-      a[mt] = (q < NQ - 1 || last_valid) ? v : (T)0;
+      for (int s = 0; s < S; ++s)
+        if (4 * S * q + S * g + s >= NC) a[mt][s] = (T)0;
     }
   };
-  T a0[NT], a1[NT];
-  load(0, a0);
-  if (NQ > 1) load(1, a1);
+#pragma unroll
+  for (int mt = 0; mt < NT; ++mt) load(0, mt);
   static_for<NQ>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
-    T a2[NT];
-    if constexpr (q + 2 < NQ) load(q + 2, a2);
-    T bv[2];
+    T bv[2][S];
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
+    for (int n = N0; n < N1; ++n) {
+      constexpr MfmaChunks<D, S> tab{};
       // the leaf mask first: products of the pass, not hoisted out of it
-      T p[4];
+      T p[4 * S], zy = (T)0;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        constexpr MfmaChunks<D> tab{};
-        const int m = 4 * q + s;
-        const T zm = in[n] ? tz[n][tab.i[m]] : (T)0;
-        p[s] = m < NC ? zm * ty[n][tab.j[m]] * tx[n][tab.k[m]] : (T)0;
+      for (int s = 0; s < 4 * S; ++s) {
+        const int m = 4 * S * q + s;
+        if (s == 0 || tab.k[m] == 0) zy = (in[n] ? tz[n][tab.i[m]] : (T)0) * ty[n][tab.j[m]];
+        p[s] = m < NC ? zy * tx[n][tab.k[m]] : (T)0;
       }
-      T b = p[0] * w[0];
 #pragma unroll
-      for (int s = 1; s < 4; ++s) b = fma_t(p[s], w[s], b);
-      bv[n] = b;
+      for (int s = 0; s < S; ++s) {
+        const T lo = odd ? p[S + s] : p[s], hi = odd ? p[3 * S + s] : p[2 * S + s];
+        bv[n][s] = high ? hi : lo;
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int mt = 0; mt < NT; ++mt)
-#pragma unroll
-      for (int n = 0; n < 2; ++n) acc[mt][n] = Acc::mma(a0[mt], bv[n], acc[mt][n]);
-#pragma unroll
     for (int mt = 0; mt < NT; ++mt) {
-      a0[mt] = a1[mt];
-      if constexpr (q + 2 < NQ) a1[mt] = a2[mt];
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int n = N0; n < N1; ++n) acc[mt][n] = Acc::mma(a[mt][s], bv[n][s], acc[mt][n]);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (q + 1 < NQ) load(q + 1, mt);
     }
     __builtin_amdgcn_sched_barrier(0);
   });
@@ -253,24 +259,30 @@ __device__ __forceinline__ void eval_dof_mfma(const TreeView &t, int leaf, doubl
         const int lf = __builtin_amdgcn_readlane(leaf, __builtin_ctzll(pending));
         pending &= ~__builtin_amdgcn_ballot_w64(leaf == lf);
         const bool in[2] = {pleaf[0] == lf, pleaf[1] == lf};
-        // the buffer: components c0 .. c0 + 16 ntile - 1 of leaf lf
+        // the buffer: components c0 .. c0 + 16 ntile - 1 of leaf lf, and the
+        // last chunk's padding behind them (coefficient arrays end in 256
+        // bytes of it)
         const T *cb = coeff + ((int64_t)lf * dof + c0) * NC;
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<T *>(cb), 0, (int)sizeof(T) * 16 * ntile * NC, kBufferWord3);
-        const int voff = (int)sizeof(T) * (col * NC + g);
-        switch (ntile) {  // wave-uniform
-          case 4:
-            mfma_leaf_terms<D, T, 4>(rsrc, voff, g, in, tz, ty, tx, acc);
-            break;
-          case 3:
-            mfma_leaf_terms<D, T, 3>(rsrc, voff, g, in, tz, ty, tx, acc);
-            break;
-          case 2:
-            mfma_leaf_terms<D, T, 2>(rsrc, voff, g, in, tz, ty, tx, acc);
-            break;
-          default:
-            mfma_leaf_terms<D, T, 1>(rsrc, voff, g, in, tz, ty, tx, acc);
-            break;
+            const_cast<T *>(cb), 0, (int)sizeof(T) * 16 * ntile * NC + kChunkBytes, kBufferWord3);
+        const int voff = (int)sizeof(T) * col * NC + 16 * g;
+        // runs of a leaf are whole N tiles: where the two are of different
+        // leaves, each pass does the tile that is in its leaf
+        const bool any0 = __builtin_amdgcn_ballot_w64(in[0]) != 0,
+                   any1 = __builtin_amdgcn_ballot_w64(in[1]) != 0;
+        if (ntile == 4) {  // wave-uniform
+          if (any0 && any1)
+            mfma_leaf_terms<D, T, 4, 0, 2>(rsrc, voff, g, in, tz, ty, tx, acc);
+          else if (any0)
+            mfma_leaf_terms<D, T, 4, 0, 1>(rsrc, voff, g, in, tz, ty, tx, acc);
+          else
+            mfma_leaf_terms<D, T, 4, 1, 2>(rsrc, voff, g, in, tz, ty, tx, acc);
+        } else if (ntile == 3) {
+          mfma_leaf_terms<D, T, 3, 0, 2>(rsrc, voff, g, in, tz, ty, tx, acc);
+        } else if (ntile == 2) {
+          mfma_leaf_terms<D, T, 2, 0, 2>(rsrc, voff, g, in, tz, ty, tx, acc);
+        } else {
+          mfma_leaf_terms<D, T, 1, 0, 2>(rsrc, voff, g, in, tz, ty, tx, acc);
         }
       }
       // lane l holds D[row(g, r)][col]: component c0 + 16 mt + row(g, r)
