@@ -92,6 +92,11 @@ __global__ __launch_bounds__(kBlock) void k_to_f32(const double *__restrict__ in
   if (i < n) out[i] = (float)in[i];
 }
 
+constexpr int kXcds = 8;
+constexpr int kMetaStride = 32;  // words: a cache line each
+constexpr int kFewLeaves = 1024;
+constexpr int kMetaWords = (1 + kXcds) * kMetaStride;
+
 // Order of a call's points by leaf (counting sort; order_words(n, L) words of
 // scratch): leaf and rank of every point, hist, then perm.  Groups follow
 // each other in no particular order; a point's place in its group depends on
@@ -99,8 +104,13 @@ __global__ __launch_bounds__(kBlock) void k_to_f32(const double *__restrict__ in
 //
 // k_order_count: rank = the point's number in its leaf.  A wavefront adds
 // once per leaf that several of its lanes share, so that many points of one
-// leaf do not queue on its counter.  meta[1] counts the wavefronts whose
-// neighbouring lanes change leaf eight times or more.
+// leaf do not queue on its counter.  Each of the eight XCDs (workgroups go to
+// them in turn) has its own counters, hist[x][L], and its own word of meta,
+// which counts the wavefronts whose neighbouring lanes change leaf eight
+// times or more: a line that the XCDs add to in turn travels between their
+// L2s.  FEW (L <= kFewLeaves): a workgroup counts in LDS and adds once per
+// leaf, for many points on few leaves would all queue on the same counters.
+template <bool FEW>
 __global__ __launch_bounds__(kBlock) void k_order_count(TreeView t,
                                                         const double *__restrict__ pts,
                                                         int64_t n, int bc,
@@ -108,6 +118,7 @@ __global__ __launch_bounds__(kBlock) void k_order_count(TreeView t,
                                                         int32_t *__restrict__ rank,
                                                         int32_t *__restrict__ hist,
                                                         int32_t *__restrict__ meta) {
+  __shared__ int cnt[FEW ? kFewLeaves : 1];
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const bool live = i < n;
   const int lane = (int)(threadIdx.x & 63u);
@@ -125,7 +136,23 @@ __global__ __launch_bounds__(kBlock) void k_order_count(TreeView t,
   const int changes =
       __builtin_popcountll(__builtin_amdgcn_ballot_w64(live && lane > 0 && lf != left));
   const int scattered = __syncthreads_count(lane == 0 && changes >= 8);
-  if (threadIdx.x == 0 && scattered) atomicAdd(&meta[1], scattered);
+  const int xcd = (int)(blockIdx.x % kXcds);
+  hist += xcd * t.L;
+  if (threadIdx.x == 0 && scattered) atomicAdd(&meta[(1 + xcd) * kMetaStride], scattered);
+  if constexpr (FEW) {
+    for (int l = (int)threadIdx.x; l < t.L; l += kBlock) cnt[l] = 0;
+    __syncthreads();
+    int r = live ? atomicAdd(&cnt[lf], 1) : 0;
+    __syncthreads();
+    for (int l = (int)threadIdx.x; l < t.L; l += kBlock)
+      if (cnt[l]) cnt[l] = atomicAdd(&hist[l], cnt[l]);
+    __syncthreads();
+    if (live) {
+      leaf[i] = lf;
+      rank[i] = r + cnt[lf];
+    }
+    return;
+  }
   uint64_t pending = __builtin_amdgcn_ballot_w64(live);
   bool todo = live;
   int r = 0;
@@ -158,7 +185,9 @@ __global__ __launch_bounds__(kBlock) void k_order_start(int32_t *__restrict__ hi
                                                         int32_t *__restrict__ meta) {
   const int64_t l = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int lane = (int)(threadIdx.x & 63u);
-  const int c = l < L ? hist[l] : 0;
+  int c = 0;
+  if (l < L)
+    for (int x = 0; x < kXcds; ++x) c += hist[x * L + l];
   int incl = c;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -168,7 +197,13 @@ __global__ __launch_bounds__(kBlock) void k_order_start(int32_t *__restrict__ hi
   int base = 0;
   if (lane == 63 && incl) base = atomicAdd(&meta[0], incl);
   base = __builtin_amdgcn_readlane(base, 63);
-  if (l < L) hist[l] = base + incl - c;
+  if (l >= L) return;
+  int start = base + incl - c;  // the leaf's places, XCD by XCD
+  for (int x = 0; x < kXcds; ++x) {
+    const int h = hist[x * L + l];
+    hist[x * L + l] = start;
+    start += h;
+  }
 }
 
 // perm[place] = point; the identity where the points came in runs of a leaf
@@ -178,11 +213,14 @@ __global__ __launch_bounds__(kBlock) void k_order_place(const int32_t *__restric
                                                         const int32_t *__restrict__ rank,
                                                         const int32_t *__restrict__ hist,
                                                         const int32_t *__restrict__ meta,
-                                                        int64_t n, int32_t *__restrict__ perm) {
+                                                        int64_t n, int64_t L,
+                                                        int32_t *__restrict__ perm) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  const bool scattered = 4 * (int64_t)meta[1] > (n + 63) / 64;
-  perm[scattered ? hist[leaf[i]] + rank[i] : i] = (int32_t)i;
+  int64_t waves = 0;
+  for (int x = 0; x < kXcds; ++x) waves += meta[(1 + x) * kMetaStride];
+  const bool scattered = 4 * waves > (n + 63) / 64;
+  perm[scattered ? hist[(blockIdx.x % kXcds) * L + leaf[i]] + rank[i] : i] = (int32_t)i;
 }
 
 __global__ __launch_bounds__(kBlock) void k_zero_words(int32_t *__restrict__ p, int64_t n) {
@@ -205,18 +243,19 @@ hipError_t launch_locate(const TreeView &t, const double *pts, int64_t n,
   return hipGetLastError();
 }
 
-int64_t order_words(int64_t n, int64_t L) { return 3 * n + L + 2; }
+int64_t order_words(int64_t n, int64_t L) { return 3 * n + kXcds * L + kMetaWords; }
 
 hipError_t launch_order_points(const TreeView &t, const double *pts, int64_t n, int bc,
                                int32_t *words, int32_t **perm, hipStream_t s) {
-  int32_t *leaf = words, *rank = leaf + n, *meta = rank + n, *hist = meta + 2;
-  *perm = hist + t.L;
-  hipLaunchKernelGGL(k_zero_words, dim3(grid_for(t.L + 2)), dim3(kBlock), 0, s, meta, t.L + 2);
-  hipLaunchKernelGGL(k_order_count, dim3(grid_for(n)), dim3(kBlock), 0, s, t, pts, n, bc, leaf,
-                     rank, hist, meta);
+  int32_t *leaf = words, *rank = leaf + n, *meta = rank + n, *hist = meta + kMetaWords;
+  *perm = hist + kXcds * t.L;
+  const int64_t zero = kXcds * t.L + kMetaWords;
+  hipLaunchKernelGGL(k_zero_words, dim3(grid_for(zero)), dim3(kBlock), 0, s, meta, zero);
+  hipLaunchKernelGGL(t.L <= kFewLeaves ? k_order_count<true> : k_order_count<false>,
+                     dim3(grid_for(n)), dim3(kBlock), 0, s, t, pts, n, bc, leaf, rank, hist, meta);
   hipLaunchKernelGGL(k_order_start, dim3(grid_for(t.L)), dim3(kBlock), 0, s, hist, t.L, meta);
   hipLaunchKernelGGL(k_order_place, dim3(grid_for(n)), dim3(kBlock), 0, s, leaf, rank, hist,
-                     meta, n, *perm);
+                     meta, n, t.L, *perm);
   return hipGetLastError();
 }
 

@@ -645,8 +645,14 @@ bool capturing(hipStream_t s) {
 // where it pays: perm stays null, and the points are taken as they come,
 //  - in TBX_EXACT (its kernels take points as they come);
 //  - under kOrderWork multiply-adds in all (ordering costs some 15 us of
-//    launches and 40 us per million points), or fewer than two points a
+//    launches and 30 us per million points), or fewer than two points a
 //    leaf (nothing to bring together);
+//  - on few leaves, which a workgroup orders by itself with little padding:
+//    up to 16 always (degree 14, 8 leaves: 1.5 M points 109 us, ordered first
+//    132; 60,007 points 16, ordered 44), up to 64 under 600 multiply-adds a
+//    point (64 leaves, degree 6, 2 M points 70 us, ordered 125; but degree
+//    14, 1.5 M points 235 us, ordered 131, and trajectories of degree 10,
+//    60,007 points 225 us, ordered 64);
 //  - on a stream that is being captured (nothing is allocated there), and
 //    without memory for it.
 constexpr double kOrderWork = 3e7;
@@ -656,7 +662,8 @@ struct PointOrder {
   hipStream_t s = nullptr;
   hipError_t make(const tbx_tree *t, const double *pts, int64_t n, int bc, int mode, double evals,
                   hipStream_t st) {
-    if (mode == kExact64 || n < 2 * t->L || n > INT32_MAX ||
+    if (mode == kExact64 || n < 2 * t->L || n > INT32_MAX || t->L <= 16 ||
+        (t->L <= 64 && evals * t->nc < 600) ||
         (double)n * evals * t->nc < kOrderWork || capturing(st))
       return hipSuccess;
     words = pool_alloc(sizeof(int32_t) * (size_t)order_words(n, t->L), st);

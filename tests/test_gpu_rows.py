@@ -90,6 +90,24 @@ def test_points_ordered_by_leaf_keep_their_values(tb, mode, kind):
     assert torch.equal(y, want)
 
 
+@pytest.mark.parametrize("depth", [1, 2, 3, 4])
+@pytest.mark.parametrize("spread", [1.0, 0.05])
+def test_order_over_leaf_counts(tb, depth, spread):
+    # 8, 64, 512 and 4,096 leaves: points as they come, and counted in LDS or
+    # in memory; over the domain or on a few leaves.  The same bits as 3,000
+    # at a time, which are never ordered.
+    import torch
+
+    anchor, dep = tb.uniform_leaves(depth)
+    rng = np.random.default_rng(depth)
+    t = tb.Tree(anchor, dep, 9, 3, rng.standard_normal((len(dep), 3, tb.ncoef(9))))
+    g = torch.Generator(device="cuda").manual_seed(depth)
+    x = torch.rand((70001, 3), dtype=torch.float64, device="cuda", generator=g) * spread + 0.45 * (1 - spread)
+    whole = t.eval(x)
+    parts = torch.cat([t.eval(x[a:a + 3000].contiguous()) for a in range(0, len(x), 3000)])
+    assert torch.equal(whole, parts)
+
+
 @pytest.mark.parametrize("nrk", [1, 3, 16, 17, 33])
 def test_ordered_trajectories_keep_their_values(tb, nrk):
     import torch
