@@ -53,13 +53,23 @@ __device__ __forceinline__ void row_samples(const T *p, T (&r)[4]) {
 // All dof components of a leaf at (x, y, z) through store(c, value): inf is
 // the leaf's anchor and depth, data its samples [dof][N^3] (FP32 samples for
 // kFp32, FP64 otherwise), in global memory or in LDS.
-// A plane of 16 samples at a time: 93 registers, five waves per SIMD; with
-// every gather of the 64 issued up front (223 registers, two waves) the step
-// on 32,768 leaves of 8^3 samples took 1.81 ms in FP64, now 1.73, and the
-// evaluation of as many points 0.54, now 0.44.  Both read 2 KB of samples
-// per point and are bound by what the L1 returns: 34 GB in 1.73 ms is 32
-// bytes per clock and compute unit, whether in 8- or 16-byte loads.
-template <int MODE, typename T, typename Store>
+// U2: planes of 16 samples unrolled.  From global memory (grid_unroll) the 64-
+// bit modes take one at a time: 93 registers, five waves per SIMD; with every
+// gather of the 64 issued up front (223 registers, two waves) the step on
+// 32,768 leaves of 8^3 samples took 1.81 ms in FP64, now 1.73, the evaluation
+// of as many points 0.54, now 0.44, and the two in TBX_EXACT 5.08, now 3.18.
+// FP32 fits all four (4,096 leaves of 10^3 samples, both: 377 us, one at a
+// time 398).  FP64 reads 2 KB of samples per point and is bound by what the
+// L1 returns: 34 GB in 1.73 ms is 32 bytes per clock and compute unit,
+// whether in 8- or 16-byte loads.  The sibling blocks, whose gathers are from
+// LDS but for the points outside, take one at a time everywhere (FP32, 4,096
+// leaves of 8^3: 206 us; four outside, 290).
+template <int MODE>
+constexpr int grid_unroll() {
+  return MODE == kFp32 ? 4 : 1;
+}
+
+template <int MODE, int U2, typename T, typename Store>
 __device__ __forceinline__ void grid_interp_at(const uint4 inf, const T *data, int N, int dof,
                                                double x, double y, double z, Store store) {
   const double s = (double)(1u << inf.w), len = 1.0 / s;
@@ -93,7 +103,7 @@ __device__ __forceinline__ void grid_interp_at(const uint4 inf, const T *data, i
     const T *cb = data + c * N3 + base;
     if constexpr (MODE == kExact64) {
       double val = 0;  // tree_functor.h:137-151
-#pragma unroll 1
+#pragma unroll U2
       for (int j2 = 0; j2 < 4; ++j2)
 #pragma unroll
         for (int j1 = 0; j1 < 4; ++j1) {
@@ -111,7 +121,7 @@ __device__ __forceinline__ void grid_interp_at(const uint4 inf, const T *data, i
 #pragma unroll
         for (int k = 0; k < 4; ++k) mf[j][k] = (float)M[j][k];
       float val = 0.f;
-#pragma unroll 1
+#pragma unroll U2
       for (int j2 = 0; j2 < 4; ++j2) {
         float vz = 0.f;
 #pragma unroll
@@ -128,7 +138,7 @@ __device__ __forceinline__ void grid_interp_at(const uint4 inf, const T *data, i
       store(c, (double)val);
     } else {
       double val = 0.0;
-#pragma unroll 1
+#pragma unroll U2
       for (int j2 = 0; j2 < 4; ++j2) {
         double vz = 0.0;
 #pragma unroll
@@ -147,14 +157,14 @@ __device__ __forceinline__ void grid_interp_at(const uint4 inf, const T *data, i
   }
 }
 
-template <int MODE, typename Store>
+template <int MODE, int U2 = grid_unroll<MODE>(), typename Store>
 __device__ __forceinline__ void grid_interp(const TreeView &t, const GridData &g, int leaf,
                                             double x, double y, double z, Store store) {
   const int64_t off = (int64_t)leaf * g.dof * g.n * g.n * g.n;
   if constexpr (MODE == kFp32)
-    grid_interp_at<MODE>(t.info[leaf], g.s32 + off, g.n, g.dof, x, y, z, store);
+    grid_interp_at<MODE, U2>(t.info[leaf], g.s32 + off, g.n, g.dof, x, y, z, store);
   else
-    grid_interp_at<MODE>(t.info[leaf], g.s + off, g.n, g.dof, x, y, z, store);
+    grid_interp_at<MODE, U2>(t.info[leaf], g.s + off, g.n, g.dof, x, y, z, store);
 }
 
 template <int MODE>
@@ -336,9 +346,9 @@ __global__ __launch_bounds__(kBlkThreads) void k_grid_step_blk(TreeView tv, Grid
       else v2 = v;
     };
     if (lb >= 0 && lb < kBlkLeaves)
-      grid_interp_at<MODE>(tv.info[leaf], sv + lb * 3 * kBlkN3, N, 3, x, y, z, st);
+      grid_interp_at<MODE, 1>(tv.info[leaf], sv + lb * 3 * kBlkN3, N, 3, x, y, z, st);
     else
-      grid_interp<MODE>(tv, vel, leaf, x, y, z, st);
+      grid_interp<MODE, 1>(tv, vel, leaf, x, y, z, st);
     if (a.scaled) {
       v0 = v0 * f;
       v1 = v1 * f;
@@ -400,9 +410,9 @@ __global__ __launch_bounds__(kBlkThreads) void k_grid_step_blk(TreeView tv, Grid
     double *o = out + leaf * kBlkN3 + m;
     auto st = [&](int, double v) { *o = v; };
     if (lb >= 0 && lb < kBlkLeaves)
-      grid_interp_at<MODE>(tc.info[cl], sc + lb * kBlkN3, N, 1, x, y, z, st);
+      grid_interp_at<MODE, 1>(tc.info[cl], sc + lb * kBlkN3, N, 1, x, y, z, st);
     else
-      grid_interp<MODE>(tc, conc, cl, x, y, z, st);
+      grid_interp<MODE, 1>(tc, conc, cl, x, y, z, st);
   }
 }
 
