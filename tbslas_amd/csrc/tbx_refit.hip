@@ -133,6 +133,49 @@ __global__ __launch_bounds__(kGemmThreads) void k_refit_gemm(
     }
 }
 
+// The same product for few rows: a wavefront per 16 x 16 tile of C, its
+// operands from global memory, no LDS and no barrier.  The sums run over k in
+// the same steps of four: the same bits.  Few rows leave k_refit_gemm one
+// workgroup on a compute unit, which waits at every chunk's loads and barrier:
+// 64 rows of degree 6 10.0 us there, 5.4 here; of degree 11 30.8 and 14.7;
+// 512 rows of degree 14 65.5 and 37.8.  With more tiles than two wavefronts
+// per SIMD the operands' repeated reads cost more: 1,536 rows of degree 14
+// (4,128 tiles) 86.5 and 101, 1,536 of degree 11 (2,208) 32.0 and 31.4.
+__global__ __launch_bounds__(64) void k_refit_gemm_few(
+    const double *__restrict__ A, int64_t lda, int64_t rows, int K, int KP,
+    const double *__restrict__ H, int np, double *__restrict__ C, int64_t ldc, int ncols,
+    float *__restrict__ C32, int ncb) {
+  const int lane = (int)threadIdx.x, li = lane & 15, lg = lane >> 4;
+  const int64_t r0 = (int64_t)(blockIdx.x / ncb) * 16;
+  const int c0 = (int)(blockIdx.x % ncb) * 16;
+  const bool ok = r0 + li < rows;
+  const double *ap = A + (ok ? r0 + li : 0) * lda;
+  const double *hp = H + c0 + li;
+  acc4 acc{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+  for (int k0 = 0; k0 < KP; k0 += kGemmBK) {
+    double av[kGemmBK / 4], bv[kGemmBK / 4];
+#pragma unroll
+    for (int s = 0; s < kGemmBK / 4; ++s) {
+      const int k = k0 + 4 * s + lg;
+      av[s] = ok && k < K ? ap[k] : 0.0;
+      bv[s] = hp[(int64_t)k * np];
+    }
+#pragma unroll
+    for (int s = 0; s < kGemmBK / 4; ++s)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s], bv[s], acc, 0, 0, 0);
+  }
+  const int col = c0 + li;
+  if (col >= ncols) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int64_t row = r0 + lg + 4 * r;
+    if (row >= rows) continue;
+    C[row * ldc + col] = acc[r];
+    if (C32) C32[row * ldc + col] = (float)acc[r];
+  }
+}
+
 constexpr int kRefitThreads = 256;
 
 // Rows a workgroup works on at once: as many teams of D^2 threads (one per
@@ -505,10 +548,19 @@ hipError_t launch_metric(const uint4 *info, int n, const double *val, const doub
   return hipGetLastError();
 }
 
+// Tiles of 16 x 16 up to which k_refit_gemm_few runs: two wavefronts per SIMD.
+constexpr int64_t kGemmFewTiles = 2048;
+
 hipError_t launch_refit_gemm(const double *A, int64_t lda, int64_t rows, int K, int KP,
                              const double *H, int np, double *C, int64_t ldc, int ncols,
                              float *C32, hipStream_t s) {
   if (rows <= 0) return hipSuccess;
+  const int ncb = (ncols + 15) / 16;
+  if (rows <= 16 * kGemmFewTiles && (rows + 15) / 16 * ncb <= kGemmFewTiles) {
+    hipLaunchKernelGGL(k_refit_gemm_few, dim3((unsigned)((rows + 15) / 16 * ncb)), dim3(64), 0, s,
+                       A, lda, rows, K, KP, H, np, C, ldc, ncols, C32, ncb);
+    return hipGetLastError();
+  }
   // at most 2^22 tiles (2^30 work-items) per dispatch
   const int64_t chunk = ((int64_t)1 << 22) / (np / kGemmBN) * kGemmBM;
   for (int64_t r0 = 0; r0 < rows; r0 += chunk) {

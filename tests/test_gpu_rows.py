@@ -175,3 +175,20 @@ def test_adjoint_dot_product_across_degrees(tb, q, bc):
     # the velocity cotangent is the sum over substeps: one step's against two
     # half steps' chain is covered elsewhere; here that it is finite and moves
     assert bool(torch.isfinite(grad).all()) and float(grad.abs().max()) > 0
+
+
+@pytest.mark.parametrize("q", [6, 8, 11, 16])
+@pytest.mark.parametrize("depth", [0, 1, 2, 3])
+def test_refit_of_few_rows_has_the_same_bits(tb, q, depth):
+    # 3, 24, 192 and 1,536 rows, by the few-row product up to 2,048 tiles of
+    # 16 x 16, and the same rows within the tiled product of 12,288: sums in
+    # the same order
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(q)
+    v = torch.randn((4096, 3, (q + 1) ** 3), dtype=torch.float64, device="cuda", generator=g)
+    whole = tb.Tree(*tb.uniform_leaves(4), q, 3)
+    whole.set_grid_values(v)
+    few = tb.Tree(*tb.uniform_leaves(depth), q, 3)
+    few.set_grid_values(v[:8 ** depth].contiguous())
+    assert np.array_equal(few.get_coeffs(), whole.get_coeffs()[:8 ** depth])
