@@ -679,15 +679,15 @@ def combined_measure(steps: int = 2, nprob: int = 32):
     return out
 
 
-def traffic_from_profiles(kernel: str, shape: int):
-    """HBM bytes per launch of a kernel at a launch shape from the committed
-    rocprofv3 counter summary (profiles/step_traffic.txt: "kernel shape
+def traffic_from_profiles(kernel: str, threads: int):
+    """HBM bytes per launch of a kernel at a workgroup size from the committed
+    rocprofv3 counter summary (profiles/step_traffic.txt: "kernel threads
     bytes" lines), if measured."""
     p = os.path.join(ROOT, "profiles", "step_traffic.txt")
     try:
         for line in open(p):
             f = line.split()
-            if len(f) == 3 and not line.startswith("#") and f[0] == kernel and int(f[1]) == shape:
+            if len(f) == 3 and not line.startswith("#") and f[0] == kernel and int(f[1]) == threads:
                 return float(f[2])
     except OSError:
         pass
@@ -862,14 +862,13 @@ def main():
         k_s = res[mode]["step_kernel_ms"] * 1e-3
         ach = flops_per_point(Q) * N / k_s / 1e12
         peak = PEAK["fp64" if mode == "fp64" else "fp32"]
-        shape = _lib.step_shape(mode, Q)
-        kname = "k_step" if shape in (0, 1, 2, 3) else "k_step_rg"
-        name = f"{kname}<{kmode[mode]}>"
+        threads = 256 if mode == "fp64" else 512
+        name = f"k_step_rows<{kmode[mode]}>"
         r = {"bound": "valu", "achieved": ach, "peak": peak, "unit": "TFLOP/s",
-             "frac": ach / peak, "traffic": traffic_from_profiles(name, shape),
+             "frac": ach / peak, "traffic": traffic_from_profiles(name, threads),
              "traffic_source": "profiles/step_traffic.txt (rocprofv3 --pmc FETCH_SIZE and "
-                               "WRITE_SIZE of this kernel at this shape, scaled by a 1 GiB copy)",
-             "kernel": name, "launch_shape": shape, "flops_per_point": flops_per_point(Q),
+                               "WRITE_SIZE of this kernel, scaled by a 1 GiB copy)",
+             "kernel": name, "threads": threads, "flops_per_point": flops_per_point(Q),
              "points_per_launch": N, "timing": "HIP events on the launch stream"}
         if mode != "fp64":
             r["peak_note"] = ("published FP32 vector peak, reached only by packed FP32, which "

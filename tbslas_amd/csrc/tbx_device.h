@@ -3,7 +3,8 @@
 // Execution model of the point kernels: one departure point per lane.  A
 // lane finds its leaf (Morton key -> coarse-cell directory -> bounded binary
 // search), maps the point to the leaf's [-1,1]^3 and builds T_0..T_q per
-// axis in registers.  The coefficient contraction then runs as a waterfall
+// axis in registers.  The coefficient contraction of TBX_EXACT (the other
+// modes': tbx_rows.h) then runs as a waterfall
 // over the distinct leaves present in the wavefront: the first active lane's
 // leaf is broadcast (readfirstlane), every lane in that leaf contracts with
 // that leaf's coefficients, which are wave-uniform and therefore fetched by

@@ -554,7 +554,8 @@ hipError_t with_mode(int mode, F f) {
 // the leaf's box from a hash of i; every component of the leaf is
 // contracted there one after another (as in a velocity evaluation) and
 // out[i] = ((0 + u_0) + u_1) + ... .  pts (optional) receives the points.
-// It measures the contraction's own rate, the ceiling of the step's.
+// It measures the rate of the contraction with scalar operands (TBX_EXACT's
+// form, in each mode's arithmetic).
 __device__ __forceinline__ double unit_hash(uint64_t v) {
   v += 0x9E3779B97F4A7C15ull;  // SplitMix64 finaliser
   v = (v ^ (v >> 30)) * 0xBF58476D1CE4E5B9ull;
