@@ -40,7 +40,10 @@ typedef double acc4 __attribute__((ext_vector_type(4)));
 // (KP >= K a multiple of 16, np a multiple of 64).  C32 (may be null)
 // receives C rounded to FP32 with the same layout.  Workgroups are remapped
 // so each XCD runs a contiguous range of tiles (the column tiles of one row
-// block share its A rows in that XCD's L2).
+// block share its A rows in that XCD's L2).  A chunk without a remainder in K
+// is loaded without a test per element: 36,324 rows of degree 14 712 -> 684
+// us (49 TFLOP/s without the padding; a large FP64 matrix product reaches 73
+// here), 262,144 rows of degree 8 474 -> 454 us.
 __global__ __launch_bounds__(kGemmThreads) void k_refit_gemm(
     const double *__restrict__ A, int64_t lda, int64_t rows, int K, int KP,
     const double *__restrict__ H, int np, double *__restrict__ C, int64_t ldc, int ncols,
@@ -65,10 +68,12 @@ __global__ __launch_bounds__(kGemmThreads) void k_refit_gemm(
   const double *ap = A + (arow_ok ? arow : 0) * lda;
   double ra[4], rb[4];
   auto load = [&](int k0) {
+    if (k0 + kGemmBK <= K) {  // whole chunks: wide loads (row 0 past the last)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int k = k0 + ak + u;
-      ra[u] = (arow_ok && k < K) ? ap[k] : 0.0;
+      for (int u = 0; u < 4; ++u) ra[u] = ap[k0 + ak + u];
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) ra[u] = k0 + ak + u < K ? ap[k0 + ak + u] : 0.0;
     }
     const double *hp = H + (int64_t)(k0 + bk) * np + c0 + bc;
 #pragma unroll
