@@ -206,16 +206,22 @@ __device__ __forceinline__ void rows_gradient(AdjLds<BLOCK> &s, const TreeView &
       const bool mine = leaf == lf;
       pending &= ~__builtin_amdgcn_ballot_w64(mine);
       const double *cb = t.coeff + ((size_t)lf * t.dof + c0) * NC + (lane & 15);
+      // summed from zero in each pass: a row that is done goes through its
+      // first lane's leaf again while another row has leaves left
+      double kx = 0.0, ky = 0.0, kz = 0.0;
 #pragma unroll 1
       for (int c = 0; c < nc; ++c) {
         double gx, gy, gz;
         row_grad(cb, px, dx, py, dy, z, gx, gy, gz);
         const double a = s.w[c][src];
-        jx = mine ? __builtin_fma(a, gx, jx) : jx;
-        jy = mine ? __builtin_fma(a, gy, jy) : jy;
-        jz = mine ? __builtin_fma(a, gz, jz) : jz;
+        kx = __builtin_fma(a, gx, kx);
+        ky = __builtin_fma(a, gy, ky);
+        kz = __builtin_fma(a, gz, kz);
         cb += NC;
       }
+      jx = mine ? kx : jx;
+      jy = mine ? ky : jy;
+      jz = mine ? kz : jz;
     }
     s.g[0][src] = in ? jx : 0.0;
     s.g[1][src] = in ? jy : 0.0;
