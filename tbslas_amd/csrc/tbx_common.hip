@@ -2,6 +2,8 @@
 // FP32 coefficient mirror.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "tbx_device.h"
 
 namespace tbx {
@@ -94,24 +96,69 @@ __global__ __launch_bounds__(kBlock) void k_to_f32(const double *__restrict__ in
 
 constexpr int kXcds = 8;
 constexpr int kMetaStride = 32;  // words: a cache line each
+constexpr int kMetaWords = 2 * kMetaStride;  // [0] scattered, [kMetaStride] places taken
 constexpr int kFewLeaves = 1024;
-constexpr int kMetaWords = (1 + kXcds) * kMetaStride;
+constexpr int kProbeBlock = 1024;
+constexpr int kProbes = kProbeBlock / 64;  // a wavefront each
+constexpr int kOrderBlocks = 16384;  // a multiple of kXcds
 
 // Order of a call's points by leaf (counting sort; order_words(n, L) words of
 // scratch): leaf and rank of every point, hist, then perm.  Groups follow
 // each other in no particular order; a point's place in its group depends on
 // the run, its value does not.
 //
+// k_order_begin decides whether there is anything to order, from kProbes
+// windows of 64 consecutive points spread over the call: scattered (meta[0])
+// where more than a quarter of them change leaf eight times or more between
+// neighbours.  Points that come in runs of a leaf are taken as they come
+// (their accesses stay coalesced), and the kernels after this one return at
+// once.  Counting and placing every point before it was known took, for
+// points in leaf order, 20 us and as much again per million: 1 M of them on
+// 512 leaves of degree 8 48 us, now 32; 4 M on 4,096 leaves of degree 4, three
+// components, 123 us, now 71.  Block 0 probes, the others clear the counters.
+__global__ __launch_bounds__(kProbeBlock) void k_order_begin(TreeView t,
+                                                             const double *__restrict__ pts,
+                                                             int64_t n, int bc,
+                                                             int32_t *__restrict__ meta,
+                                                             int64_t words) {
+  if (blockIdx.x > 0) {
+    const int64_t stride = (int64_t)(gridDim.x - 1) * kProbeBlock;
+    for (int64_t i = kMetaStride + (int64_t)(blockIdx.x - 1) * kProbeBlock + threadIdx.x;
+         i < words; i += stride)
+      meta[i] = 0;
+    return;
+  }
+  __shared__ int scattered;
+  if (threadIdx.x == 0) scattered = 0;
+  __syncthreads();
+  const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
+  int64_t i = (n > 64 ? n - 64 : 0) * wave / (kProbes - 1) + lane;
+  i = i < n ? i : n - 1;
+  double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
+  if (bc == TBX_BC_PERIODIC) {
+    x = wrap1(x);
+    y = wrap1(y);
+    z = wrap1(z);
+  }
+  const int lf = locate(t, x, y, z);
+  const int left = __shfl_up(lf, 1, 64);
+  const int changes = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane > 0 && lf != left));
+  if (lane == 0 && changes >= 8) atomicAdd(&scattered, 1);
+  __syncthreads();
+  if (threadIdx.x == 0) meta[0] = 4 * scattered > kProbes;
+}
+
 // k_order_count: rank = the point's number in its leaf.  A wavefront adds
 // once per leaf that several of its lanes share, so that many points of one
 // leaf do not queue on its counter.  Each of the eight XCDs (workgroups go to
-// them in turn) has its own counters, hist[x][L], and its own word of meta,
-// which counts the wavefronts whose neighbouring lanes change leaf eight
-// times or more: a line that the XCDs add to in turn travels between their
-// L2s (1,000,003 scattered points of a call 172 us with one array, 139 with
-// eight).  FEW (L <= kFewLeaves): a workgroup counts in LDS and adds once per
-// leaf, for many points on few leaves would all queue on the same counters
-// (457,182 points on 512 leaves 90 us, 68 in LDS).
+// them in turn) has its own counters, hist[x][L]: a line that the XCDs add to
+// in turn travels between their L2s (1,000,003 scattered points of a call 172
+// us with one array, 139 with eight).  FEW (L <= kFewLeaves): a workgroup
+// counts in LDS and adds once per leaf, for many points on few leaves would
+// all queue on the same counters (457,182 points on 512 leaves 90 us, 68 in
+// LDS).  At most kOrderBlocks workgroups, so that a call whose points are not
+// ordered does not wait for 62,500 empty ones (14 us); tile b of the points
+// is on XCD b % kXcds in any case.
 template <bool FEW>
 __global__ __launch_bounds__(kBlock) void k_order_count(TreeView t,
                                                         const double *__restrict__ pts,
@@ -119,72 +166,68 @@ __global__ __launch_bounds__(kBlock) void k_order_count(TreeView t,
                                                         int32_t *__restrict__ leaf,
                                                         int32_t *__restrict__ rank,
                                                         int32_t *__restrict__ hist,
-                                                        int32_t *__restrict__ meta) {
+                                                        const int32_t *__restrict__ meta) {
+  if (meta[0] == 0) return;
   __shared__ int cnt[FEW ? kFewLeaves : 1];
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const bool live = i < n;
-  const int lane = (int)(threadIdx.x & 63u);
-  int lf = 0;
-  if (live) {
-    double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
-    if (bc == TBX_BC_PERIODIC) {
-      x = wrap1(x);
-      y = wrap1(y);
-      z = wrap1(z);
+  hist += (int)(blockIdx.x % kXcds) * t.L;
+  for (int64_t i0 = (int64_t)blockIdx.x * kBlock; i0 < n; i0 += (int64_t)gridDim.x * kBlock) {
+    const int64_t i = i0 + threadIdx.x;
+    const bool live = i < n;
+    int lf = 0;
+    if (live) {
+      double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
+      if (bc == TBX_BC_PERIODIC) {
+        x = wrap1(x);
+        y = wrap1(y);
+        z = wrap1(z);
+      }
+      lf = locate(t, x, y, z);
     }
-    lf = locate(t, x, y, z);
-  }
-  const int left = __shfl_up(lf, 1, 64);
-  const int changes =
-      __builtin_popcountll(__builtin_amdgcn_ballot_w64(live && lane > 0 && lf != left));
-  const int scattered = __syncthreads_count(lane == 0 && changes >= 8);
-  const int xcd = (int)(blockIdx.x % kXcds);
-  hist += xcd * t.L;
-  if (threadIdx.x == 0 && scattered) atomicAdd(&meta[(1 + xcd) * kMetaStride], scattered);
-  if constexpr (FEW) {
-    for (int l = (int)threadIdx.x; l < t.L; l += kBlock) cnt[l] = 0;
-    __syncthreads();
-    int r = live ? atomicAdd(&cnt[lf], 1) : 0;
-    __syncthreads();
-    for (int l = (int)threadIdx.x; l < t.L; l += kBlock)
-      if (cnt[l]) cnt[l] = atomicAdd(&hist[l], cnt[l]);
-    __syncthreads();
+    int r = 0;
+    if constexpr (FEW) {
+      for (int l = (int)threadIdx.x; l < t.L; l += kBlock) cnt[l] = 0;
+      __syncthreads();
+      if (live) r = atomicAdd(&cnt[lf], 1);
+      __syncthreads();
+      for (int l = (int)threadIdx.x; l < t.L; l += kBlock)
+        if (cnt[l]) cnt[l] = atomicAdd(&hist[l], cnt[l]);
+      __syncthreads();
+      r += cnt[lf];
+      __syncthreads();  // the next tile counts again
+    } else {
+      const int lane = (int)(threadIdx.x & 63u);
+      uint64_t pending = __builtin_amdgcn_ballot_w64(live);
+      bool todo = live;
+      for (int it = 0; it < 3 && pending; ++it) {
+        const int src = __builtin_ctzll(pending);
+        const int k = __builtin_amdgcn_readlane(lf, src);
+        const bool mine = todo && lf == k;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
+        if (__builtin_popcountll(m) < 4) break;
+        int base = 0;
+        if (lane == src) base = atomicAdd(&hist[k], __builtin_popcountll(m));
+        base = __builtin_amdgcn_readlane(base, src);
+        if (mine) {
+          r = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+          todo = false;
+        }
+        pending &= ~m;
+      }
+      if (todo) r = atomicAdd(&hist[lf], 1);
+    }
     if (live) {
       leaf[i] = lf;
-      rank[i] = r + cnt[lf];
+      rank[i] = r;
     }
-    return;
-  }
-  uint64_t pending = __builtin_amdgcn_ballot_w64(live);
-  bool todo = live;
-  int r = 0;
-  for (int it = 0; it < 3 && pending; ++it) {
-    const int src = __builtin_ctzll(pending);
-    const int k = __builtin_amdgcn_readlane(lf, src);
-    const bool mine = todo && lf == k;
-    const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
-    if (__builtin_popcountll(m) < 4) break;
-    int base = 0;
-    if (lane == src) base = atomicAdd(&hist[k], __builtin_popcountll(m));
-    base = __builtin_amdgcn_readlane(base, src);
-    if (mine) {
-      r = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-      todo = false;
-    }
-    pending &= ~m;
-  }
-  if (todo) r = atomicAdd(&hist[lf], 1);
-  if (live) {
-    leaf[i] = lf;
-    rank[i] = r;
   }
 }
 
 // hist[l] = first place of leaf l's points: a wavefront's 64 leaves take
-// their places together.  meta[0]: places taken so far.
+// their places together.
 __global__ __launch_bounds__(kBlock) void k_order_start(int32_t *__restrict__ hist, int64_t L,
                                                         int32_t *__restrict__ meta) {
+  if (meta[0] == 0) return;
   const int64_t l = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int lane = (int)(threadIdx.x & 63u);
   int c = 0;
@@ -197,7 +240,7 @@ __global__ __launch_bounds__(kBlock) void k_order_start(int32_t *__restrict__ hi
     if (lane >= d) incl += o;
   }
   int base = 0;
-  if (lane == 63 && incl) base = atomicAdd(&meta[0], incl);
+  if (lane == 63 && incl) base = atomicAdd(&meta[kMetaStride], incl);
   base = __builtin_amdgcn_readlane(base, 63);
   if (l >= L) return;
   int start = base + incl - c;  // the leaf's places, XCD by XCD
@@ -208,26 +251,18 @@ __global__ __launch_bounds__(kBlock) void k_order_start(int32_t *__restrict__ hi
   }
 }
 
-// perm[place] = point; the identity where the points came in runs of a leaf
-// already (under a quarter of the wavefronts scattered), which keeps their
-// accesses coalesced.
+// perm[place] = point.
 __global__ __launch_bounds__(kBlock) void k_order_place(const int32_t *__restrict__ leaf,
                                                         const int32_t *__restrict__ rank,
                                                         const int32_t *__restrict__ hist,
                                                         const int32_t *__restrict__ meta,
                                                         int64_t n, int64_t L,
                                                         int32_t *__restrict__ perm) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  int64_t waves = 0;
-  for (int x = 0; x < kXcds; ++x) waves += meta[(1 + x) * kMetaStride];
-  const bool scattered = 4 * waves > (n + 63) / 64;
-  perm[scattered ? hist[(blockIdx.x % kXcds) * L + leaf[i]] + rank[i] : i] = (int32_t)i;
-}
-
-__global__ __launch_bounds__(kBlock) void k_zero_words(int32_t *__restrict__ p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) p[i] = 0;
+  if (meta[0] == 0) return;
+  hist += (int)(blockIdx.x % kXcds) * L;
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kBlock)
+    perm[hist[leaf[i]] + rank[i]] = (int32_t)i;
 }
 
 inline unsigned grid_for(int64_t n) {
@@ -248,16 +283,21 @@ hipError_t launch_locate(const TreeView &t, const double *pts, int64_t n,
 int64_t order_words(int64_t n, int64_t L) { return 3 * n + kXcds * L + kMetaWords; }
 
 hipError_t launch_order_points(const TreeView &t, const double *pts, int64_t n, int bc,
-                               int32_t *words, int32_t **perm, hipStream_t s) {
+                               int32_t *words, PointPerm *perm, hipStream_t s) {
   int32_t *leaf = words, *rank = leaf + n, *meta = rank + n, *hist = meta + kMetaWords;
-  *perm = hist + kXcds * t.L;
-  const int64_t zero = kXcds * t.L + kMetaWords;
-  hipLaunchKernelGGL(k_zero_words, dim3(grid_for(zero)), dim3(kBlock), 0, s, meta, zero);
-  hipLaunchKernelGGL(t.L <= kFewLeaves ? k_order_count<true> : k_order_count<false>,
-                     dim3(grid_for(n)), dim3(kBlock), 0, s, t, pts, n, bc, leaf, rank, hist, meta);
+  perm->use = meta;
+  perm->perm = hist + kXcds * t.L;
+  const int64_t clear = kXcds * t.L + kMetaWords;
+  const unsigned grid = std::min<unsigned>(grid_for(n), kOrderBlocks);
+  hipLaunchKernelGGL(k_order_begin,
+                     dim3(1 + (unsigned)std::min<int64_t>((clear + 4 * kProbeBlock - 1) /
+                                                              (4 * kProbeBlock), kOrderBlocks)),
+                     dim3(kProbeBlock), 0, s, t, pts, n, bc, meta, clear);
+  hipLaunchKernelGGL(t.L <= kFewLeaves ? k_order_count<true> : k_order_count<false>, dim3(grid),
+                     dim3(kBlock), 0, s, t, pts, n, bc, leaf, rank, hist, meta);
   hipLaunchKernelGGL(k_order_start, dim3(grid_for(t.L)), dim3(kBlock), 0, s, hist, t.L, meta);
-  hipLaunchKernelGGL(k_order_place, dim3(grid_for(n)), dim3(kBlock), 0, s, leaf, rank, hist,
-                     meta, n, t.L, *perm);
+  hipLaunchKernelGGL(k_order_place, dim3(grid), dim3(kBlock), 0, s, leaf, rank, hist, meta, n,
+                     t.L, const_cast<int32_t *>(perm->perm));
   return hipGetLastError();
 }
 

@@ -482,7 +482,7 @@ int prepare_view(tbx_tree *t, int mode, hipStream_t s, ScratchArena *arena, Tree
   X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16)
 
 hipError_t dispatch_eval(int q, int mode, const TreeView &t, double *pts,
-                         int64_t n, int bc, int wb, double *out, const int32_t *perm,
+                         int64_t n, int bc, int wb, double *out, PointPerm perm,
                          hipStream_t s) {
   switch (q) {
 #define X(Q) \
@@ -520,7 +520,7 @@ hipError_t dispatch_veval(int q, int mode, const VelSource &vel, double *pts, in
 }
 
 hipError_t dispatch_traj(int q, int mode, const VelSource &vel, const double *x0, double *x,
-                         int64_t n, const SubArgs &a, const int32_t *perm, hipStream_t s) {
+                         int64_t n, const SubArgs &a, PointPerm perm, hipStream_t s) {
   switch (q) {
 #define X(Q) \
   case Q:    \
@@ -582,15 +582,28 @@ int check_bc(int bc) {
   return TBX_OK;
 }
 
-// Scratch of one call, stream-ordered: from a pool per device that keeps up
-// to kPoolKeep bytes between calls (a plain hipMallocAsync returns its memory
-// to the system at the next synchronisation) and gives them back when the
-// device's last tree is destroyed.  Safe from several threads and streams.
+// Scratch of calls, stream-ordered: from a pool per device, and kept between
+// calls up to kPoolKeep bytes (a plain hipMallocAsync returns its memory to
+// the system at the next synchronisation, and hipFreeAsync takes 9 us of the
+// host).  A block goes to the next call on its stream, which waits for the
+// event recorded behind the last call's kernels (done already where the
+// stream is the same; not where the handle is a new stream's).  Given back
+// when the device's last tree is destroyed.  Safe from several threads and
+// streams.
 constexpr uint64_t kPoolKeep = (uint64_t)256 << 20;
+constexpr size_t kPoolBlocks = 32;
+struct PoolBlock {
+  void *mem = nullptr;
+  size_t bytes = 0;
+  hipStream_t stream = nullptr;
+  hipEvent_t done = nullptr;
+};
 std::mutex g_pool_mu;
 struct DevicePool {
   hipMemPool_t pool = nullptr;
   int64_t trees = 0;
+  std::vector<PoolBlock> idle;  // the longest idle first
+  size_t idle_bytes = 0;
 };
 std::map<int, DevicePool> g_pools;
 
@@ -598,18 +611,32 @@ void pool_tree_count(int device, int change) {
   std::lock_guard<std::mutex> lk(g_pool_mu);
   DevicePool &p = g_pools[device];
   p.trees += change;
-  if (p.trees == 0 && p.pool) (void)hipMemPoolTrimTo(p.pool, 0);
+  if (p.trees == 0 && p.pool) {
+    for (const PoolBlock &b : p.idle) {
+      (void)hipFree(b.mem);
+      (void)hipEventDestroy(b.done);
+    }
+    p.idle.clear();
+    p.idle_bytes = 0;
+    (void)hipMemPoolTrimTo(p.pool, 0);
+  }
 }
 
-// null without an error message where the memory is not to be had.
-void *pool_alloc(size_t bytes, hipStream_t s) {
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess) return nullptr;
+// mem stays null, without an error message, where there is no memory.
+PoolBlock pool_take(int device, size_t bytes, hipStream_t s) {
+  PoolBlock b;
   hipMemPool_t pool;
   {
     std::lock_guard<std::mutex> lk(g_pool_mu);
     DevicePool &p = g_pools[device];
-    if (!p.pool) {
+    for (size_t k = p.idle.size(); k-- > 0;)
+      if (p.idle[k].stream == s && p.idle[k].bytes >= bytes) {
+        b = p.idle[k];
+        p.idle.erase(p.idle.begin() + k);
+        p.idle_bytes -= b.bytes;
+        break;
+      }
+    if (!b.mem && !p.pool) {
       hipMemPoolProps props{};
       props.allocType = hipMemAllocationTypePinned;
       props.location.type = hipMemLocationTypeDevice;
@@ -619,17 +646,56 @@ void *pool_alloc(size_t bytes, hipStream_t s) {
           hipMemPoolSetAttribute(p.pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
         (void)hipGetLastError();
         p.pool = nullptr;
-        return nullptr;
+        return b;
       }
+      p.idle.reserve(kPoolBlocks + 1);
     }
     pool = p.pool;
   }
-  void *m = nullptr;
-  if (hipMallocFromPoolAsync(&m, bytes, pool, s) != hipSuccess) {
+  if (b.mem) {
+    if (hipStreamWaitEvent(s, b.done, 0) == hipSuccess) return b;
     (void)hipGetLastError();
-    return nullptr;
+    (void)hipEventSynchronize(b.done);
+    return b;
   }
-  return m;
+  b.stream = s;
+  b.bytes = bytes;
+  if (hipEventCreateWithFlags(&b.done, hipEventDisableTiming) != hipSuccess ||
+      hipMallocFromPoolAsync(&b.mem, bytes, pool, s) != hipSuccess) {
+    (void)hipGetLastError();
+    if (b.done) (void)hipEventDestroy(b.done);
+    return PoolBlock{};
+  }
+  return b;
+}
+
+// Back from a call on b.stream, whose kernels may still run.  The longest
+// idle blocks beyond the bounds are freed behind their own last call.
+void pool_give(int device, const PoolBlock &b) {
+  if (hipEventRecord(b.done, b.stream) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipFreeAsync(b.mem, b.stream);
+    (void)hipEventDestroy(b.done);
+    return;
+  }
+  for (bool first = true;; first = false) {
+    PoolBlock gone;
+    {
+      std::lock_guard<std::mutex> lk(g_pool_mu);
+      DevicePool &p = g_pools[device];
+      if (first) {
+        p.idle.push_back(b);
+        p.idle_bytes += b.bytes;
+      }
+      if (p.idle.size() <= kPoolBlocks && p.idle_bytes <= kPoolKeep) return;
+      gone = p.idle.front();
+      p.idle_bytes -= gone.bytes;
+      p.idle.erase(p.idle.begin());
+    }
+    (void)hipStreamWaitEvent(b.stream, gone.done, 0);
+    (void)hipFreeAsync(gone.mem, b.stream);
+    (void)hipEventDestroy(gone.done);
+  }
 }
 
 bool capturing(hipStream_t s) {
@@ -642,37 +708,43 @@ bool capturing(hipStream_t s) {
 }
 
 // The order by leaf of n points that `evals` components are evaluated at,
-// where it pays: perm stays null, and the points are taken as they come,
+// where it pays; the points are taken as they come
 //  - in TBX_EXACT (its kernels take points as they come);
-//  - under kOrderWork multiply-adds in all (ordering costs some 15 us of
-//    launches and 30 us per million points), or fewer than two points a
-//    leaf (nothing to bring together);
+//  - under kOrderPoint multiply-adds a point (4,096 leaves, scattered: 4 M
+//    points of degree 4, 35 a point, 209 us, ordered 339; 8 M of degree 3 and
+//    three components, 60 a point, 614 us, ordered 756; but 4 M of degree 4
+//    and three, 105 a point, 445 us, ordered 360) or kOrderWork in all (60,000
+//    points of degree 14 on 512 leaves, 4e7 in all: scattered 76 us, ordered
+//    27; in leaf order 10 us, 22 with the launches that find them so), or
+//    with fewer than two points a leaf (nothing to bring together);
 //  - on few leaves, which a workgroup orders by itself with little padding:
 //    up to 16 always (degree 14, 8 leaves: 1.5 M points 109 us, ordered first
 //    132; 60,007 points 16, ordered 44), up to 64 under 600 multiply-adds a
 //    point (64 leaves, degree 6, 2 M points 70 us, ordered 125; but degree
 //    14, 1.5 M points 235 us, ordered 131, and trajectories of degree 10,
 //    60,007 points 225 us, ordered 64);
+//  - where they come in runs of a leaf already (k_order_begin);
 //  - on a stream that is being captured (nothing is allocated there), and
 //    without memory for it.
 constexpr double kOrderWork = 3e7;
+constexpr double kOrderPoint = 80;
 struct PointOrder {
-  void *words = nullptr;
-  int32_t *perm = nullptr;
-  hipStream_t s = nullptr;
+  PointPerm perm{nullptr, nullptr};
+  PoolBlock block;
+  int device = 0;
   hipError_t make(const tbx_tree *t, const double *pts, int64_t n, int bc, int mode, double evals,
                   hipStream_t st) {
+    const double work = evals * t->nc;
     if (mode == kExact64 || n < 2 * t->L || n > INT32_MAX || t->L <= 16 ||
-        (t->L <= 64 && evals * t->nc < 600) ||
-        (double)n * evals * t->nc < kOrderWork || capturing(st))
+        (t->L <= 64 && work < 600) || work < kOrderPoint || (double)n * work < kOrderWork ||
+        capturing(st) || hipGetDevice(&device) != hipSuccess)
       return hipSuccess;
-    words = pool_alloc(sizeof(int32_t) * (size_t)order_words(n, t->L), st);
-    if (!words) return hipSuccess;
-    s = st;
-    return launch_order_points(t->view(), pts, n, bc, (int32_t *)words, &perm, st);
+    block = pool_take(device, sizeof(int32_t) * (size_t)order_words(n, t->L), st);
+    if (!block.mem) return hipSuccess;
+    return launch_order_points(t->view(), pts, n, bc, (int32_t *)block.mem, &perm, st);
   }
   ~PointOrder() {
-    if (words) (void)hipFreeAsync(words, s);
+    if (block.mem) pool_give(device, block);
   }
 };
 
@@ -1504,7 +1576,7 @@ int tbx_adjoint_run(const tbx_tree *vel, tbx_tfac_fn g, void *gctx, tbx_tree *co
     auto forward = [&](int n, double *dep) -> int {
       if (stationary && keep_dep && have_dep && conc->dof == 1) {
         HIP_TRY(dispatch_eval(conc->q, c.mode, conc->view(), deps[0], (int64_t)conc->L * conc->P(),
-                              bc, 0, conc->d_vals, nullptr, st));
+                              bc, 0, conc->d_vals, PointPerm{}, st));
         return refit(conc, conc->d_vals, st);
       }
       const int r = step_insitu(&v, conc, n, dt, 1, bc, flags, dep, st, "tbx_adjoint_run");
@@ -2333,7 +2405,7 @@ int tbx_check_cheb_output(const tbx_tree *tc, const double *ref, uint32_t flags,
     double x[TBX_MAX_Q + 1];
     first_kind_nodes_host(n, x);
     HIP_TRY(launch_grid_points(t->view(), x, n, pts, st));
-    HIP_TRY(dispatch_eval(t->q, mode, t->view(), pts, npts, TBX_BC_FREESPACE, 0, val, nullptr,
+    HIP_TRY(dispatch_eval(t->q, mode, t->view(), pts, npts, TBX_BC_FREESPACE, 0, val, PointPerm{},
                           st));
     std::vector<double> h((size_t)nb * std::max(dof, 4));
     // pass 0: the volume-weighted mean error per component (utils.txx:158-187)
@@ -2868,7 +2940,7 @@ int tbx_tree_write_vtu(const tbx_tree *tc, const char *prefix, int order, tbx_st
     HIP_TRY(hipMallocAsync((void **)&pts, sizeof(double) * 3 * (size_t)npts, st));
     HIP_TRY(hipMallocAsync((void **)&val, sizeof(double) * t->dof * (size_t)npts, st));
     HIP_TRY(launch_grid_points(t->view(), node, n, pts, st));
-    HIP_TRY(dispatch_eval(t->q, kFma64, t->view(), pts, npts, TBX_BC_FREESPACE, 0, val, nullptr,
+    HIP_TRY(dispatch_eval(t->q, kFma64, t->view(), pts, npts, TBX_BC_FREESPACE, 0, val, PointPerm{},
                           st));
     HIP_TRY(hipMemcpyAsync(hval.data(), val, sizeof(double) * hval.size(), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));

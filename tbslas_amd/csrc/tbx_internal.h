@@ -130,14 +130,21 @@ constexpr int kBlock = 256;
 constexpr int rows_step_block(int mode) { return mode == kFma64 ? 256 : 512; }
 constexpr int kAdjBlock = 256;  // workgroup of the adjoint concentration kernel
 
+// The order in which a call's points are taken: perm lists them, those of a
+// leaf together, where *use is set (on the device, from the points); as they
+// come where it is not, or perm is null.
+struct PointPerm {
+  const int32_t *perm, *use;
+};
+
 // Launchers instantiated once per degree Q (tbx_kernels.hip, -DTBX_Q=Q).
 #define TBX_DECLARE_Q(Q)                                                      \
   hipError_t launch_eval_q##Q(int mode, const TreeView &t, double *pts,       \
                               int64_t n, int bc, int write_back, double *out, \
-                              const int32_t *perm, hipStream_t s);            \
+                              PointPerm perm, hipStream_t s);                 \
   hipError_t launch_traj_q##Q(int mode, const VelSource &vel,                 \
                               const double *x0, double *x, int64_t n,         \
-                              const SubArgs &a, const int32_t *perm,          \
+                              const SubArgs &a, PointPerm perm,               \
                               hipStream_t s);                                 \
   hipError_t launch_step_q##Q(int mode, const VelSource &vel,                 \
                               const TreeView &conc, const StepArgs &a,        \
@@ -283,11 +290,11 @@ hipError_t launch_gather_rows(const double *src, const int64_t *map, int64_t nro
                               double *dst, hipStream_t s);
 
 // Degree-independent launchers (tbx_common.hip).
-// Order of n points by leaf: *perm (inside words, order_words(n, L) 32-bit
-// words) lists the points, those of a leaf together.  n < 2^31.
+// Order of n points by leaf in words, order_words(n, L) 32-bit words.
+// n < 2^31.
 int64_t order_words(int64_t n, int64_t L);
 hipError_t launch_order_points(const TreeView &t, const double *pts, int64_t n, int bc,
-                               int32_t *words, int32_t **perm, hipStream_t s);
+                               int32_t *words, PointPerm *perm, hipStream_t s);
 hipError_t launch_locate(const TreeView &t, const double *pts, int64_t n,
                          int bc, int32_t *leaf, hipStream_t s);
 hipError_t launch_grid_points(const TreeView &t, const double *node, int d,

@@ -94,17 +94,17 @@ __global__ __launch_bounds__(kBlock) void k_traj_exact(VelSource vel, const doub
 
 // The same three in the other modes: a workgroup's points ordered by leaf
 // and contracted row by row (tbx_rows.h).  Threads past the last point hold
-// a copy of it and take no part.  BLOCK: with_rows_block.  perm (may be
-// null): the order of the points, those of a leaf together.
+// a copy of it and take no part.  BLOCK: with_rows_block.
 template <int MODE, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_eval(
     TreeView t, double *__restrict__ pts, int64_t n, int bc, int write_back,
-    double *__restrict__ out, const int32_t *__restrict__ perm) {
+    double *__restrict__ out, PointPerm perm) {
   __shared__ RowsLds<BLOCK> sh;
   const int64_t i0 = (int64_t)blockIdx.x * BLOCK;
   const bool live = i0 + (int)threadIdx.x < n;
   int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
-  if (perm) i = perm[i];
+  const bool ordered = perm.perm && *perm.use;
+  if (ordered) i = perm.perm[i];
   double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
   if (bc == TBX_BC_PERIODIC) {
     x = wrap1(x);
@@ -117,11 +117,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
     }
   }
   const int lf = locate(t, x, y, z);
-  const int count = order_by_leaf(sh, live, lf);
   double *o = out + i * t.dof;
-  rows_dof<D, MODE>(sh, t, count, lf, x, y, z, [&](int l, double v) {
+  auto store = [&](int l, double v) {
     if (live) o[l] = v;
-  });
+  };
+  // In place only up to three components (200,000 points of degree 4, 16
+  // components: 51 us in order, 69 in place), and not for points taken
+  // through perm, whose components are stored together (4 M of degree 4,
+  // three: 360 us, in place 406).
+  if constexpr (BLOCK == 256) {
+    if (!ordered && t.dof <= 3 && rows_in_place(lf)) {
+      in_place_dof<D, MODE>(t, lf, x, y, z, store);
+      return;
+    }
+  }
+  const int count = order_by_leaf(sh, live, lf);
+  rows_dof<D, MODE>(sh, t, count, lf, x, y, z, store);
 }
 
 template <int MODE, int KIND, int BLOCK>
@@ -156,12 +167,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
 template <int MODE, int KIND, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_traj(
     VelSource vel, const double *x0, double *xs, int64_t n, SubArgs a,
-    const int32_t *__restrict__ perm) {
+    PointPerm perm) {
   __shared__ RowsLds<BLOCK> sh;
   const int64_t i0 = (int64_t)blockIdx.x * BLOCK;
   const bool live = i0 + (int)threadIdx.x < n;
   int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
-  if (perm) i = perm[i];
+  if (perm.perm && *perm.use) i = perm.perm[i];
   double x = x0[3 * i + 0], y = x0[3 * i + 1], z = x0[3 * i + 2];
 #pragma unroll 1
   for (int s = 0; s < a.nsub; ++s)
@@ -694,7 +705,7 @@ hipError_t launch_step_mode(const VelSource &vel, const TreeView &conc, const St
 hipError_t TBX_CAT(launch_eval_q, TBX_Q)(int mode, const TreeView &t,
                                          double *pts, int64_t n, int bc,
                                          int write_back, double *out,
-                                         const int32_t *perm, hipStream_t s) {
+                                         PointPerm perm, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   return with_mode(mode, [&](auto m) {
     constexpr int M = decltype(m)::value;
@@ -749,7 +760,7 @@ hipError_t TBX_CAT(launch_veval_q, TBX_Q)(int mode, const VelSource &vel,
 hipError_t TBX_CAT(launch_traj_q, TBX_Q)(int mode, const VelSource &vel,
                                          const double *x0, double *x,
                                          int64_t n, const SubArgs &a,
-                                         const int32_t *perm, hipStream_t s) {
+                                         PointPerm perm, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   return with_mode(mode, [&](auto m) {
     return with_kind(vel.kind, [&](auto k) {

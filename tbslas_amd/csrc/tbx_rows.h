@@ -569,6 +569,52 @@ __device__ __forceinline__ void rows_dof(RowsLds<BLOCK> &s, const TreeView &t, i
   }
 }
 
+// Whether the 16 lanes of every DPP row of the workgroup hold points of at
+// most two leaves, the row's first lane's and its last's: points that come in
+// runs of a leaf.  They are contracted as they come (in_place_dof): the order
+// in LDS, its barriers and the second round that its padding takes bring such
+// points nothing (1 M of them on 512 leaves of degree 8 24.0 us, in place
+// 20; 16 M of degree 1 141 us, in place 118).  All threads of the workgroup
+// must call it.
+__device__ __forceinline__ bool rows_in_place(int leaf) {
+  const int lane = (int)(threadIdx.x & 63u);
+  const int first = __builtin_amdgcn_ds_bpermute((lane & 48) << 2, leaf);
+  const int last = __builtin_amdgcn_ds_bpermute((lane | 15) << 2, leaf);
+  return !__syncthreads_or(leaf != first && leaf != last);
+}
+
+// All components of t at the thread's point, contracted in its own lane, each
+// through store(l, value): the bits of rows_dof.
+template <int D, int MODE, typename Store>
+__device__ __forceinline__ void in_place_dof(const TreeView &t, int leaf, double x, double y,
+                                             double z, Store store) {
+  using T = typename ModeType<MODE>::T;
+  constexpr int NC = D * (D + 1) * (D + 2) / 6;
+  double ex, ey, ez;
+  leaf_xi(t, leaf, x, y, z, ex, ey, ez);
+  const bool in = fabs(ex) <= 1.0 && fabs(ey) <= 1.0 && fabs(ez) <= 1.0;
+  T px[D], py[D];
+  row_cheb<D>(in ? ex : 0.0, px);
+  row_cheb<D>(in ? ey : 0.0, py);
+  const double zx = in ? ez : 0.0;
+  uint64_t pending = __builtin_amdgcn_ballot_w64(true);
+#pragma unroll 1
+  while (pending) {
+    const int lf = row_leaf(pending, leaf);
+    const bool mine = leaf == lf;
+    pending &= ~__builtin_amdgcn_ballot_w64(mine);
+    const T *cb = coeff_base<MODE>(t) + (size_t)lf * t.dof * NC + (threadIdx.x & 15);
+#pragma unroll 1
+    for (int l = 0; l < t.dof; ++l) {
+      double u = (double)row_contract<D, MODE == kFp32h>(cb, px, py, zx);
+      u = in ? u : 0.0;
+      if constexpr (MODE == kFp32h) u += head_value<D>(t, l, leaf, ex, ey, ez);
+      if (mine) store(l, u);
+      cb += NC;
+    }
+  }
+}
+
 // eval_velocity for a workgroup: the functor at the active threads' points,
 // ordered by their leaves in the first tree (hint0: the thread's point's).
 // Idle threads' values are not defined.
