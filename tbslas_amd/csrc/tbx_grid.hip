@@ -53,8 +53,8 @@ __device__ __forceinline__ void row_samples(const T *p, T (&r)[4]) {
 // All dof components of a leaf at (x, y, z) through store(c, value): inf is
 // the leaf's anchor and depth, data its samples [dof][N^3] (FP32 samples for
 // kFp32, FP64 otherwise), in global memory or in LDS.
-// U2: planes of 16 samples unrolled.  From global memory (grid_unroll) the 64-
-// bit modes take one at a time: 93 registers, five waves per SIMD; with every
+// U2: planes of 16 samples unrolled.  From global memory (with_grid_mode) the
+// 64-bit modes take one at a time: 93 registers, five waves per SIMD; with every
 // gather of the 64 issued up front (223 registers, two waves) the step on
 // 32,768 leaves of 8^3 samples took 1.81 ms in FP64, now 1.73, the evaluation
 // of as many points 0.54, now 0.44, and the two in TBX_EXACT 5.08, now 3.18.
@@ -64,11 +64,6 @@ __device__ __forceinline__ void row_samples(const T *p, T (&r)[4]) {
 // whether in 8- or 16-byte loads.  The sibling blocks, whose gathers are from
 // LDS but for the points outside, take one at a time everywhere (FP32, 4,096
 // leaves of 8^3: 206 us; four outside, 290).
-template <int MODE>
-constexpr int grid_unroll() {
-  return MODE == kFp32 ? 4 : 1;
-}
-
 template <int MODE, int U2, typename T, typename Store>
 __device__ __forceinline__ void grid_interp_at(const uint4 inf, const T *data, int N, int dof,
                                                double x, double y, double z, Store store) {
@@ -157,7 +152,7 @@ __device__ __forceinline__ void grid_interp_at(const uint4 inf, const T *data, i
   }
 }
 
-template <int MODE, int U2 = grid_unroll<MODE>(), typename Store>
+template <int MODE, int U2, typename Store>
 __device__ __forceinline__ void grid_interp(const TreeView &t, const GridData &g, int leaf,
                                             double x, double y, double z, Store store) {
   const int64_t off = (int64_t)leaf * g.dof * g.n * g.n * g.n;
@@ -167,12 +162,12 @@ __device__ __forceinline__ void grid_interp(const TreeView &t, const GridData &g
     grid_interp_at<MODE, U2>(t.info[leaf], g.s + off, g.n, g.dof, x, y, z, store);
 }
 
-template <int MODE>
+template <int MODE, int U2>
 __device__ __forceinline__ void grid_vel(const TreeView &t, const GridData &g, double x,
                                          double y, double z, int scaled, double f, double &v0,
                                          double &v1, double &v2) {
   const int leaf = locate(t, x, y, z);
-  grid_interp<MODE>(t, g, leaf, x, y, z, [&](int c, double v) {
+  grid_interp<MODE, U2>(t, g, leaf, x, y, z, [&](int c, double v) {
     if (c == 0) v0 = v;
     else if (c == 1) v1 = v;
     else v2 = v;
@@ -211,7 +206,7 @@ __device__ __forceinline__ bool grid_node_velocity(const TreeView &tv, const T *
   return true;
 }
 
-template <int MODE>
+template <int MODE, int U2>
 __global__ __launch_bounds__(kBlock) void k_grid_eval(TreeView t, GridData g,
                                                       double *__restrict__ pts, int64_t n,
                                                       int bc, int write_back,
@@ -231,13 +226,13 @@ __global__ __launch_bounds__(kBlock) void k_grid_eval(TreeView t, GridData g,
   }
   const int leaf = locate(t, x, y, z);
   double *o = out + i * g.dof;
-  grid_interp<MODE>(t, g, leaf, x, y, z, [&](int c, double v) { o[c] = v; });
+  grid_interp<MODE, U2>(t, g, leaf, x, y, z, [&](int c, double v) { o[c] = v; });
 }
 
 // SolveSemilagInSitu for grid leaves, fused: sample point -> num_rk_step
 // RK2 substeps through the velocity grid tree (traj.inc:20-68) -> conc at
 // the departure point -> out[leaf][c][sample].
-template <int MODE>
+template <int MODE, int U2>
 __global__ __launch_bounds__(kBlock) void k_grid_step(TreeView tv, GridData vel, TreeView tc,
                                                       GridData conc, GridStepArgs a,
                                                       double *__restrict__ out,
@@ -270,14 +265,14 @@ __global__ __launch_bounds__(kBlock) void k_grid_step(TreeView tv, GridData vel,
         nodal = grid_node_velocity(tv, vel.s, lf, inf, (int)m, N, lf, a.scaled, a.g[0], v0, v1,
                                    v2);
     }
-    if (!nodal) grid_vel<MODE>(tv, vel, x, y, z, a.scaled, a.g[2 * s], v0, v1, v2);
+    if (!nodal) grid_vel<MODE, U2>(tv, vel, x, y, z, a.scaled, a.g[2 * s], v0, v1, v2);
     double hx = x + a.htau * v0, hy = y + a.htau * v1, hz = z + a.htau * v2;  // traj.inc:36
     if (a.bc == TBX_BC_PERIODIC) {
       hx = wrap1(hx);
       hy = wrap1(hy);
       hz = wrap1(hz);
     }
-    grid_vel<MODE>(tv, vel, hx, hy, hz, a.scaled, a.g[2 * s + 1], v0, v1, v2);
+    grid_vel<MODE, U2>(tv, vel, hx, hy, hz, a.scaled, a.g[2 * s + 1], v0, v1, v2);
     x = x + a.tau * v0;  // traj.inc:41-42
     y = y + a.tau * v1;
     z = z + a.tau * v2;
@@ -294,7 +289,7 @@ __global__ __launch_bounds__(kBlock) void k_grid_step(TreeView tv, GridData vel,
   }
   const int cl = locate(tc, x, y, z);
   double *o = out + leaf * conc.dof * N3 + m;
-  grid_interp<MODE>(tc, conc, cl, x, y, z, [&](int c, double v) { o[c * N3] = v; });
+  grid_interp<MODE, U2>(tc, conc, cl, x, y, z, [&](int c, double v) { o[c * N3] = v; });
 }
 
 // The same step for a uniform tree of 8^3-sample leaves whose velocity and
@@ -416,19 +411,33 @@ __global__ __launch_bounds__(kBlkThreads) void k_grid_step_blk(TreeView tv, Grid
   }
 }
 
+// Calls f with the arithmetic mode and the planes unrolled, four where few is
+// set or the mode is kFp32.
 template <typename F>
-hipError_t with_grid_mode(int mode, F f) {
+hipError_t with_grid_mode(int mode, bool few, F f) {
+  using One = std::integral_constant<int, 1>;
+  using Four = std::integral_constant<int, 4>;
+  const std::integral_constant<int, kFma64> fma64;
+  const std::integral_constant<int, kExact64> exact;
   switch (mode) {
     case kFma64:
-      return f(std::integral_constant<int, kFma64>{});
+      return few ? f(fma64, Four{}) : f(fma64, One{});
     case kExact64:
-      return f(std::integral_constant<int, kExact64>{});
+      return few ? f(exact, Four{}) : f(exact, One{});
     case kFp32:
-      return f(std::integral_constant<int, kFp32>{});
+      return f(std::integral_constant<int, kFp32>{}, Four{});
     default:
       return hipErrorInvalidValue;
   }
 }
+
+// Points of a step up to which the 64-bit modes issue every gather up front:
+// a workgroup per compute unit, which has registers to spare and waits for
+// each plane in turn (64 leaves of 10^3 samples 15.0 us one plane at a time,
+// 13.3 all four; 512 of 5^3 15.2 and 13.6; from 131,072 points on one is the
+// faster).  TBX_EXACT with several components is at or below the latter's
+// times with one.
+constexpr int64_t kFewPoints = 256 * kBlock;
 
 }  // namespace
 
@@ -437,8 +446,8 @@ hipError_t launch_grid_eval(int mode, const TreeView &t, const double *s, const 
                             double *out, hipStream_t st) {
   if (npts <= 0) return hipSuccess;
   const GridData g{s, s32, n, dof};
-  return with_grid_mode(mode, [&](auto md) {
-    hipLaunchKernelGGL(k_grid_eval<decltype(md)::value>,
+  return with_grid_mode(mode, false, [&](auto md, auto u2) {
+    hipLaunchKernelGGL((k_grid_eval<decltype(md)::value, decltype(u2)::value>),
                        dim3((unsigned)((npts + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, t, g,
                        pts, npts, bc, write_back, out);
     return hipGetLastError();
@@ -455,14 +464,15 @@ hipError_t launch_grid_step(int mode, const TreeView &tv, const double *vs, cons
     if (vn != 8 || cn != 8 || cdof != 1 || a.npts % (kBlkLeaves * kBlkN3))
       return hipErrorInvalidValue;
     const int64_t nb = a.npts / (kBlkLeaves * kBlkN3);
-    return with_grid_mode(mode, [&](auto md) {
+    return with_grid_mode(mode, false, [&](auto md, auto) {
       hipLaunchKernelGGL(k_grid_step_blk<decltype(md)::value>, dim3((unsigned)nb),
                          dim3(kBlkThreads), 0, st, tv, vel, tc, conc, a, out, dep);
       return hipGetLastError();
     });
   }
-  return with_grid_mode(mode, [&](auto md) {
-    hipLaunchKernelGGL(k_grid_step<decltype(md)::value>,
+  const bool few = a.npts <= kFewPoints && (mode == kFma64 || cdof == 1);
+  return with_grid_mode(mode, few, [&](auto md, auto u2) {
+    hipLaunchKernelGGL((k_grid_step<decltype(md)::value, decltype(u2)::value>),
                        dim3((unsigned)((a.npts + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, tv,
                        vel, tc, conc, a, out, dep);
     return hipGetLastError();
