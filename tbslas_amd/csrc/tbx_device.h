@@ -375,11 +375,6 @@ __host__ __device__ constexpr int tri_start(int D, int i, int j) {
   return (D * (D + 1) * (D + 2) - n * (n + 1) * (n + 2)) / 6 + j * n - j * (j - 1) / 2;
 }
 
-template <typename T>
-__device__ __forceinline__ T load_uniform(const T *p) {
-  return *(const __attribute__((address_space(4))) T *)(p);
-}
-
 // The head of one leaf's contraction in FP64: the terms with
 // i + j + k <= kHeadDeg, nested as the full contraction (k, then j, then i),
 // from the FP64 coefficients (wave-uniform: scalar loads).  load() reads

@@ -20,7 +20,8 @@ constexpr int D = TBX_Q + 1;
 
 // Waves per SIMD asked of the row kernels: the basis in registers, 2 D
 // values, leaves FP64 four up to degree 9 and three above, FP32 five and
-// four, without spills.
+// four.  Nothing is spilled but in the step through four velocity trees (2 to
+// 12 vector registers, by degree and mode).
 constexpr int rows_waves(int mode) {
   return mode == kFma64 ? (TBX_Q <= 9 ? 4 : 3) : (TBX_Q <= 9 ? 5 : 4);
 }
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
   xs[3 * i + 2] = z;
 }
 
-// SolveSemilagInSitu fused (tree_semilag.h:92-135): arrival point of
+// SolveSemilagInSitu fused (tree_semilag.h:92-135), TBX_EXACT's: arrival point of
 // (leaf, node) -> num_rk_step RK2 substeps through vel -> conc at the
 // departure point -> vals[leaf][l][node] for the refit.  Workgroups are
 // remapped so that each XCD runs a contiguous range of arrival points and a
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
 // minimum waves per SIMD the register budget must allow) select the launch
 // shape: wide workgroups keep the waves resident on a CU inside one or two
 // leaves, so their scalar coefficient loads hit the same cache lines.
-template <int MODE, int KIND, int BLOCK, int WPE>
+template <int KIND, int BLOCK, int WPE>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step(
     VelSource vel, TreeView conc, StepArgs a, double *__restrict__ vals,
     double *__restrict__ dep) {
@@ -210,27 +211,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
   double y = (double)inf.y * len + len * a.node[(m / D) % D];
   double z = (double)inf.z * len + len * a.node[m / (D * D)];
   // ComputeTrajRK2 (traj.inc:48-68), tinit -> tfinal = tinit - dt
-  int s = 0;
-  if constexpr (KIND == kVelTree || KIND == kVelExtrap) {
-    if (a.vnode) {  // the first stage at the arrival node from the nodal values
-      if (a.bc == TBX_BC_PERIODIC) {
-        x = wrap1(x);
-        y = wrap1(y);
-        z = wrap1(z);
-      }
-      const int lf = locate(vel.t[0], x, y, z);
-      double v0, v1, v2;
-      if (!nodal_velocity<D>((const NodalT<MODE> *)a.vnode, vel.t[0], inf, m, lf, a.P, a.scaled, a.g[0], v0, v1, v2))
-        eval_velocity<D, MODE, KIND>(vel, 1, a.ts[0], a.scaled, a.g[0], a.bc, x, y, z, v0, v1,
-                                     v2, lf);
-      rk2_finish<D, MODE, KIND>(vel, a.bc, a.htau, a.tau, a.scaled, a.g[1], a.ts[1], x, y, z,
-                                v0, v1, v2);
-      s = 1;
-    }
-  }
-  for (; s < a.nsub; ++s)
-    rk2_substep<D, MODE, KIND>(vel, a.bc, a.htau, a.tau, a.scaled, a.g[2 * s],
-                         a.g[2 * s + 1], a.ts[2 * s], a.ts[2 * s + 1], x, y, z);
+  for (int s = 0; s < a.nsub; ++s)
+    rk2_substep<D, kExact64, KIND>(vel, a.bc, a.htau, a.tau, a.scaled, a.g[2 * s],
+                                   a.g[2 * s + 1], a.ts[2 * s], a.ts[2 * s + 1], x, y, z);
   // con_evaluator(departure points) wraps them in place (semilag.inc:43)
   if (a.bc == TBX_BC_PERIODIC) {
     x = wrap1(x);
@@ -244,8 +227,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
   }
   const int dof = conc.dof;
   double *o = vals + leaf * dof * a.P + m;
-  eval_dof<D, MODE>(conc, x, y, z,
-                    [&](int l, double v) { o[(int64_t)l * a.P] = v; });
+  eval_dof<D, kExact64>(conc, x, y, z,
+                        [&](int l, double v) { o[(int64_t)l * a.P] = v; });
 }
 
 // The start point of this thread's RK2 substep, read back from its row of
@@ -262,33 +245,16 @@ __device__ __forceinline__ void reload_start(RegroupLds<BLOCK, NF> &sh, double (
   st[2] = sh.f[2][threadIdx.x];
 }
 
-// Leaf and node of arrival point i0 + t of a workgroup starting at point i0
-// (t < the workgroup size), points past the last taken as the last: the
-// workgroup-uniform i0 / P in scalar registers, the rest in 32 bits.
-__device__ __forceinline__ void arrival_node(const StepArgs &a, int64_t i0, int t,
-                                             int64_t &leaf, int &m) {
-  if (i0 + t >= a.npts) {
-    leaf = a.npts / a.P - 1;
-    m = a.P - 1;
-    return;
-  }
-  const int64_t l0 = i0 / a.P;
-  const uint32_t r = (uint32_t)(i0 - l0 * a.P) + (uint32_t)t;
-  const uint32_t q = r / (uint32_t)a.P;
-  leaf = l0 + q;
-  m = (int)(r - q * (uint32_t)a.P);
-}
-
 // The same step with the workgroup's points regrouped by leaf before each
 // of the 2 num_rk_step + 1 evaluations (regroup_pos in tbx_device.h).  The
 // thread that holds a point after a regroup carries it on: the RK2 state
 // (start point, wrapped midpoint) travels with the point through LDS, and
 // the leaf found for the regroup is the one the evaluation uses.  Lanes
 // past the last arrival point carry a copy of it and store nothing.
-template <int MODE, int KIND, int BLOCK>
-__device__ __forceinline__ void k_step_rg_body(const VelSource &vel, const TreeView &conc,
-                                               const StepArgs &a, double *__restrict__ vals,
-                                               double *__restrict__ dep) {
+template <int KIND, int BLOCK, int WPE>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step_rg(
+    VelSource vel, TreeView conc, StepArgs a, double *__restrict__ vals,
+    double *__restrict__ dep) {
   __shared__ RegroupLds<BLOCK, 6> sh;
   const uint32_t b = blockIdx.x;
   const int64_t lb = (int64_t)(b & 7u) * a.per_xcd + (int64_t)(b >> 3);
@@ -315,45 +281,16 @@ __device__ __forceinline__ void k_step_rg_body(const VelSource &vel, const TreeV
       }
       lf = locate(vel.t[0], st[0], st[1], st[2]);
       double v0, v1, v2;
-      bool nodal = false;
-      if constexpr (KIND == kVelTree || KIND == kVelExtrap) {
-        // the first substep starts at the arrival nodes: their velocities
-        // from the nodal values, and the regroup and contraction only in
-        // workgroups holding a node of another depth's leaf (whose points
-        // then take the nodal value again where they have one, so that a
-        // point's result does not depend on the workgroup it falls in)
-        if (s == 0 && a.vnode) {
-          // (the arrival node recomputed from the thread index: nothing of it
-          // stays live through the substeps)
-          int64_t jl;
-          int jm;
-          arrival_node(a, i0, (int)threadIdx.x, jl, jm);
-          const bool got = nodal_velocity<D>((const NodalT<MODE> *)a.vnode, vel.t[0], conc.info[jl], jm, lf, a.P,
-                                             a.scaled, a.g[0], v0, v1, v2);
-          nodal = !__syncthreads_or(!got);
-        }
+      {
+        double p3[3] = {st[0], st[1], st[2]};
+        regroup(sh, orig, lf, p3);
+        st[0] = p3[0];
+        st[1] = p3[1];
+        st[2] = p3[2];
       }
-      if (!nodal) {
-        {
-          double p3[3] = {st[0], st[1], st[2]};
-          regroup(sh, orig, lf, p3);
-          st[0] = p3[0];
-          st[1] = p3[1];
-          st[2] = p3[2];
-        }
-        eval_velocity<D, MODE, KIND>(vel, 1, a.ts[2 * s], a.scaled, a.g[2 * s], a.bc, st[0],
-                                     st[1], st[2], v0, v1, v2, lf);
-        reload_start(sh, st);
-        if constexpr (KIND == kVelTree || KIND == kVelExtrap) {
-          if (s == 0 && a.vnode) {  // the point this thread now holds
-            int64_t jl;
-            int jm;
-            arrival_node(a, i0, orig, jl, jm);
-            nodal_velocity<D>((const NodalT<MODE> *)a.vnode, vel.t[0], conc.info[jl], jm, lf, a.P, a.scaled, a.g[0],
-                              v0, v1, v2);
-          }
-        }
-      }
+      eval_velocity<D, kExact64, KIND>(vel, 1, a.ts[2 * s], a.scaled, a.g[2 * s], a.bc, st[0],
+                                       st[1], st[2], v0, v1, v2, lf);
+      reload_start(sh, st);
       // midpoint xtmp = xinit + (0.5 * dt) * vtmp (traj.inc:36), wrapped
       // for its evaluation only
       st[3] = st[0] + a.htau * v0;
@@ -366,8 +303,8 @@ __device__ __forceinline__ void k_step_rg_body(const VelSource &vel, const TreeV
       }
       lf = locate(vel.t[0], st[3], st[4], st[5]);
       regroup(sh, orig, lf, st);
-      eval_velocity<D, MODE, KIND>(vel, 2, a.ts[2 * s + 1], a.scaled, a.g[2 * s + 1], a.bc, st[3],
-                             st[4], st[5], v0, v1, v2, lf);
+      eval_velocity<D, kExact64, KIND>(vel, 2, a.ts[2 * s + 1], a.scaled, a.g[2 * s + 1], a.bc,
+                                       st[3], st[4], st[5], v0, v1, v2, lf);
       reload_start(sh, st);
       // xsol = xinit + dt * vtmp (traj.inc:41-42)
       st[0] = st[0] + a.tau * v0;
@@ -393,20 +330,13 @@ __device__ __forceinline__ void k_step_rg_body(const VelSource &vel, const TreeV
     const int64_t al = gi / a.P;
     const int am = (int)(gi - al * a.P);
     double *o = vals + al * conc.dof * a.P + am;
-    eval_dof<D, MODE>(
+    eval_dof<D, kExact64>(
         conc, p3[0], p3[1], p3[2],
         [&](int l, double v) {
           if (live) o[(int64_t)l * a.P] = v;
         },
         lf);
   }
-}
-
-template <int MODE, int KIND, int BLOCK, int WPE>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step_rg(
-    VelSource vel, TreeView conc, StepArgs a, double *__restrict__ vals,
-    double *__restrict__ dep) {
-  k_step_rg_body<MODE, KIND, BLOCK>(vel, conc, a, vals, dep);
 }
 
 // The step in every mode but TBX_EXACT (tbx_rows.h).  A thread keeps its
@@ -618,18 +548,18 @@ hipError_t with_kind(int kind, F f) {
   }
 }
 
-template <int MODE, int KIND, int BLOCK, int WPE>
+template <int KIND, int BLOCK, int WPE>
 hipError_t launch_step_shape(const VelSource &vel, const TreeView &conc, const StepArgs &a,
                              double *vals, double *dep, hipStream_t s) {
-  hipLaunchKernelGGL((k_step<MODE, KIND, BLOCK, WPE>), dim3((unsigned)(8 * a.per_xcd)),
+  hipLaunchKernelGGL((k_step<KIND, BLOCK, WPE>), dim3((unsigned)(8 * a.per_xcd)),
                      dim3(BLOCK), 0, s, vel, conc, a, vals, dep);
   return hipGetLastError();
 }
 
-template <int MODE, int KIND, int BLOCK, int WPE>
+template <int KIND, int BLOCK, int WPE>
 hipError_t launch_step_rg_shape(const VelSource &vel, const TreeView &conc, const StepArgs &a,
                                 double *vals, double *dep, hipStream_t s) {
-  hipLaunchKernelGGL((k_step_rg<MODE, KIND, BLOCK, WPE>), dim3((unsigned)(8 * a.per_xcd)),
+  hipLaunchKernelGGL((k_step_rg<KIND, BLOCK, WPE>), dim3((unsigned)(8 * a.per_xcd)),
                      dim3(BLOCK), 0, s, vel, conc, a, vals, dep);
   return hipGetLastError();
 }
@@ -662,37 +592,37 @@ hipError_t launch_step_mode(const VelSource &vel, const TreeView &conc, const St
   // the composite velocity kinds run the default shape only (the host
   // sizes the grid for the shape it asks for: kDefaultStepShape then)
   if (vel.kind == kVelExtrap)
-    return launch_step_rg_shape<MODE, kVelExtrap, 1024, 4>(vel, conc, a, vals, dep, s);
+    return launch_step_rg_shape<kVelExtrap, 1024, 4>(vel, conc, a, vals, dep, s);
   if (vel.kind == kVelSet)
-    return launch_step_rg_shape<MODE, kVelSet, 1024, 4>(vel, conc, a, vals, dep, s);
+    return launch_step_rg_shape<kVelSet, 1024, 4>(vel, conc, a, vals, dep, s);
   // launch shapes of kStepShapes (tbx_internal.h); the extra shapes are
   // built for the degrees of the benchmark workloads only
   constexpr int T = kVelTree;
   switch (a.shape) {
     case 0:
-      return launch_step_shape<MODE, T, 256, 1>(vel, conc, a, vals, dep, s);
+      return launch_step_shape<T, 256, 1>(vel, conc, a, vals, dep, s);
 #if TBX_Q == 8 || TBX_Q == 14
     case 4:
-      return launch_step_rg_shape<MODE, T, 256, 2>(vel, conc, a, vals, dep, s);
+      return launch_step_rg_shape<T, 256, 2>(vel, conc, a, vals, dep, s);
     case 1:
-      return launch_step_shape<MODE, T, 256, 4>(vel, conc, a, vals, dep, s);
+      return launch_step_shape<T, 256, 4>(vel, conc, a, vals, dep, s);
     case 2:
-      return launch_step_shape<MODE, T, 1024, 4>(vel, conc, a, vals, dep, s);
+      return launch_step_shape<T, 1024, 4>(vel, conc, a, vals, dep, s);
     case 3:
-      return launch_step_shape<MODE, T, 512, 4>(vel, conc, a, vals, dep, s);
+      return launch_step_shape<T, 512, 4>(vel, conc, a, vals, dep, s);
     case 5:
-      return launch_step_rg_shape<MODE, T, 512, 2>(vel, conc, a, vals, dep, s);
+      return launch_step_rg_shape<T, 512, 2>(vel, conc, a, vals, dep, s);
     case 7:
-      return launch_step_rg_shape<MODE, T, 512, 4>(vel, conc, a, vals, dep, s);
+      return launch_step_rg_shape<T, 512, 4>(vel, conc, a, vals, dep, s);
     case 8:
-      return launch_step_rg_shape<MODE, T, 1024, 8>(vel, conc, a, vals, dep, s);
+      return launch_step_rg_shape<T, 1024, 8>(vel, conc, a, vals, dep, s);
     case 9:
-      return launch_step_rg_shape<MODE, T, 512, 6>(vel, conc, a, vals, dep, s);
+      return launch_step_rg_shape<T, 512, 6>(vel, conc, a, vals, dep, s);
     case 10:
-      return launch_step_rg_shape<MODE, T, 768, 6>(vel, conc, a, vals, dep, s);
+      return launch_step_rg_shape<T, 768, 6>(vel, conc, a, vals, dep, s);
 #endif
     default:  // shape 6, and the shapes not built for this degree
-      return launch_step_rg_shape<MODE, T, 1024, 4>(vel, conc, a, vals, dep, s);
+      return launch_step_rg_shape<T, 1024, 4>(vel, conc, a, vals, dep, s);
   }
   }
 }

@@ -67,13 +67,6 @@ struct MfmaAcc<float> {
   static __device__ __forceinline__ int row(int g, int r) { return 4 * g + r; }
 };
 
-__device__ __forceinline__ double fma_t(double a, double b, double c) {
-  return __builtin_fma(a, b, c);
-}
-__device__ __forceinline__ float fma_t(float a, float b, float c) {
-  return __builtin_fmaf(a, b, c);
-}
-
 template <typename T>
 __device__ __forceinline__ T lane_read(T v, int src) {
   if constexpr (sizeof(T) == 8) {
