@@ -230,9 +230,12 @@ __global__ __launch_bounds__(kBlock) void k_order_start(int32_t *__restrict__ hi
   if (meta[0] == 0) return;
   const int64_t l = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int lane = (int)(threadIdx.x & 63u);
-  int c = 0;
-  if (l < L)
-    for (int x = 0; x < kXcds; ++x) c += hist[x * L + l];
+  int h[kXcds], c = 0;
+#pragma unroll
+  for (int x = 0; x < kXcds; ++x) {
+    h[x] = l < L ? hist[x * L + l] : 0;
+    c += h[x];
+  }
   int incl = c;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -244,10 +247,10 @@ __global__ __launch_bounds__(kBlock) void k_order_start(int32_t *__restrict__ hi
   base = __builtin_amdgcn_readlane(base, 63);
   if (l >= L) return;
   int start = base + incl - c;  // the leaf's places, XCD by XCD
+#pragma unroll
   for (int x = 0; x < kXcds; ++x) {
-    const int h = hist[x * L + l];
     hist[x * L + l] = start;
-    start += h;
+    start += h[x];
   }
 }
 
