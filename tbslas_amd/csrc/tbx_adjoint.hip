@@ -223,9 +223,9 @@ __device__ __forceinline__ void rows_gradient(AdjLds<BLOCK> &s, const TreeView &
       jy = mine ? ky : jy;
       jz = mine ? kz : jz;
     }
-    s.g[0][src] = in ? jx : 0.0;
-    s.g[1][src] = in ? jy : 0.0;
-    s.g[2][src] = in ? jz : 0.0;
+    s.g[0][src] = in_box(in, jx);
+    s.g[1][src] = in_box(in, jy);
+    s.g[2][src] = in_box(in, jz);
   }
 }
 

@@ -451,6 +451,13 @@ __device__ __forceinline__ int order_by_leaf(RowsLds<BLOCK> &s, bool active, int
   return count;
 }
 
+// A sum u over the basis at a point: outside the leaf's box, where the basis
+// is zero (cheb_poly), it was taken at the box's middle instead, and counts as
+// zero times every coefficient: a NaN where one of them is not finite.
+__device__ __forceinline__ double in_box(bool in, double u) {
+  return in ? u : __builtin_fma(0.0, u, 0.0);
+}
+
 // Components c0 .. c0 + nc - 1 (nc <= 3) of t at the points in order[0,
 // count): s.e / s.leaf hold every point's leaf coordinates and leaf, and
 // component c is returned in s.e[c] (the coordinates are gone).  The caller
@@ -469,7 +476,6 @@ __device__ __forceinline__ void rows(RowsLds<BLOCK> &s, const TreeView &t, int c
     const int src = s.order[p0 + lane < count ? p0 + lane : count - 1] & kPlaceMask;
     const int leaf = s.leaf[src];
     const double ex = s.e[0][src], ey = s.e[1][src], ez = s.e[2][src];
-    // zero outside [-1, 1] (cheb_poly); evaluated at 0 there and dropped
     const bool in = fabs(ex) <= 1.0 && fabs(ey) <= 1.0 && fabs(ez) <= 1.0;
     T px[D], py[D];
     row_cheb<D>(in ? ex : 0.0, px);
@@ -485,7 +491,7 @@ __device__ __forceinline__ void rows(RowsLds<BLOCK> &s, const TreeView &t, int c
 #pragma unroll 1
       for (int c = 0; c < nc; ++c) {
         const double u = (double)row_contract<D, MODE == kFp32h>(cb, px, py, z);
-        if (mine) s.e[c][src] = in ? u : 0.0;
+        if (mine) s.e[c][src] = in_box(in, u);
         cb += NC;
       }
     }
@@ -607,7 +613,7 @@ __device__ __forceinline__ void in_place_dof(const TreeView &t, int leaf, double
 #pragma unroll 1
     for (int l = 0; l < t.dof; ++l) {
       double u = (double)row_contract<D, MODE == kFp32h>(cb, px, py, zx);
-      u = in ? u : 0.0;
+      u = in_box(in, u);
       if constexpr (MODE == kFp32h) u += head_value<D>(t, l, leaf, ex, ey, ez);
       if (mine) store(l, u);
       cb += NC;
