@@ -183,9 +183,9 @@ __device__ __forceinline__ void batch_item(const BatchProblem &pb, int parity, i
     }
     int lf = locate(vel, x, y, z);
     // stage 1 from the nodal values; the order and contraction only in
-    // workgroups holding a node of another depth's leaf, whose points then
-    // take the nodal value again where they have one (a point's result does
-    // not depend on the workgroup it falls in)
+    // workgroups holding a node of another depth's leaf, whose points keep
+    // the nodal value where they have one (a point's result does not depend
+    // on the workgroup it falls in)
     double v[3];
     bool got = false;
     if (pb.vnode) got = nodal_velocity<D>(pb.vnode, vel, inf, m, lf, P, 0, 1.0, v[0], v[1], v[2]);

@@ -109,18 +109,21 @@ constexpr int kOrderBlocks = 16384;  // a multiple of kXcds
 //
 // k_order_begin decides whether there is anything to order, from kProbes
 // windows of 64 consecutive points spread over the call: scattered (meta[0])
-// where more than a quarter of them change leaf eight times or more between
-// neighbours.  Points that come in runs of a leaf are taken as they come
-// (their accesses stay coalesced), and the kernels after this one return at
-// once.  Counting and placing every point before it was known took, for
-// points in leaf order, 20 us and as much again per million: 1 M of them on
-// 512 leaves of degree 8 48 us, now 32; 4 M on 4,096 leaves of degree 4, three
-// components, 123 us, now 71.  Block 0 probes, the others clear the counters.
+// where more than a quarter of them hold more than run_leaves leaves.  Others
+// are taken as they come (their accesses stay coalesced, a workgroup orders
+// its few leaves by itself), and the kernels after this one return at once.
+// Counting and placing every point before it was known took 20 us, and 20 to
+// 60 per million points, of calls that gained nothing: 1 M points in leaf
+// order on 512 leaves of degree 8 48 us, now 32; 4 M on 4,096 leaves of degree
+// 4, three components, 123 us, now 71.  Points in the order of a tree's grid
+// change leaf at every face and hold few all the same: 23.9 M departure points
+// of 32,768 leaves of degree 8 1,937 us ordered, now 794.  Block 0 probes, the
+// others clear the counters.
 __global__ __launch_bounds__(kProbeBlock) void k_order_begin(TreeView t,
                                                              const double *__restrict__ pts,
                                                              int64_t n, int bc,
                                                              int32_t *__restrict__ meta,
-                                                             int64_t words) {
+                                                             int64_t words, int run_leaves) {
   if (blockIdx.x > 0) {
     const int64_t stride = (int64_t)(gridDim.x - 1) * kProbeBlock;
     for (int64_t i = kMetaStride + (int64_t)(blockIdx.x - 1) * kProbeBlock + threadIdx.x;
@@ -141,9 +144,11 @@ __global__ __launch_bounds__(kProbeBlock) void k_order_begin(TreeView t,
     z = wrap1(z);
   }
   const int lf = locate(t, x, y, z);
-  const int left = __shfl_up(lf, 1, 64);
-  const int changes = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane > 0 && lf != left));
-  if (lane == 0 && changes >= 8) atomicAdd(&scattered, 1);
+  uint64_t rest = __builtin_amdgcn_ballot_w64(true);
+#pragma unroll 1
+  for (int k = 0; k < run_leaves && rest; ++k)
+    rest &= ~__builtin_amdgcn_ballot_w64(lf == __builtin_amdgcn_readlane(lf, __builtin_ctzll(rest)));
+  if (lane == 0 && rest) atomicAdd(&scattered, 1);
   __syncthreads();
   if (threadIdx.x == 0) meta[0] = 4 * scattered > kProbes;
 }
@@ -286,16 +291,22 @@ hipError_t launch_locate(const TreeView &t, const double *pts, int64_t n,
 int64_t order_words(int64_t n, int64_t L) { return 3 * n + kXcds * L + kMetaWords; }
 
 hipError_t launch_order_points(const TreeView &t, const double *pts, int64_t n, int bc,
-                               int32_t *words, PointPerm *perm, hipStream_t s) {
+                               double work, int32_t *words, PointPerm *perm, hipStream_t s) {
   int32_t *leaf = words, *rank = leaf + n, *meta = rank + n, *hist = meta + kMetaWords;
   perm->use = meta;
   perm->perm = hist + kXcds * t.L;
   const int64_t clear = kXcds * t.L + kMetaWords;
   const unsigned grid = std::min<unsigned>(grid_for(n), kOrderBlocks);
+  // On few leaves counting is cheap and large triangles gain from whole runs:
+  // grid points of 512 leaves of degree 14 119 us ordered and 131 as they come,
+  // three components 223 and 258; of degree 8, three components (495
+  // multiply-adds a point) 45.8 and 38.4; of 4,096 leaves of degree 14 1,526
+  // and 847.
+  const int run_leaves = t.L <= kFewLeaves && work >= 600 ? 2 : 8;
   hipLaunchKernelGGL(k_order_begin,
                      dim3(1 + (unsigned)std::min<int64_t>((clear + 4 * kProbeBlock - 1) /
                                                               (4 * kProbeBlock), kOrderBlocks)),
-                     dim3(kProbeBlock), 0, s, t, pts, n, bc, meta, clear);
+                     dim3(kProbeBlock), 0, s, t, pts, n, bc, meta, clear, run_leaves);
   hipLaunchKernelGGL(t.L <= kFewLeaves ? k_order_count<true> : k_order_count<false>, dim3(grid),
                      dim3(kBlock), 0, s, t, pts, n, bc, leaf, rank, hist, meta);
   hipLaunchKernelGGL(k_order_start, dim3(grid_for(t.L)), dim3(kBlock), 0, s, hist, t.L, meta);

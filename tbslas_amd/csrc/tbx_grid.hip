@@ -59,9 +59,9 @@ __device__ __forceinline__ void row_samples(const T *p, T (&r)[4]) {
 // 32,768 leaves of 8^3 samples took 1.81 ms in FP64, now 1.73, the evaluation
 // of as many points 0.54, now 0.44, and the two in TBX_EXACT 5.08, now 3.18.
 // FP32 fits all four (4,096 leaves of 10^3 samples, both: 377 us, one at a
-// time 398).  FP64 reads 2 KB of samples per point and is bound by what the
-// L1 returns: 34 GB in 1.73 ms is 32 bytes per clock and compute unit,
-// whether in 8- or 16-byte loads.  The sibling blocks, whose gathers are from
+// time 398).  FP64 reads 2 KB of samples per point, 34 GB in 1.73 ms or 32
+// bytes per clock and compute unit, whether in 8- or 16-byte loads: the
+// address units are busy 75 % of that time, the vector ALU 34 %.  The sibling blocks, whose gathers are from
 // LDS but for the points outside, take one at a time everywhere (FP32, 4,096
 // leaves of 8^3: 206 us; four outside, 290).
 template <int MODE, int U2, typename T, typename Store>

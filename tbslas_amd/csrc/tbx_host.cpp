@@ -743,7 +743,7 @@ struct PointOrder {
       return hipSuccess;
     block = pool_take(device, sizeof(int32_t) * (size_t)order_words(n, t->L), st);
     if (!block.mem) return hipSuccess;
-    return launch_order_points(t->view(), pts, n, bc, (int32_t *)block.mem, &perm, st);
+    return launch_order_points(t->view(), pts, n, bc, work, (int32_t *)block.mem, &perm, st);
   }
   ~PointOrder() {
     if (block.mem) pool_give(device, block);

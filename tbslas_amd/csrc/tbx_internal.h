@@ -292,11 +292,11 @@ hipError_t launch_gather_rows(const double *src, const int64_t *map, int64_t nro
                               double *dst, hipStream_t s);
 
 // Degree-independent launchers (tbx_common.hip).
-// Order of n points by leaf in words, order_words(n, L) 32-bit words.
-// n < 2^31.
+// Order of n points by leaf, work multiply-adds to be done at each, in words,
+// order_words(n, L) 32-bit words.  n < 2^31.
 int64_t order_words(int64_t n, int64_t L);
 hipError_t launch_order_points(const TreeView &t, const double *pts, int64_t n, int bc,
-                               int32_t *words, PointPerm *perm, hipStream_t s);
+                               double work, int32_t *words, PointPerm *perm, hipStream_t s);
 hipError_t launch_locate(const TreeView &t, const double *pts, int64_t n,
                          int bc, int32_t *leaf, hipStream_t s);
 hipError_t launch_grid_points(const TreeView &t, const double *node, int d,

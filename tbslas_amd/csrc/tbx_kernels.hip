@@ -126,13 +126,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
   // components: 51 us in order, 69 in place), and not for points taken
   // through perm, whose components are stored together (4 M of degree 4,
   // three: 360 us, in place 406).
-  if constexpr (BLOCK == 256) {
-    if (!ordered && t.dof <= 3 && rows_in_place(lf)) {
+  order_clear(sh);
+  if (BLOCK == 256 && !ordered && t.dof <= 3) {
+    if (rows_in_place(lf)) {
       in_place_dof<D, MODE>(t, lf, x, y, z, store);
       return;
     }
+  } else {
+    __syncthreads();
   }
-  const int count = order_by_leaf(sh, live, lf);
+  const int count = order_by_leaf<true>(sh, live, lf);
   rows_dof<D, MODE>(sh, t, count, lf, x, y, z, store);
 }
 

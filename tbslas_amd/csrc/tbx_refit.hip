@@ -256,8 +256,10 @@ constexpr int refit_waves() {
 // lines past the last, and rows of idle threads, are computed and dropped.
 // With scalar table operands and two buffers, before: 36,324 rows of degree
 // 14 644 us, now 331; 4,096 x 3 rows of degree 10 56 -> 44 us, 4,096 rows of
-// degree 8 14 -> 11 us.  Bound by its LDS stages; the values' read alone
-// would take 0.19 ms, 25 us and 4.6 us.
+// degree 8 14 -> 11 us; the values' read alone would take 0.19 ms, 25 us and
+// 4.6 us.  The vector ALU issues in 71, 58 and 30 % of the time, of the waits
+// a tenth are for LDS; the rest is the chain of load, three lines and two
+// barriers of each row at under three waves per SIMD.
 template <int D, bool ACC>
 __global__ __launch_bounds__(kRefitThreads) __attribute__((
     amdgpu_waves_per_eu(refit_waves<D>()))) void k_refit_project(const double *__restrict__ V,

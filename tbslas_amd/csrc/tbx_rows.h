@@ -371,6 +371,15 @@ struct RowsLds {
   int total;
 };
 
+// Empties the table of leaves.
+template <int BLOCK>
+__device__ __forceinline__ void order_clear(RowsLds<BLOCK> &s) {
+  for (int i = (int)threadIdx.x; i <= kRgSlots; i += BLOCK) {  // a block may hold 64 threads
+    if (i < kRgSlots) s.key[i] = -1;
+    s.cnt[i] = 0;
+  }
+}
+
 // Orders the active threads' points by leaf: afterwards order[0, count) are
 // their threads, points of one leaf together and padded to a multiple of 16
 // with copies of the last one; returns count, a multiple of 16.  Leaves
@@ -380,14 +389,14 @@ struct RowsLds {
 // parallel: one after another 64 leaves would take some 20,000 clocks).
 // Every thread of the workgroup must call it; the caller synchronises
 // before order is read.
-template <int BLOCK>
+// CLEARED: order_clear was called, and the workgroup synchronised, before.
+template <bool CLEARED = false, int BLOCK>
 __device__ __forceinline__ int order_by_leaf(RowsLds<BLOCK> &s, bool active, int leaf) {
   const int tid = (int)threadIdx.x, lane = tid & 63;
-  for (int i = tid; i <= kRgSlots; i += BLOCK) {  // a block may hold 64 threads
-    if (i < kRgSlots) s.key[i] = -1;
-    s.cnt[i] = 0;
+  if constexpr (!CLEARED) {
+    order_clear(s);
+    __syncthreads();
   }
-  __syncthreads();
   int slot = kRgSlots, rank = 0;
   bool todo = active;
   auto insert = [&]() {  // the thread's leaf into the table: its slot
@@ -579,13 +588,13 @@ __device__ __forceinline__ void rows_dof(RowsLds<BLOCK> &s, const TreeView &t, i
 // most two leaves, the row's first lane's and its last's: points that come in
 // runs of a leaf.  They are contracted as they come (in_place_dof): the order
 // in LDS, its barriers and the second round that its padding takes bring such
-// points nothing (1 M of them on 512 leaves of degree 8 24.0 us, in place
-// 20; 16 M of degree 1 141 us, in place 118).  All threads of the workgroup
-// must call it.
+// points nothing (1 M of them on 512 leaves of degree 8 36.7 us, in place
+// 32.0; 16 M of degree 1 140 us, in place 118; to look costs others up to 1.7
+// us per million points).  All threads of the workgroup must call it.
 __device__ __forceinline__ bool rows_in_place(int leaf) {
-  const int lane = (int)(threadIdx.x & 63u);
-  const int first = __builtin_amdgcn_ds_bpermute((lane & 48) << 2, leaf);
-  const int last = __builtin_amdgcn_ds_bpermute((lane | 15) << 2, leaf);
+  // row_newbcast:0 and row_newbcast:15
+  const int first = __builtin_amdgcn_update_dpp(leaf, leaf, 0x150, 0xf, 0xf, false);
+  const int last = __builtin_amdgcn_update_dpp(leaf, leaf, 0x15f, 0xf, 0xf, false);
   return !__syncthreads_or(leaf != first && leaf != last);
 }
 

@@ -29,6 +29,9 @@ def _points(tree, n, kind, seed, size=1.0):
     s = x[tree.locate(x, int(size > 1)).argsort(stable=True)].contiguous()
     if kind == "runs":
         return s
+    if kind == "grid":  # faces belong to the neighbours: many changes of leaf, few leaves
+        g = tree.grid_points()
+        return g.repeat(1 + n // len(g), 1)[:n].contiguous()
     if kind == "half":  # the last half scattered
         return torch.cat([s[:n // 2], x[:n - n // 2]]).contiguous()
     if kind == "runs of 20":  # more leaves in a wavefront, at most two in some rows
@@ -45,7 +48,7 @@ def _parts(f, x):
 
 
 @pytest.mark.parametrize("mode", ["fp64", "fp32", "fp32h"])
-@pytest.mark.parametrize("kind", ["runs", "half", "runs of 20", "scattered"])
+@pytest.mark.parametrize("kind", ["runs", "half", "runs of 20", "grid", "scattered"])
 @pytest.mark.parametrize("q,dof", [(1, 1), (2, 3), (5, 2), (8, 1), (8, 4), (13, 1), (16, 3)])
 def test_route_keeps_values(tb, q, dof, kind, mode):
     import torch
