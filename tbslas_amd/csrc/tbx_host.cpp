@@ -671,10 +671,11 @@ PoolBlock pool_take(int device, size_t bytes, hipStream_t s) {
   return b;
 }
 
-// Back from a call on b.stream, whose kernels may still run.  The longest
-// idle blocks beyond the bounds are freed behind their own last call.
+// Back from a call on b.stream, whose kernels may still run.  A block larger
+// than all that is kept is freed behind them, the longest idle blocks beyond
+// the bounds behind their own last call.
 void pool_give(int device, const PoolBlock &b) {
-  if (hipEventRecord(b.done, b.stream) != hipSuccess) {
+  if (b.bytes > kPoolKeep || hipEventRecord(b.done, b.stream) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFreeAsync(b.mem, b.stream);
     (void)hipEventDestroy(b.done);
