@@ -128,7 +128,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
   // three: 360 us, in place 406).
   order_clear(sh);
   if (BLOCK == 256 && !ordered && t.dof <= 3) {
-    if (rows_in_place(lf)) {
+    if (rows_in_place(sh, lf)) {
       in_place_dof<D, MODE>(t, lf, x, y, z, store);
       return;
     }

@@ -369,6 +369,7 @@ struct RowsLds {
   int key[kRgSlots];
   int cnt[kRgSlots + 1];
   int total;
+  int spread[BLOCK / 64];  // rows_in_place's vote
 };
 
 // Empties the table of leaves.
@@ -591,11 +592,18 @@ __device__ __forceinline__ void rows_dof(RowsLds<BLOCK> &s, const TreeView &t, i
 // points nothing (1 M of them on 512 leaves of degree 8 36.7 us, in place
 // 32.0; 16 M of degree 1 140 us, in place 118; to look costs others up to 1.7
 // us per million points).  All threads of the workgroup must call it.
-__device__ __forceinline__ bool rows_in_place(int leaf) {
+template <int BLOCK>
+__device__ __forceinline__ bool rows_in_place(RowsLds<BLOCK> &s, int leaf) {
   // row_newbcast:0 and row_newbcast:15
   const int first = __builtin_amdgcn_update_dpp(leaf, leaf, 0x150, 0xf, 0xf, false);
   const int last = __builtin_amdgcn_update_dpp(leaf, leaf, 0x15f, 0xf, 0xf, false);
-  return !__syncthreads_or(leaf != first && leaf != last);
+  const uint64_t others = __builtin_amdgcn_ballot_w64(leaf != first && leaf != last);
+  if ((threadIdx.x & 63u) == 0) s.spread[threadIdx.x >> 6] = others != 0;
+  __syncthreads();  // one barrier, where __syncthreads_or takes more
+  int any = 0;
+#pragma unroll
+  for (int w = 0; w < BLOCK / 64; ++w) any |= s.spread[w];
+  return __builtin_amdgcn_readfirstlane(any) == 0;
 }
 
 // All components of t at the thread's point, contracted in its own lane, each
