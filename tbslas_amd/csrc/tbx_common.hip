@@ -114,10 +114,10 @@ constexpr int kOrderBlocks = 16384;  // a multiple of kXcds
 // its few leaves by itself), and the kernels after this one return at once.
 // Counting and placing every point before it was known took 20 us, and 20 to
 // 60 per million points, of calls that gained nothing: 1 M points in leaf
-// order on 512 leaves of degree 8 48 us, now 32; 4 M on 4,096 leaves of degree
+// order on 512 leaves of degree 8 48 us, now 30; 4 M on 4,096 leaves of degree
 // 4, three components, 123 us, now 71.  Points in the order of a tree's grid
 // change leaf at every face and hold few all the same: 23.9 M departure points
-// of 32,768 leaves of degree 8 1,937 us ordered, now 794.  Block 0 probes, the
+// of 32,768 leaves of degree 8 1,937 us ordered, now 645.  Block 0 probes, the
 // others clear the counters.
 __global__ __launch_bounds__(kProbeBlock) void k_order_begin(TreeView t,
                                                              const double *__restrict__ pts,
@@ -301,7 +301,7 @@ hipError_t launch_order_points(const TreeView &t, const double *pts, int64_t n, 
   // grid points of 512 leaves of degree 14 119 us ordered and 131 as they come,
   // three components 223 and 258; of degree 8, three components (495
   // multiply-adds a point) 45.8 and 38.4; of 4,096 leaves of degree 14 1,526
-  // and 847.
+  // and 829.
   const int run_leaves = t.L <= kFewLeaves && work >= 600 ? 2 : 8;
   hipLaunchKernelGGL(k_order_begin,
                      dim3(1 + (unsigned)std::min<int64_t>((clear + 4 * kProbeBlock - 1) /

@@ -718,7 +718,7 @@ bool capturing(hipStream_t s) {
 //    three components, 60 a point, 614 us, ordered 756; but 4 M of degree 4
 //    and three, 105 a point, 445 us, ordered 360) or kOrderWork in all (60,000
 //    points of degree 14 on 512 leaves, 4e7 in all: scattered 76 us, ordered
-//    27; in leaf order 10 us, 22 with the launches that find them so), or
+//    27; in leaf order 10 us, 20 with the launches that find them so), or
 //    with fewer than two points a leaf (nothing to bring together);
 //  - on few leaves, which a workgroup orders by itself with little padding:
 //    up to 16 always (degree 14, 8 leaves: 1.5 M points 109 us, ordered first

@@ -96,7 +96,15 @@ __global__ __launch_bounds__(kBlock) void k_traj_exact(VelSource vel, const doub
 // The same three in the other modes: a workgroup's points ordered by leaf
 // and contracted row by row (tbx_rows.h).  Threads past the last point hold
 // a copy of it and take no part.  BLOCK: with_rows_block.
-template <int MODE, int BLOCK>
+//
+// RUNS: the call's points were looked at (perm), and may come in runs of a
+// leaf.  In place only up to three components (200,000 points of degree 4, 16
+// components: 51 us in order, 69 in place), and not for points taken through
+// perm, whose components are stored together (4 M of degree 4, three: 360 us,
+// in place 406).  A kernel of its own: with the branch in it, scattered points
+// that are not looked at took 3 % longer (846,243 on eight leaves of degree 12
+// 41.6 us, 43.2).
+template <int MODE, int BLOCK, bool RUNS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_waves(MODE)))) void k_eval(
     TreeView t, double *__restrict__ pts, int64_t n, int bc, int write_back,
     double *__restrict__ out, PointPerm perm) {
@@ -104,8 +112,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
   const int64_t i0 = (int64_t)blockIdx.x * BLOCK;
   const bool live = i0 + (int)threadIdx.x < n;
   int64_t i = live ? i0 + (int)threadIdx.x : n - 1;
-  const bool ordered = perm.perm && *perm.use;
-  if (ordered) i = perm.perm[i];
+  bool ordered = true;
+  if constexpr (RUNS) {
+    ordered = *perm.use;
+    if (ordered) i = perm.perm[i];
+  }
   double x = pts[3 * i + 0], y = pts[3 * i + 1], z = pts[3 * i + 2];
   if (bc == TBX_BC_PERIODIC) {
     x = wrap1(x);
@@ -119,24 +130,20 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(rows_wave
   }
   const int lf = locate(t, x, y, z);
   double *o = out + i * t.dof;
-  auto store = [&](int l, double v) {
-    if (live) o[l] = v;
-  };
-  // In place only up to three components (200,000 points of degree 4, 16
-  // components: 51 us in order, 69 in place), and not for points taken
-  // through perm, whose components are stored together (4 M of degree 4,
-  // three: 360 us, in place 406).
-  order_clear(sh);
-  if (BLOCK == 256 && !ordered && t.dof <= 3) {
-    if (rows_in_place(sh, lf)) {
-      in_place_dof<D, MODE>(t, lf, x, y, z, store);
-      return;
+  bool rest = live;
+  if constexpr (RUNS) {
+    if (!ordered && t.dof <= 3 && rows_in_place(lf)) {
+      in_place_dof<D, MODE>(t, lf, x, y, z, [&](int l, double v) {
+        if (live) o[l] = v;
+      });
+      rest = false;
     }
-  } else {
-    __syncthreads();
   }
-  const int count = order_by_leaf<true>(sh, live, lf);
-  rows_dof<D, MODE>(sh, t, count, lf, x, y, z, store);
+  const int count = order_by_leaf(sh, rest, lf);
+  if (RUNS && count == 0) return;  // uniform over the workgroup
+  rows_dof<D, MODE>(sh, t, count, lf, x, y, z, [&](int l, double v) {
+    if (rest) o[l] = v;
+  });
 }
 
 template <int MODE, int KIND, int BLOCK>
@@ -647,8 +654,13 @@ hipError_t TBX_CAT(launch_eval_q, TBX_Q)(int mode, const TreeView &t,
                          write_back, out);
     } else {
       with_rows_block(n, [&](auto b, unsigned grid) {
-        hipLaunchKernelGGL((k_eval<M, decltype(b)::value>), dim3(grid), dim3(decltype(b)::value),
-                           0, s, t, pts, n, bc, write_back, out, perm);
+        constexpr int B = decltype(b)::value;
+        if (perm.perm)
+          hipLaunchKernelGGL((k_eval<M, B, true>), dim3(grid), dim3(B), 0, s, t, pts, n, bc,
+                             write_back, out, perm);
+        else
+          hipLaunchKernelGGL((k_eval<M, B, false>), dim3(grid), dim3(B), 0, s, t, pts, n, bc,
+                             write_back, out, perm);
       });
     }
     return hipGetLastError();

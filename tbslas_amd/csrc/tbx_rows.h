@@ -369,17 +369,7 @@ struct RowsLds {
   int key[kRgSlots];
   int cnt[kRgSlots + 1];
   int total;
-  int spread[BLOCK / 64];  // rows_in_place's vote
 };
-
-// Empties the table of leaves.
-template <int BLOCK>
-__device__ __forceinline__ void order_clear(RowsLds<BLOCK> &s) {
-  for (int i = (int)threadIdx.x; i <= kRgSlots; i += BLOCK) {  // a block may hold 64 threads
-    if (i < kRgSlots) s.key[i] = -1;
-    s.cnt[i] = 0;
-  }
-}
 
 // Orders the active threads' points by leaf: afterwards order[0, count) are
 // their threads, points of one leaf together and padded to a multiple of 16
@@ -390,14 +380,14 @@ __device__ __forceinline__ void order_clear(RowsLds<BLOCK> &s) {
 // parallel: one after another 64 leaves would take some 20,000 clocks).
 // Every thread of the workgroup must call it; the caller synchronises
 // before order is read.
-// CLEARED: order_clear was called, and the workgroup synchronised, before.
-template <bool CLEARED = false, int BLOCK>
+template <int BLOCK>
 __device__ __forceinline__ int order_by_leaf(RowsLds<BLOCK> &s, bool active, int leaf) {
   const int tid = (int)threadIdx.x, lane = tid & 63;
-  if constexpr (!CLEARED) {
-    order_clear(s);
-    __syncthreads();
+  for (int i = tid; i <= kRgSlots; i += BLOCK) {  // a block may hold 64 threads
+    if (i < kRgSlots) s.key[i] = -1;
+    s.cnt[i] = 0;
   }
+  __syncthreads();
   int slot = kRgSlots, rank = 0;
   bool todo = active;
   auto insert = [&]() {  // the thread's leaf into the table: its slot
@@ -585,25 +575,17 @@ __device__ __forceinline__ void rows_dof(RowsLds<BLOCK> &s, const TreeView &t, i
   }
 }
 
-// Whether the 16 lanes of every DPP row of the workgroup hold points of at
+// Whether the 16 lanes of every DPP row of the wavefront hold points of at
 // most two leaves, the row's first lane's and its last's: points that come in
 // runs of a leaf.  They are contracted as they come (in_place_dof): the order
-// in LDS, its barriers and the second round that its padding takes bring such
-// points nothing (1 M of them on 512 leaves of degree 8 36.7 us, in place
-// 32.0; 16 M of degree 1 140 us, in place 118; to look costs others up to 1.7
-// us per million points).  All threads of the workgroup must call it.
-template <int BLOCK>
-__device__ __forceinline__ bool rows_in_place(RowsLds<BLOCK> &s, int leaf) {
+// in LDS and the second round that its padding takes bring such points nothing
+// (1 M of them on 512 leaves of degree 8 36.7 us, in place 29.9; of degree 6
+// 29.6, in place 25.2).  All lanes are active.
+__device__ __forceinline__ bool rows_in_place(int leaf) {
   // row_newbcast:0 and row_newbcast:15
   const int first = __builtin_amdgcn_update_dpp(leaf, leaf, 0x150, 0xf, 0xf, false);
   const int last = __builtin_amdgcn_update_dpp(leaf, leaf, 0x15f, 0xf, 0xf, false);
-  const uint64_t others = __builtin_amdgcn_ballot_w64(leaf != first && leaf != last);
-  if ((threadIdx.x & 63u) == 0) s.spread[threadIdx.x >> 6] = others != 0;
-  __syncthreads();  // one barrier, where __syncthreads_or takes more
-  int any = 0;
-#pragma unroll
-  for (int w = 0; w < BLOCK / 64; ++w) any |= s.spread[w];
-  return __builtin_amdgcn_readfirstlane(any) == 0;
+  return __builtin_amdgcn_ballot_w64(leaf != first && leaf != last) == 0;
 }
 
 // All components of t at the thread's point, contracted in its own lane, each
