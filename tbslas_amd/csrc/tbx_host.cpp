@@ -614,6 +614,7 @@ void pool_tree_count(int device, int change) {
   p.trees += change;
   if (p.trees == 0 && p.pool) {
     for (const PoolBlock &b : p.idle) {
+      (void)hipEventSynchronize(b.done);  // the caller's device may be another
       (void)hipFree(b.mem);
       (void)hipEventDestroy(b.done);
     }
